@@ -546,7 +546,7 @@ def main():
     hip_sync()
     profiled_ms = (time.perf_counter() - tp0) / args.steps * 1e3
     progress(f"{args.workload}: {step_s * 1e3:.3f} ms per step")
-    kernels = ["gen", "gen_coarse", "sort_rec_hist", "sort_rec_scatter", "region", "bucket", "runs", "pairs_small",
+    kernels = ["tiles", "tile_cols", "bins", "gen", "gen_coarse", "sort_rec_hist", "sort_rec_scatter", "region", "bucket", "runs", "pairs_small",
                "pairs_big",
                "sort_seg_hist", "sort_seg_scatter", "tail_hist", "sort_pairs", "select", "pack", "scan",
                "gen_count"]
@@ -556,7 +556,8 @@ def main():
     # (repeated variants of a sequence left out), and the passes after it
     # move those: their algorithmic bytes per launch, from the run's counts
     rs = eng.stats()
-    per_launch = {"gen_coarse": 8.0 * rs["n_records"] + 24.0 * rs["n_sequences"],
+    per_launch = {"tiles": 4.0 * rs["n_records"] + 24.0 * rs["n_sequences"], "bins": 4.0 * rs["n_records"],
+                  "gen_coarse": 8.0 * rs["n_records"] + 24.0 * rs["n_sequences"],
                   "region": 16.0 * rs["n_records"], "bucket": 8.0 * rs["n_records"]}
     for k, b in per_launch.items():
         if prof[k][0] and rs["n_chunks"] == 1:

@@ -37,6 +37,7 @@
 #include "xtn_overlap.hpp"
 #include "xtn_serve.hpp"
 #include "xtn_tail.hpp"
+#include "xtn_tiles.hpp"
 
 using namespace xtn;
 
@@ -80,6 +81,7 @@ struct xtn_handle {
 	DBuf bcount, ctl;  // region layout: bucket cursors, coarse bucket/tile table
 	DBuf recs_all, recs_part;  // chunked runs: every record once, then ordered by part
 	DBuf seg_cur, seg_ctl;  // the generator's coarse pass: sub-range cursors, digit tiling
+	DBuf tile_rec, tile_offs, tile_cols;  // tiles ordered by bin, their bin starts by tile and by bin
 	DBuf pk, voff, recs, recs_alt, hist, scan_tmp, runs_small, runs_big, big_pre, pairs, pairs_alt,
 	    flags, pos, dist, out_pairs, out_dist, ctrs, part_hist, scalar;
 	// overlap-mode workspaces
@@ -123,6 +125,7 @@ struct xtn_handle {
 	int tune_low = 0;           // pair bits left unsorted for the select's in-group ranking: 0, 8, 16, 24
 	int tune_coarse_sep = 0;    // 1: the records' first ordering pass as a pass of its own (tuned)
 	bool tail_full = false;     // a group outgrew the select's window: full sorts until new sequences
+	bool bin_parts = false;     // a bin listed more records than fit: bins in parts until new sequences
 	bool coarse_off = false;    // a sub-range of the generator's coarse pass overflowed: the separate
 	                            // pass until new sequences
 	double tune_ms = 0, tune_ms_default = 0;
@@ -246,6 +249,13 @@ int grow_keep(xtn_handle* h, DBuf& b, size_t bytes, size_t keep) {
 	release(b);
 	b = nb;
 	return XTN_OK;
+}
+
+int bits_for(int64_t maxval) {
+	int b = 1;
+	while (b < 62 && (1ll << b) <= maxval)
+		++b;
+	return b;
 }
 
 // sum_{k <= min(d, L)} C(L, k) for the 18-residue prefix of a len-residue
@@ -491,13 +501,6 @@ int read_ctrs(xtn_handle* h, RunCtrs* out) {
 	return XTN_OK;
 }
 
-int bits_for(int64_t maxval) {
-	int b = 1;
-	while (b < 62 && (1ll << b) <= maxval)
-		++b;
-	return b;
-}
-
 double now_ms() {
 	using namespace std::chrono;
 	return duration<double, std::milli>(steady_clock::now().time_since_epoch()).count();
@@ -506,6 +509,7 @@ double now_ms() {
 // ----------------------------------------------------------- NN pipeline --
 
 constexpr int KEY_BITS = 32;             // hash bits that order records into runs
+constexpr int64_t TILES_MIN_RECORDS = 600000;  // fewer records of a chunk take the sorted layout
 
 // device control block: the counters of the candidate search, then the
 // tail's block
@@ -793,7 +797,64 @@ struct Grouping {
 	int64_t sub_cap = 0;
 	int64_t rtiles = 0;
 	BucketArgs ba{};
+	bool tiles = false;  // tiles ordered by bin (xtn_tiles.hpp) instead of any of the above
+	TileArgs ta{};
+	BinArgs bn{};
 };
+
+// ---- tiles and bins of one chunk (xtn_tiles.hpp)
+
+// the bin kernel: 512 threads of 18 groups of four records, two workgroups
+// per CU (one's loads and barriers under the other's work: 430 us against
+// 476 at 1M CDR3s, d = 2, for one of 1024 threads over half as many bins)
+constexpr int BIN_NT = 512, BIN_QPT = 18, BIN_PER_CU = 2;
+
+struct TilePlan {
+	uint32_t tile = 0;  // records between the starts of two tiles
+	int64_t ntiles = 0;
+	int bin_bits = 0;
+	int idx_bits = 0;
+};
+
+// the tiling of V records of n sequences
+TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
+	// a tile holds the sequences starting in its stretch of `tile` records,
+	// so up to one sequence's variants more, and no more sequences than its
+	// tables (half of that on average, for uneven lengths)
+	const int64_t most = TL_CAP - (int64_t)host_variant_count(MAX_PREFIX, d);
+	const double avg = (double)V / n;
+	int64_t tile = std::min<int64_t>(most, (int64_t)(0.5 * tl_seqs(d) * avg));
+	// whole rounds of one workgroup per CU
+	const int64_t rounds = (V + n_cu * tile - 1) / (n_cu * tile);
+	tile = std::max<int64_t>(std::min<int64_t>(tile, (V + n_cu * rounds - 1) / (n_cu * rounds)), 2048);
+	tile = std::min(tile, most);
+	TilePlan p;
+	p.tile = (uint32_t)tile;
+	p.ntiles = (V + tile - 1) / tile;
+	// index bits for twice the average tile's sequences
+	p.idx_bits = std::min(bits_for((int64_t)(2.0 * (double)tile / avg) + 1), tl_idx_bits(d));
+	// The fewest bins whose runs fit the bin kernel's registers (a run, the
+	// records that one tile has for one bin, is Poisson and takes a group per
+	// four of them), and enough of them that bin and record leave 16 keys per
+	// record: two records meet by chance once in 30 or so.
+	const double key_bits = std::log2((double)V) + 4.0;
+	for (p.bin_bits = 6; (1 << p.bin_bits) < TL_BINS_MAX; ++p.bin_bits) {
+		const double lambda = (double)tile / (1 << p.bin_bits);
+		double q = 0, w = std::exp(-lambda);
+		if (lambda > 200)
+			q = lambda / 4 + 0.375;
+		else
+			for (int k = 1; k < 400; ++k) {
+				w *= lambda / k;
+				q += w * ((k + 3) / 4);
+			}
+		// (at distance 3 a neighbouring pair shares a hundred variants and a
+		// fifth of the records may be listed: half as many records a bin)
+		if (q * (double)p.ntiles <= (d == 3 ? 0.45 : 0.92) * BIN_NT * BIN_QPT && p.bin_bits + 30 - p.idx_bits >= key_bits)
+			break;
+	}
+	return p;
+}
 
 // sub-ranges per coarse digit in the generator's coarse pass: a generator
 // tile takes the one of its index mod 64 (tiles of one sub-range run on one
@@ -808,6 +869,15 @@ constexpr int COARSE_SUB_BITS = 6;
 int issue_grouping(xtn_handle* h, Grouping& g) {
 	hipStream_t s = h->stream;
 	BucketArgs& ba = g.ba;
+	if (g.tiles) {
+		StageScope sg(h, "sort");
+		ProfScope ps(h, "tile_cols", 4.0 * (double)g.bn.nb * (double)g.bn.ntiles);
+		const dim3 grid((unsigned)(g.bn.cpitch / 64), (unsigned)(g.bn.nb / 64 + 1));
+		k_tile_cols<<<grid, 256, 0, s>>>(g.ta.offs, g.bn.ntiles, g.bn.nb, g.ta.pitch, h->tile_cols.as<uint16_t>(),
+		                                 g.bn.cpitch, ctr_field(h, offsetof(RunCtrs, n_records)));
+		HIP_LAUNCH_CHECK(h);
+		return XTN_OK;
+	}
 	if (g.region && g.coarse) {
 		StageScope sg(h, "sort");
 		k_seg_tiles<1 << COARSE_SUB_BITS><<<1, SEG_NT, 0, s>>>(h->seg_cur.as<uint32_t>(), g.sub_cap,
@@ -945,12 +1015,30 @@ int regroup_exact(xtn_handle* h, Grouping& g) {
 }
 
 int issue_buckets(xtn_handle* h, Grouping& g, uint32_t lo, uint32_t hi, int64_t pcap) {
+	const bool ranged = lo > 0 || (int64_t)hi < g.nseq;
+	if (g.tiles) {
+		BinArgs& bn = g.bn;
+		bn.pairs = h->pairs.as<uint64_t>();
+		bn.pcap = pcap;
+		bn.id_lo = lo;
+		bn.id_hi = hi;
+		StageScope sg(h, "pairs");
+		ProfScope ps(h, "bins", (double)g.nrec * 4.0);
+		const unsigned grid = (unsigned)std::min<int64_t>(bn.nb, (int64_t)h->n_cu * BIN_PER_CU);
+		if (h->bin_parts)
+			ranged ? k_bins<BIN_NT, BIN_QPT, true, true><<<grid, BIN_NT, 0, h->stream>>>(bn)
+			       : k_bins<BIN_NT, BIN_QPT, false, true><<<grid, BIN_NT, 0, h->stream>>>(bn);
+		else
+			ranged ? k_bins<BIN_NT, BIN_QPT, true, false><<<grid, BIN_NT, 0, h->stream>>>(bn)
+			       : k_bins<BIN_NT, BIN_QPT, false, false><<<grid, BIN_NT, 0, h->stream>>>(bn);
+		HIP_LAUNCH_CHECK(h);
+		return XTN_OK;
+	}
 	BucketArgs& ba = g.ba;
 	ba.pairs = h->pairs.as<uint64_t>();
 	ba.pcap = pcap;
 	ba.id_lo = lo;
 	ba.id_hi = hi;
-	const bool ranged = lo > 0 || (int64_t)hi < g.nseq;
 	StageScope sg(h, "pairs");
 	ProfScope ps(h, "bucket", (double)g.nrec * 8.0);
 	// persistent workgroups, as many per CU as the LDS of the instantiation
@@ -1144,6 +1232,14 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	ga.part_bits = pbits;
 	ga.V = (int64_t)V;
 	ga.set_of = set_of;
+	// one chunk of enough records at distances 1 to 3: tiles ordered by bin
+	// (xtn_tiles.hpp), until a bound there is outgrown
+	auto use_tiles = [&]() {
+		return nparts == 1 && d <= 3 && (int64_t)V >= TILES_MIN_RECORDS && !h->no_alloc &&
+		       h->cfg.max_records_per_chunk <= 0 && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
+		       !h->coarse_off && !h->tail_safe;
+	};
+	const TilePlan tplan = use_tiles() ? plan_tiles((int64_t)V, nseq, d, h->n_cu) : TilePlan{};
 	// packing (unless done above to learn V) and the generator's tile table
 	bool prologue_done = false;
 	auto prologue = [&]() -> int {
@@ -1153,7 +1249,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			// packing, offsets and tile table in one launch (its look-back
 			// shares the error flag the single-chunk run reads at its end)
 			const int64_t nb = (nseq + PK_SEQ - 1) / PK_SEQ;
-			const uint64_t ntiles = (V + GEN_TILE - 1) / GEN_TILE;
+			const bool tl = use_tiles();
+			const uint64_t ntiles = tl ? (uint64_t)tplan.ntiles : (V + GEN_TILE - 1) / GEN_TILE;
 			TRY(ensure(h, h->pack_state, sizeof(uint64_t) * (size_t)nb));
 			TRY(ensure(h, h->tseq, sizeof(uint32_t) * (size_t)(ntiles + 1)));
 			StageScope sg(h, "generate");
@@ -1162,14 +1259,22 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			ProfScope ps(h, "pack", (double)nseq * (16.0 + 16.0 + 8.0));
 			k_pack_scan<<<(unsigned)nb, PK_NT, 0, s>>>(h->chars.as<uint8_t>(), h->offs.as<uint32_t>(), seq_map, row_base,
 			                                         set_of, nseq, d, h->pk.as<uint64_t>(), h->voff.as<uint64_t>(),
-			                                         h->tseq.as<uint32_t>(), h->pack_state.as<uint64_t>(),
-			                                         LB_SPIN_LIMIT, &ctl_block(h)->tc.error);
+			                                         h->tseq.as<uint32_t>(), tl ? tplan.tile : 0u,
+			                                         h->pack_state.as<uint64_t>(), LB_SPIN_LIMIT,
+			                                         &ctl_block(h)->tc.error);
 			HIP_LAUNCH_CHECK(h);
 			ga.tile_seq = h->tseq.as<uint32_t>();
 		} else {
 			if (v_known)
 				TRY(issue_pack());
-			TRY(tile_seq_table(h, s, nseq, V, &ga.tile_seq));
+			if (use_tiles()) {
+				TRY(ensure(h, h->tseq, sizeof(uint32_t) * (size_t)(tplan.ntiles + 1)));
+				k_tile_first<<<grid_for(nseq, 256), 256, 0, s>>>(h->voff.as<uint64_t>(), nseq, tplan.tile,
+				                                                 (uint32_t)tplan.ntiles, h->tseq.as<uint32_t>());
+				HIP_LAUNCH_CHECK(h);
+			} else {
+				TRY(tile_seq_table(h, s, nseq, V, &ga.tile_seq));
+			}
 		}
 		prologue_done = true;
 		return XTN_OK;
@@ -1308,14 +1413,6 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	}
 	if (cap_recs > (int64_t)INT32_MAX)
 		return fail(h, XTN_ERR_CAPACITY, "chunk of %lld records exceeds 2^31", (long long)cap_recs);
-	TRY(ensure(h, h->recs, sizeof(uint64_t) * (size_t)cap_recs));
-	TRY(ensure(h, h->recs_alt, sizeof(uint64_t) * (size_t)cap_recs));
-	TRY(ensure(h, h->runs_small, sizeof(Run) * (size_t)(cap_recs / 2 + 1)));
-	TRY(ensure(h, h->runs_big, sizeof(Run) * (size_t)(cap_recs / (SMALL_RUN_MAX + 1) + 1)));
-	TRY(ensure(h, h->bstart, sizeof(uint32_t) * (65536 + 1)));
-	TRY(ensure(h, h->bcount, sizeof(uint32_t) * 65536));
-	TRY(ensure(h, h->ctl, sizeof(uint32_t) * CTL_WORDS));
-	TRY(ensure(h, h->ovf, sizeof(uint32_t) * 65536));
 	const int bucket_cap = h->cfg.bucket_capacity > 0 ? std::min(h->cfg.bucket_capacity, h->tune_cap) : h->tune_cap;
 
 	// the grouping plan of a chunk of nrec records
@@ -1323,6 +1420,45 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		g = Grouping{};
 		g.nrec = nrec;
 		g.nseq = nseq;
+		if (use_tiles()) {
+			g.tiles = true;
+			const int64_t cpitch = (tplan.ntiles + 63) / 64 * 64;
+			const int nbins = 1 << tplan.bin_bits, pitch = (nbins + 64 + 63) / 64 * 64;
+			// slots, with room for the 16-byte read at the end of the last run
+			TRY(ensure(h, h->tile_rec, sizeof(uint32_t) * (size_t)(tplan.ntiles * TL_CAP + 4)));
+			TRY(ensure(h, h->tile_offs, sizeof(uint16_t) * (size_t)(tplan.ntiles * pitch)));
+			TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
+			TileArgs& ta = g.ta;
+			ta.pk = h->pk.as<uint64_t>();
+			ta.voff = h->voff.as<uint64_t>();
+			ta.first = h->tseq.as<uint32_t>();
+			ta.out = h->tile_rec.as<uint32_t>();
+			ta.offs = h->tile_offs.as<uint16_t>();
+			ta.ovf = ctr_field(h, offsetof(RunCtrs, coarse_ovf));
+			ta.pitch = pitch;
+			ta.bin_bits = tplan.bin_bits;
+			ta.lb = tplan.idx_bits;
+			ta.sets = set_of ? 1 : 0;
+			BinArgs& bn = g.bn;
+			bn.rec = ta.out;
+			bn.cols = h->tile_cols.as<uint16_t>();
+			bn.first = ta.first;
+			bn.pk = ta.pk;
+			bn.ntiles = tplan.ntiles;
+			bn.cpitch = cpitch;
+			bn.nb = nbins;
+			bn.lb = tplan.idx_bits;
+			bn.idb = idb;
+			bn.distance = d;
+			bn.ctr = h->ctrs.as<RunCtrs>();
+			return XTN_OK;
+		}
+		TRY(ensure(h, h->runs_small, sizeof(Run) * (size_t)(cap_recs / 2 + 1)));
+		TRY(ensure(h, h->runs_big, sizeof(Run) * (size_t)(cap_recs / (SMALL_RUN_MAX + 1) + 1)));
+		TRY(ensure(h, h->bstart, sizeof(uint32_t) * (65536 + 1)));
+		TRY(ensure(h, h->bcount, sizeof(uint32_t) * 65536));
+		TRY(ensure(h, h->ctl, sizeof(uint32_t) * CTL_WORDS));
+		TRY(ensure(h, h->ovf, sizeof(uint32_t) * 65536));
 		g.kernel_cap = h->tune_cap;
 		// bucket bits: the B hash bits right below the chunk bits, B such that
 		// buckets hold about tune_target records; the sort orders the
@@ -1381,6 +1517,20 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	bool used_coarse = false;
 	auto issue_gen = [&](int part, Grouping& g) -> int {
 		used_coarse = false;
+		if (g.tiles) {
+			StageScope sg(h, "generate");
+			ProfScope ps(h, "tiles", (double)V * 4.0 + (double)nseq * 24.0);
+			const unsigned grid = (unsigned)g.bn.ntiles;
+			if (d == 1)
+				k_tiles1<<<grid, TL_NT, 0, s>>>(g.ta);
+			else if (d == 2)
+				k_tiles<2><<<grid, TL_NT, 0, s>>>(g.ta);
+			else
+				k_tiles<3><<<grid, TL_NT, 0, s>>>(g.ta);
+			HIP_LAUNCH_CHECK(h);
+			used_coarse = true;
+			return XTN_OK;
+		}
 		ga.out = h->recs.as<uint64_t>();
 		ga.cap = cap_recs;
 		if (g.fused_hist) {
@@ -1458,6 +1608,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	int64_t out_total = 0, max_round = 0;
 	Grouping g1;
 	bool grouped = false;  // single chunk: the grouping is done once for every round
+	int64_t n_written = 0;  // records the generator wrote, counted once for every round
 	bool no_graph = false;  // a replay needed the host: the rest of this run is eager
 	TailPlan tp;
 	CtlHead head{};
@@ -1516,7 +1667,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				sig.select_nt = h->tune_select_nt;
 				sig.low = h->tail_full ? 0 : h->tune_low;
 				sig.coarse = h->coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
-				sig.pad = 0;
+				sig.pad = h->bin_parts ? 1 : 0;
 			}
 			bool via_graph = false;
 			if (graph_ok && h->graph_exec && sig == h->graph_sig) {
@@ -1565,11 +1716,23 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				TRY(issue_all());
 			}
 			TRY(read_head(h, &head));
-			if (head.rc.coarse_ovf) {
+			n_written = std::max<int64_t>(n_written, (int64_t)head.rc.n_records);
+			if (head.rc.coarse_ovf || (g1.tiles && head.rc.pairs_small > V)) {
 				// a sub-range of the generator's coarse pass overflowed and lost
-				// records: the run again with the separate pass, which these
-				// sequences keep from now on
+				// records, or the tiles and bins outgrew a bound or met more
+				// equal pairs than records (many copies of some strings, which
+				// the run kernels take by their long runs): the run again with
+				// the separate pass, which these sequences keep from now on
 				h->coarse_off = true;
+				grouped = false;
+				prologue_done = false;
+				continue;
+			}
+			if (g1.tiles && head.rc.n_big) {
+				// bins listed more records than fit: the run again with the bins
+				// in parts, which these sequences keep from now on
+				h->bin_parts = true;
+				no_graph = no_graph || via_graph;
 				grouped = false;
 				prologue_done = false;
 				continue;
@@ -1675,12 +1838,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		for (int p = 0; p < nparts; ++p)
 			st.n_records += (int64_t)part_count[p];
 	} else if (used_coarse) {
-		if (head.rc.n_records == 0) {  // no tail ran: the counters were not read back
-			RunCtrs rc{};
-			TRY(read_ctrs(h, &rc));
-			head.rc.n_records = rc.n_records;
-		}
-		st.n_records = (int64_t)head.rc.n_records;
+		st.n_records = n_written;
 	}
 	h->last_pairs = max_round;
 	h->last_unique = st.n_unique;
@@ -1936,7 +2094,7 @@ void xtn_close(xtn_handle* h) {
 		return;
 	(void)hipSetDevice(h->cfg.device);
 	(void)hipStreamSynchronize(h->stream);
-	DBuf* bufs[] = {&h->recs_all, &h->recs_part, &h->seg_cur, &h->seg_ctl, &h->bcount, &h->ctl, &h->chars, &h->offs, &h->pk, &h->voff,
+	DBuf* bufs[] = {&h->tile_rec, &h->tile_offs, &h->tile_cols, &h->recs_all, &h->recs_part, &h->seg_cur, &h->seg_ctl, &h->bcount, &h->ctl, &h->chars, &h->offs, &h->pk, &h->voff,
 	                &h->recs, &h->recs_alt, &h->hist,
 	                &h->scan_tmp, &h->runs_small, &h->runs_big, &h->big_pre, &h->pairs,
 	                &h->pairs_alt, &h->flags, &h->pos, &h->dist, &h->out_pairs, &h->out_dist,
@@ -2135,6 +2293,7 @@ int xtn_set_sequences(xtn_handle* h, const char* chars, const uint32_t* offsets,
 	h->vprefix_d = 0;
 	h->tail_full = false;
 	h->coarse_off = false;
+	h->bin_parts = false;
 	return XTN_OK;
 }
 

@@ -767,7 +767,8 @@ inline SelectFn select_kernel(int distance, int measure, int nt, bool grouped) {
 // then writes its offset and records the generator tiles whose first record
 // it holds (tile_seq, as k_tile_seq); the last one writes voff[n] = V and
 // tile_seq[ceil(V / GEN_TILE)], since it holds record V - 1 (every sequence
-// has at least one variant, itself). The waits are on lower-numbered
+// has at least one variant, itself). With own_tile > 0 the table is
+// k_tile_first's over tiles of that many records instead. The waits are on lower-numbered
 // workgroups, which each XCD dispatches first; a wait past spin_limit
 // raises *error and the host redoes the run.
 constexpr int PK_NT = 1024;
@@ -779,8 +780,9 @@ __global__ __launch_bounds__(PK_NT) void k_pack_scan(const uint8_t* __restrict__
                                                    const uint32_t* __restrict__ seq_map, uint32_t row_base,
                                                    const uint32_t* __restrict__ set_of, int32_t n, int distance,
                                                    uint64_t* __restrict__ pk, uint64_t* __restrict__ voff,
-                                                   uint32_t* __restrict__ tile_seq, uint64_t* __restrict__ state,
-                                                   uint32_t spin_limit, uint32_t* __restrict__ error) {
+                                                   uint32_t* __restrict__ tile_seq, uint32_t own_tile,
+                                                   uint64_t* __restrict__ state, uint32_t spin_limit,
+                                                   uint32_t* __restrict__ error) {
 	__shared__ uint32_t s_tmp[PK_NT / WAVE + 1];
 	__shared__ uint64_t s_prefix;
 	const int t = threadIdx.x;
@@ -815,6 +817,18 @@ __global__ __launch_bounds__(PK_NT) void k_pack_scan(const uint8_t* __restrict__
 			return;
 		const uint64_t e = o + c[u];
 		voff[i] = o;
+		if (own_tile) {  // V < 2^31
+			for (uint32_t bt = (uint32_t)o / own_tile + 1; bt * own_tile <= (uint32_t)e; ++bt)
+				tile_seq[bt] = (uint32_t)i + 1u;
+			if (i == 0)
+				tile_seq[0] = 0;
+			if (i == n - 1) {
+				voff[n] = e;
+				tile_seq[((uint32_t)e + own_tile - 1) / own_tile] = (uint32_t)n;
+			}
+			o = e;
+			continue;
+		}
 		for (uint64_t bt = (o + GEN_TILE - 1) / GEN_TILE; bt * GEN_TILE < e; ++bt)
 			tile_seq[bt] = (uint32_t)i;
 		if (i == n - 1) {
