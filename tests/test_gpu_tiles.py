@@ -51,6 +51,9 @@ def mixed_lengths(seed, n):
     ("smallest", lambda: xtn.synth_nn(103, 1_100, planted=0.3, max_edits=2), 3, 0, None),
     ("ragged", lambda: xtn.synth_nn(104, 70_001, 15.0, 2.5, 6, 30, planted=0.3, max_edits=2), 2, 0, 1),
     ("ragged", lambda: xtn.synth_nn(105, 25_013, 15.0, 2.5, 6, 30, planted=0.3, max_edits=3), 3, 1, 1),
+    ("smallest", lambda: xtn.synth_nn(116, 320, planted=0.4, max_edits=2), 4, 0, None),
+    ("ragged", lambda: xtn.synth_nn(117, 6_007, 15.0, 2.5, 6, 30, planted=0.3, max_edits=3), 4, 0, 1),
+    ("mixed lengths", lambda: mixed_lengths(118, 2_400), 4, 1, None),
     ("mixed lengths", lambda: mixed_lengths(106, 24_000), 2, 0, None),
     ("mixed lengths", lambda: mixed_lengths(107, 6_000), 3, 0, None),
     ("all one length", lambda: xtn.synth_nn(108, 60_000, 18.0, 0.0, 18, 18, planted=0.3, max_edits=1), 1, 0, 1),

@@ -82,6 +82,8 @@ struct xtn_handle {
 	DBuf recs_all, recs_part;  // chunked runs: every record once, then ordered by part
 	DBuf seg_cur, seg_ctl;  // the generator's coarse pass: sub-range cursors, digit tiling
 	DBuf tile_rec, tile_offs, tile_cols;  // tiles ordered by bin, their bin starts by tile and by bin
+	DBuf del_sets_d;  // the deletion sets of distance del_sets_of (xtn_tiles.hpp)
+	int del_sets_of = 0;
 	DBuf pk, voff, recs, recs_alt, hist, scan_tmp, runs_small, runs_big, big_pre, pairs, pairs_alt,
 	    flags, pos, dist, out_pairs, out_dist, ctrs, part_hist, scalar;
 	// overlap-mode workspaces
@@ -804,10 +806,8 @@ struct Grouping {
 
 // ---- tiles and bins of one chunk (xtn_tiles.hpp)
 
-// the bin kernel: 512 threads of 18 groups of four records, two workgroups
-// per CU (one's loads and barriers under the other's work: 430 us against
-// 476 at 1M CDR3s, d = 2, for one of 1024 threads over half as many bins)
-constexpr int BIN_NT = 512, BIN_QPT = 18, BIN_PER_CU = 2;
+// groups of four records that a thread of the bin kernel holds
+constexpr int bin_groups(int d) { return d <= 2 ? 18 : 9; }
 
 struct TilePlan {
 	uint32_t tile = 0;  // records between the starts of two tiles
@@ -831,13 +831,15 @@ TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
 	TilePlan p;
 	p.tile = (uint32_t)tile;
 	p.ntiles = (V + tile - 1) / tile;
-	// index bits for twice the average tile's sequences
-	p.idx_bits = std::min(bits_for((int64_t)(2.0 * (double)tile / avg) + 1), tl_idx_bits(d));
+	// index bits for twice the average tile's sequences (at distance 4 a
+	// short string has a tenth or less of the average's variants, so that
+	// the few sequences of a tile vary more)
+	p.idx_bits = d >= 4 ? tl_idx_bits(d) : std::min(bits_for((int64_t)(2.0 * (double)tile / avg) + 1), tl_idx_bits(d));
 	// The fewest bins whose runs fit the bin kernel's registers (a run, the
 	// records that one tile has for one bin, is Poisson and takes a group per
-	// four of them), and enough of them that bin and record leave 16 keys per
-	// record: two records meet by chance once in 30 or so.
-	const double key_bits = std::log2((double)V) + 4.0;
+	// four of them), and enough of them that bin and record leave 11 keys per
+	// record: two records meet by chance once in 20 or so.
+	const double key_bits = std::log2((double)V) + 3.5;
 	for (p.bin_bits = 6; (1 << p.bin_bits) < TL_BINS_MAX; ++p.bin_bits) {
 		const double lambda = (double)tile / (1 << p.bin_bits);
 		double q = 0, w = std::exp(-lambda);
@@ -848,9 +850,7 @@ TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
 				w *= lambda / k;
 				q += w * ((k + 3) / 4);
 			}
-		// (at distance 3 a neighbouring pair shares a hundred variants and a
-		// fifth of the records may be listed: half as many records a bin)
-		if (q * (double)p.ntiles <= (d == 3 ? 0.45 : 0.92) * BIN_NT * BIN_QPT && p.bin_bits + 30 - p.idx_bits >= key_bits)
+		if (q * (double)p.ntiles <= 0.965 * BIN_NT * bin_groups(d) && p.bin_bits + 32 - tl_len_bits(d) - p.idx_bits >= key_bits)
 			break;
 	}
 	return p;
@@ -1025,12 +1025,11 @@ int issue_buckets(xtn_handle* h, Grouping& g, uint32_t lo, uint32_t hi, int64_t 
 		StageScope sg(h, "pairs");
 		ProfScope ps(h, "bins", (double)g.nrec * 4.0);
 		const unsigned grid = (unsigned)std::min<int64_t>(bn.nb, (int64_t)h->n_cu * BIN_PER_CU);
-		if (h->bin_parts)
-			ranged ? k_bins<BIN_NT, BIN_QPT, true, true><<<grid, BIN_NT, 0, h->stream>>>(bn)
-			       : k_bins<BIN_NT, BIN_QPT, false, true><<<grid, BIN_NT, 0, h->stream>>>(bn);
-		else
-			ranged ? k_bins<BIN_NT, BIN_QPT, true, false><<<grid, BIN_NT, 0, h->stream>>>(bn)
-			       : k_bins<BIN_NT, BIN_QPT, false, false><<<grid, BIN_NT, 0, h->stream>>>(bn);
+		typedef void (*BinFn)(BinArgs);
+		static const BinFn fns[2][2][2] = {
+		    {{k_bins<18, false, false>, k_bins<18, true, false>}, {k_bins<18, false, true>, k_bins<18, true, true>}},
+		    {{k_bins<9, false, false>, k_bins<9, true, false>}, {k_bins<9, false, true>, k_bins<9, true, true>}}};
+		fns[bin_groups(bn.distance) == 9][h->bin_parts][ranged]<<<grid, BIN_NT, 0, h->stream>>>(bn);
 		HIP_LAUNCH_CHECK(h);
 		return XTN_OK;
 	}
@@ -1232,10 +1231,10 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	ga.part_bits = pbits;
 	ga.V = (int64_t)V;
 	ga.set_of = set_of;
-	// one chunk of enough records at distances 1 to 3: tiles ordered by bin
+	// one chunk of enough records at distances 1 to 4: tiles ordered by bin
 	// (xtn_tiles.hpp), until a bound there is outgrown
 	auto use_tiles = [&]() {
-		return nparts == 1 && d <= 3 && (int64_t)V >= TILES_MIN_RECORDS && !h->no_alloc &&
+		return nparts == 1 && d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && !h->no_alloc &&
 		       h->cfg.max_records_per_chunk <= 0 && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
 		       !h->coarse_off && !h->tail_safe;
 	};
@@ -1428,7 +1427,16 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			TRY(ensure(h, h->tile_rec, sizeof(uint32_t) * (size_t)(tplan.ntiles * TL_CAP + 4)));
 			TRY(ensure(h, h->tile_offs, sizeof(uint16_t) * (size_t)(tplan.ntiles * pitch)));
 			TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
+			if (d >= 2 && h->del_sets_of != d) {
+				static const std::vector<uint32_t> sets[TL_MAX_D - 1] = {del_sets(2), del_sets(3), del_sets(4)};
+				const std::vector<uint32_t>& v = sets[d - 2];
+				TRY(ensure(h, h->del_sets_d, sizeof(uint32_t) * (size_t)tl_sets(TL_MAX_D)));
+				HIP_TRY(h, hipMemcpyAsync(h->del_sets_d.p, v.data(), sizeof(uint32_t) * v.size(),
+				                          hipMemcpyHostToDevice, s));
+				h->del_sets_of = d;
+			}
 			TileArgs& ta = g.ta;
+			ta.del = h->del_sets_d.as<uint32_t>();
 			ta.pk = h->pk.as<uint64_t>();
 			ta.voff = h->voff.as<uint64_t>();
 			ta.first = h->tseq.as<uint32_t>();
@@ -1448,6 +1456,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			bn.cpitch = cpitch;
 			bn.nb = nbins;
 			bn.lb = tplan.idx_bits;
+			bn.len_bits = tl_len_bits(d);
+			bn.key_low = std::max(bn.lb + bn.len_bits, tplan.bin_bits);
 			bn.idb = idb;
 			bn.distance = d;
 			bn.ctr = h->ctrs.as<RunCtrs>();
@@ -1525,8 +1535,10 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				k_tiles1<<<grid, TL_NT, 0, s>>>(g.ta);
 			else if (d == 2)
 				k_tiles<2><<<grid, TL_NT, 0, s>>>(g.ta);
-			else
+			else if (d == 3)
 				k_tiles<3><<<grid, TL_NT, 0, s>>>(g.ta);
+			else
+				k_tiles<4><<<grid, TL_NT, 0, s>>>(g.ta);
 			HIP_LAUNCH_CHECK(h);
 			used_coarse = true;
 			return XTN_OK;
@@ -2094,7 +2106,7 @@ void xtn_close(xtn_handle* h) {
 		return;
 	(void)hipSetDevice(h->cfg.device);
 	(void)hipStreamSynchronize(h->stream);
-	DBuf* bufs[] = {&h->tile_rec, &h->tile_offs, &h->tile_cols, &h->recs_all, &h->recs_part, &h->seg_cur, &h->seg_ctl, &h->bcount, &h->ctl, &h->chars, &h->offs, &h->pk, &h->voff,
+	DBuf* bufs[] = {&h->del_sets_d, &h->tile_rec, &h->tile_offs, &h->tile_cols, &h->recs_all, &h->recs_part, &h->seg_cur, &h->seg_ctl, &h->bcount, &h->ctl, &h->chars, &h->offs, &h->pk, &h->voff,
 	                &h->recs, &h->recs_alt, &h->hist,
 	                &h->scan_tmp, &h->runs_small, &h->runs_big, &h->big_pre, &h->pairs,
 	                &h->pairs_alt, &h->flags, &h->pos, &h->dist, &h->out_pairs, &h->out_dist,

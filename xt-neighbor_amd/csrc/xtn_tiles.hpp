@@ -1,4 +1,4 @@
-// xtn_tiles.hpp -- the record path of one key-space chunk at distances 1 to 3:
+// xtn_tiles.hpp -- the record path of one key-space chunk at distances 1 to 4:
 // deletion variants generated once, ordered once, and grouped where they lie.
 //
 //   k_tiles / k_tiles1  a workgroup generates the deletion variants of a range of
@@ -24,7 +24,7 @@
 // takes another 45 us off their sort.
 // Per record this moves 4 bytes out and 4 back, against 8 out, 8 in, 8 out
 // and 8 in for the sub-range path (k_gen<GEN_COARSE>, k_region_scatter,
-// k_bucket), which stays for distances above 3, for searches that ask for
+// k_bucket), which stays for distances above 4, for searches that ask for
 // the separate pass, and for inputs that outgrow a bound here (a bin, a
 // group of more than TL_GROUP_MAX equal keys, a tile of very short strings):
 // such a run raises coarse_ovf and is redone there.
@@ -32,6 +32,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <vector>
 
 #include "xtn_kernels.hpp"
 
@@ -41,14 +43,23 @@ constexpr int TL_NT = 1024;
 constexpr int TL_CAP_BITS = 15;
 constexpr int TL_CAP = 1 << TL_CAP_BITS;  // record slots of a tile
 constexpr int TL_IT = TL_CAP / TL_NT;     // records of a thread
-constexpr int TL_BINS_MAX = 4096;
+constexpr int TL_BINS_MAX = 8192;
 constexpr uint32_t TL_NONE = 0xFFFFFFFFu;  // no record (a tile's last index is never used)
 constexpr int TL_GROUP_MAX = 1024;         // equal keys before a record: a longer group is left to the run kernels
 
 // sequences a tile may hold and the bits of an index in it, by distance: the
 // tables of a tile's sequences share LDS with its records
-__host__ __device__ constexpr int tl_seqs(int d) { return d == 1 ? 4095 : d == 2 ? 768 : 480; }
-__host__ __device__ constexpr int tl_idx_bits(int d) { return d == 1 ? 12 : d == 2 ? 10 : 9; }
+__host__ __device__ constexpr int tl_seqs(int d) { return d == 1 ? 4095 : d == 2 ? 768 : d == 3 ? 480 : 127; }
+__host__ __device__ constexpr int tl_idx_bits(int d) { return d == 1 ? 12 : d == 2 ? 10 : d == 3 ? 9 : 7; }
+// bits of a variant's length kept in its record: enough to tell d + 1
+// numbers of deletions apart
+__host__ __device__ constexpr int tl_len_bits(int d) { return d <= 3 ? 2 : 3; }
+constexpr int TL_MAX_D = 4;  // at 5 half of the records are listed and the bins go in parts: 2.4 ms against
+                             // 2.0 for 9000 CDR3s on the sub-range path
+constexpr int DEL_SETS4 = DEL_SETS3 + 3060;
+__host__ __device__ constexpr int tl_sets(int d) {
+	return d == 1 ? DEL_SETS1 : d == 2 ? DEL_SETS2 : d == 3 ? DEL_SETS3 : DEL_SETS4;
+}
 
 // The key of a variant is the exclusive or of one random word per slot and
 // residue (tabulation hashing: Zobrist 1970, Carter and Wegman 1979). A
@@ -89,19 +100,48 @@ struct TileArgs {
 	const uint64_t* pk;
 	const uint64_t* voff;
 	const uint32_t* first;   // first sequence of each tile, [ntiles] = n
+	const uint32_t* del;     // the deletion sets (del_sets)
 	uint32_t* out;           // TL_CAP slots per tile
 	uint16_t* offs;          // a row of `pitch` per tile: the start of each bin, then the tile's total
 	unsigned long long* ovf;
 	int32_t pitch;
-	int32_t bin_bits;        // 6..12
+	int32_t bin_bits;        // 6..13
 	int32_t lb;              // index bits of a record
 	int32_t sets;            // the prefixes carry query sets
 };
 
-// A record: key bits below the bin, the variant's length mod 4, the index in
-// the tile. Equal keys mean equal records above the index.
+// A record: key bits below the bin, the low bits of the variant's length, the
+// index in the tile. Equal keys mean equal records above the index.
+template <int D>
 __device__ __forceinline__ uint32_t tile_record(uint32_t h, int bin_bits, uint32_t len, int lb, uint32_t idx) {
-	return ((h << bin_bits) & ~((4u << lb) - 1u)) | ((len & 3u) << lb) | idx;
+	constexpr uint32_t LM = (1u << tl_len_bits(D)) - 1u;
+	return ((h << bin_bits) & ~(((LM + 1u) << lb) - 1u)) | ((len & LM) << lb) | idx;
+}
+
+// The deletion sets of at most d positions, ordered by their largest position
+// as c_del_tables is: positions ascending, five bits each from bit 0, NO_DEL
+// above the real ones, the number of deletions from bit 25.
+inline std::vector<uint32_t> del_sets(int d) {
+	std::vector<uint32_t> r;
+	auto put = [&](const int* q, int m) {
+		uint32_t e = (uint32_t)m << 25;
+		for (int k = 0; k < TL_MAX_D; ++k)
+			e |= (uint32_t)(k < m ? q[k] : NO_DEL) << (5 * k);
+		r.push_back(e);
+	};
+	put(nullptr, 0);
+	for (int top = 0; top < MAX_PREFIX; ++top)
+		for (uint32_t below = 0; below < 1u << top; ++below) {
+			if (__builtin_popcount(below) >= d)
+				continue;
+			int q[TL_MAX_D], m = 0;
+			for (int i = 0; i < top; ++i)
+				if ((below >> i) & 1u)
+					q[m++] = i;
+			q[m++] = top;
+			put(q, m);
+		}
+	return r;
 }
 
 // the bins' counts (16 bits each, two to a word) turned into their starts,
@@ -148,23 +188,24 @@ __device__ __forceinline__ void tile_refuse(const TileArgs& a, uint16_t* row, in
 		atomicOr(a.ovf, 1ull);
 }
 
-// Distances 2 and 3. The deletion sets of a prefix come in the order of
-// their largest position (c_del_tables), a thread takes consecutive records,
+// Distances 2 to 4. The deletion sets of a prefix come in the order of
+// their largest position (del_sets), a thread takes consecutive records,
 // and the record's rank inside its bin comes from the same LDS atomic that
 // counts it; the records stay in registers until the tables are dead and
-// the ordered tile takes their LDS.
+// the ordered tile takes their LDS. At distance 4 the colex unranking this
+// replaces took 1615 us for 1.05e8 variants (50 000 CDR3s).
 template <int D>
 __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
-	static_assert(D == 2 || D == 3, "distance 1 has a kernel of its own");
+	static_assert(D >= 2 && D <= TL_MAX_D, "distance 1 has a kernel of its own");
 	constexpr int SEQS = tl_seqs(D);
 	constexpr int W = MAX_PREFIX + 1;            // words of one A_k
 	constexpr int ST = D * W + (D & 1 ? 0 : 1);  // odd: the threads of a wave build side by side without bank conflicts
-	constexpr int NSETS = D == 2 ? DEL_SETS2 : DEL_SETS3;
+	constexpr int NSETS = tl_sets(D);
 	__shared__ union {
 		uint32_t rec[TL_CAP];
 		struct {
 			uint32_t terms[MAX_PREFIX][32];
-			uint32_t del[NSETS];      // positions in bytes 0..2, their number in byte 3
+			uint32_t del[NSETS];
 			uint32_t tab[SEQS * ST];
 			uint32_t info[SEQS];      // run_mask, the length above it
 			uint16_t start[SEQS + 2];  // the sequence's first record in the tile
@@ -196,11 +237,8 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 		s_cnt[i] = 0;
 	for (int i = t; i < MAX_PREFIX * 32; i += TL_NT)
 		(&u.s.terms[0][0])[i] = (&c_tile_terms.t[0][0])[i];
-	for (int i = t; i < NSETS; i += TL_NT) {
-		const uint32_t e = D == 2 ? c_del_tables.d2[i] : c_del_tables.d3[i];
-		const uint32_t m = ((e & 0xFFu) < MAX_PREFIX) + (((e >> 8) & 0xFFu) < MAX_PREFIX) + ((e >> 16) < MAX_PREFIX);
-		u.s.del[i] = e | (m << 24);
-	}
+	for (int i = t; i < NSETS; i += TL_NT)
+		u.s.del[i] = a.del[i];
 	__syncthreads();
 	for (int i = t; i < cnt; i += TL_NT) {
 		const uint64_t lo = a.pk[2 * (int64_t)(s0 + i)];
@@ -268,15 +306,21 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 			if (r + it < total) {
 				const uint32_t e = u.s.del[k];
 				const uint32_t* tab = &u.s.tab[idx * ST];
-				uint32_t h = tab[e & 0xFFu] ^ tab[W + ((e >> 8) & 0xFFu)];
-				if constexpr (D == 3)
-					h ^= tab[2 * W + ((e >> 16) & 0xFFu)];
-				if (!dup_deletion_set(e & 0xFFFFFFu, info)) {
+				uint32_t h = 0, gone = 0;
+#pragma unroll
+				for (int j = 0; j < D; ++j) {
+					const uint32_t q = (e >> (5 * j)) & 31u;
+					h ^= tab[j * W + q];
+					gone |= 1u << q;
+				}
+				// repeated variants left out as dup_deletion_set does (NO_DEL
+				// lies on the first length bit: masked)
+				if ((gone & info & ~(gone << 1) & ((1u << MAX_PREFIX) - 1u)) == 0u) {
 					const uint32_t bin = h >> (32 - a.bin_bits);
 					const int sh = (int)(bin & 1u) * 16;
 					const uint32_t old = atomicAdd(&s_cnt[bin >> 1], 1u << sh);
 					at[it] = (bin << 16) | ((old >> sh) & 0xFFFFu);
-					rec[it] = tile_record(h, a.bin_bits, (info >> MAX_PREFIX) - (e >> 24), a.lb, (uint32_t)idx);
+					rec[it] = tile_record<D>(h, a.bin_bits, (info >> MAX_PREFIX) - (e >> 25), a.lb, (uint32_t)idx);
 				}
 				if (++k == nv && idx + 1 < cnt) {
 					++idx;
@@ -362,7 +406,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles1(TileArgs a) {
 		const uint32_t bin = h >> (32 - a.bin_bits);
 		const int sh = (int)(bin & 1u) * 16;
 		const uint32_t pos = (atomicAdd(&s_cnt[bin >> 1], 1u << sh) >> sh) & 0xFFFFu;
-		s_rec[pos] = tile_record(h, a.bin_bits, len, a.lb, idx);
+		s_rec[pos] = tile_record<1>(h, a.bin_bits, len, a.lb, idx);
 	});
 	__syncthreads();
 	tile_out(s_rec, a.out + tile * TL_CAP, total);
@@ -420,6 +464,11 @@ __global__ __launch_bounds__(256) void k_tile_cols(const uint16_t* __restrict__ 
 
 // ------------------------------------------------------------- pairs --
 
+// threads of a bin's workgroup, two workgroups per CU (one's loads and
+// barriers under the other's work: 430 us against 476 at 1M CDR3s, d = 2, for
+// one of 1024 threads over half as many bins)
+constexpr int BIN_NT = 512, BIN_PER_CU = 2;
+
 struct BinArgs {
 	const uint32_t* rec;     // the tiles
 	const uint16_t* cols;    // k_tile_cols
@@ -428,6 +477,9 @@ struct BinArgs {
 	int64_t ntiles, cpitch;
 	int32_t nb;
 	int32_t lb;              // index bits of a record
+	int32_t len_bits;        // length bits above them
+	int32_t key_low;         // lowest key bit of a record (above it the key's bits below the bin; zeros may lie
+	                         // between it and the length bits)
 	int32_t idb;
 	int32_t distance;
 	uint32_t id_lo, id_hi;   // only pairs whose smaller id lies in [id_lo, id_hi)
@@ -454,13 +506,14 @@ __device__ __forceinline__ uint32_t residue_set(uint64_t lo, uint32_t hi26) {
 // for every further deletion as well (about a dozen at distance 2, a hundred
 // at 3): the pair goes out only from the variant with the fewest deletions, which
 // both sides hold and whose length is known from the two strings.
-__device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint32_t ia, uint32_t ib, uint32_t len4,
-                                          int distance) {
+__device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint32_t ia, uint32_t ib, uint32_t len,
+                                          int len_bits, int distance) {
 	const uint64_t la = pk[2 * (int64_t)ia], wa = pk[2 * (int64_t)ia + 1];
 	const uint64_t lb = pk[2 * (int64_t)ib], wb = pk[2 * (int64_t)ib + 1];
 	const uint32_t ha = (uint32_t)wa & PK_SLOT_HI_MASK, hb = (uint32_t)wb & PK_SLOT_HI_MASK;
 	const int La = (int)(wa >> 56), Lb = (int)(wb >> 56);
-	const int ma = (La - (int)len4) & 3, mb = (Lb - (int)len4) & 3;  // deletions on each side, distance <= 3
+	const int lm = (1 << len_bits) - 1;
+	const int ma = (La - (int)len) & lm, mb = (Lb - (int)len) & lm;  // deletions on each side, at most the distance
 	if (ma > distance || mb > distance || La - ma != Lb - mb)
 		return false;
 	if (__popc(residue_set(la, ha) ^ residue_set(lb, hb)) > ma + mb)
@@ -495,7 +548,7 @@ __device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint3
 
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// Bins over resident workgroups. NT threads hold QPT groups of four records
+// Bins over resident workgroups. BIN_NT threads hold QPT groups of four records
 // each.
 //   1. the runs of the bin (k_tile_cols' row and the next one) are listed as
 //      groups of up to four records, and every group is loaded into
@@ -511,18 +564,21 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // records by their top key bits; without it such a bin raises bins_ovf
 // (n_big) and the host runs the instantiation that has it, which the common
 // case would pay for in registers (8% of the kernel).
-template <int NT, int QPT, bool RANGED, bool PARTS>
-__global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
-	constexpr int B1 = 18, B2 = 16, HBITS = 12;
-	static_assert(NT == 512 && QPT == 18, "bitmaps of 7 to 8 bits and a quarter of that per record");
+// QPT 18: bins of up to 36864 slots, an eighth of whose records may be
+// listed; QPT 9 (distances 3 and 4, where a neighbouring pair shares hundreds
+// of variants): half as many slots and a list for half of their records.
+template <int QPT, bool RANGED, bool PARTS>
+__global__ __launch_bounds__(BIN_NT, 4) void k_bins(BinArgs a) {
+	constexpr int NT = BIN_NT;
+	constexpr int B1 = 18, B2 = 16, HBITS = QPT == 18 ? 12 : 11;
+	static_assert(QPT == 18 || QPT == 9, "bitmaps of 7 bits or more and a quarter of that per record");
 	constexpr int QCAP = NT * QPT;
-	constexpr int AREA1 = (1 << B1) / 8;
-	constexpr int SVC = AREA1 / 6 / 64 * 64;  // records listed in step 3
+	constexpr int SVC = QPT == 18 ? (1 << B1) / 8 / 6 / 64 * 64 : 7168;  // records listed in step 3
 	constexpr int HEADS = 1 << HBITS;
-	constexpr int PLC = (QCAP * 4 - HEADS * 4 - SVC * 2) / 4;
+	constexpr int PLC = QPT == 18 ? (QCAP * 4 - HEADS * 4 - SVC * 2) / 4 : 1024;
 	static_assert(PLC >= NT, "room for pairs beside the lists");
 	__shared__ union {
-		uint32_t bm1[AREA1 / 4];
+		uint32_t bm1[(1 << B1) / 32];
 		struct {
 			uint32_t rec[SVC];
 			uint16_t tile[SVC];
@@ -540,7 +596,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 	__shared__ uint32_t s_tmp[NT / WAVE + 1];
 	__shared__ unsigned long long s_base;
 	__shared__ uint32_t s_nsv, s_npl;
-	static_assert(sizeof(u1) == AREA1 && sizeof(u2) == QCAP * 4, "lists fit the dead areas");
+	static_assert(sizeof(u1) + sizeof(u2) + sizeof(s_bm2) <= 79 * 1024, "two workgroups per CU");
 	const int t = threadIdx.x;
 	const int lane = lane_id();
 	const int G = (int)gridDim.x;
@@ -550,14 +606,14 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 	const int step = by_xcd ? G / 8 : G;
 	const int b_end = by_xcd ? (int)(blockIdx.x % 8 + 1) * (a.nb / 8) : a.nb;
 	const int b_beg = by_xcd ? (int)(blockIdx.x % 8) * (a.nb / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-	const int s1 = 32 - B1 > a.lb ? 32 - B1 : a.lb;
+	const int s1 = 32 - B1 > a.key_low ? 32 - B1 : a.key_low;
 	const uint32_t lmask = (1u << a.lb) - 1u;
 
 	int lp = 0, part = 0;  // PARTS: part of 2^lp; the next bin starts with as many
 	bool fresh = true;
 	for (int b = b_beg; b < b_end;) {  // uniform
 		if (!PARTS || fresh) {
-			for (int i = t; i < AREA1 / 16; i += NT)
+			for (int i = t; i < (1 << B1) / 128; i += NT)
 				reinterpret_cast<uint4*>(u1.bm1)[i] = make_uint4(0u, 0u, 0u, 0u);
 			for (int i = t; i < (1 << B2) / 128; i += NT)
 				reinterpret_cast<uint4*>(s_bm2)[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -639,7 +695,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 						const uint32_t x = r >> s1;
 						const uint32_t old = atomicOr(&u1.bm1[x >> 5], 1u << (x & 31u));
 						if ((old >> (x & 31u)) & 1u) {
-							const uint32_t y = (r >> a.lb) & ((1u << B2) - 1u);
+							const uint32_t y = (r >> a.key_low) & ((1u << B2) - 1u);
 							atomicOr(&s_bm2[y >> 5], 1u << (y & 31u));
 						}
 					}
@@ -663,7 +719,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 #pragma unroll
 			for (int j = 0; j < 4; ++j) {
 				const uint32_t r = v[k][j];
-				const uint32_t y = (r >> a.lb) & ((1u << B2) - 1u);
+				const uint32_t y = (r >> a.key_low) & ((1u << B2) - 1u);
 				uint32_t on = r != TL_NONE ? (s_bm2[y >> 5] >> (y & 31u)) & 1u : 0u;
 				if constexpr (PARTS)
 					on = (r >> 1) >> (31 - lp) == (uint32_t)part ? on : 0u;
@@ -712,7 +768,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 			u2.g.head[i] = 0xFFFFu;
 		__syncthreads();
 		for (uint32_t i = t; i < nsv; i += NT)
-			u2.g.next[i] = (uint16_t)atomicExch(&u2.g.head[(u1.sv.rec[i] >> (a.lb + 2)) & (HEADS - 1)], i);
+			u2.g.next[i] = (uint16_t)atomicExch(&u2.g.head[(u1.sv.rec[i] >> a.key_low) & (HEADS - 1)], i);
 		__syncthreads();
 		auto candidate = [&](uint32_t i, uint32_t n, uint64_t* p) -> bool {
 			const uint32_t ri = u1.sv.rec[i], rn = u1.sv.rec[n];
@@ -723,7 +779,8 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 			if (RANGED && (lo < a.id_lo || lo >= a.id_hi))
 				return false;
 			*p = ((uint64_t)lo << a.idb) | hi;
-			return tile_pair(a.pk, lo, hi, (ri >> a.lb) & 3u, a.distance);
+			return tile_pair(a.pk, lo, hi, (ri >> a.lb) & ((1u << a.len_bits) - 1u), a.len_bits,
+			                 a.distance);
 		};
 		for (uint32_t i = t; i < nsv; i += NT) {
 			const uint32_t r = u1.sv.rec[i];
