@@ -28,6 +28,7 @@
 #include <cstdio>
 #include <cstring>
 #include <cstdlib>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <vector>
@@ -137,6 +138,8 @@ struct xtn_handle {
 	void* pin = nullptr;  // pinned upload staging (xtn_set_sequences, a server worker's queries)
 	size_t pin_bytes = 0;
 	hipEvent_t pin_ev[2] = {nullptr, nullptr};
+	void* dl_pin = nullptr;  // pinned readback staging (fetch): two halves of DL_HALF bytes
+	hipEvent_t dl_ev[2] = {nullptr, nullptr};
 	void* out_pin = nullptr;  // pinned output staging of xtn_perform (two chunks of pairs and distances)
 	size_t out_pin_bytes = 0;
 	double serve_ratio = 0;  // a server worker's candidates per query record so far
@@ -497,11 +500,75 @@ int radix_sort(xtn_handle* h, DBuf& keys, DBuf& keys_alt, DBuf* vals, DBuf* vals
 	return XTN_OK;
 }
 
-int read_ctrs(xtn_handle* h, RunCtrs* out) {
-	HIP_TRY(h, hipMemcpyAsync(out, h->ctrs.p, sizeof(RunCtrs), hipMemcpyDeviceToHost, h->stream));
-	HIP_SYNC(h, h->stream);
+// Device bytes to host memory of any kind, waited for: through the handle's
+// pinned staging, one half filled by the copy engine while the other goes to
+// its place. A copy into unpinned memory goes through the runtime's own
+// staging instead: 22 against 13 us for the control block, 148 against 95 for
+// 2.7 MB, 619 against 240 for 11.5 MB.
+struct FetchPart {
+	void* dst;
+	const void* src;
+	size_t bytes;
+};
+constexpr size_t DL_HALF = (size_t)1 << 20;
+
+int fetch(xtn_handle* h, std::initializer_list<FetchPart> parts, hipStream_t s) {
+	if (!h->dl_pin && !h->no_alloc) {  // (the no-allocation form keeps no pinned memory)
+		if (hipHostMalloc(&h->dl_pin, 2 * DL_HALF, hipHostMallocDefault) != hipSuccess) {
+			(void)hipGetLastError();
+			h->dl_pin = nullptr;
+		}
+		for (hipEvent_t& e : h->dl_ev)
+			if (h->dl_pin && !e)
+				HIP_TRY(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+	}
+	size_t total = 0;
+	for (const FetchPart& p : parts)
+		total += (p.bytes + 15) & ~(size_t)15;
+	char* pin = static_cast<char*>(h->dl_pin);
+	if (!pin || total <= DL_HALF) {  // one wait for all
+		size_t at = 0;
+		for (const FetchPart& p : parts) {
+			if (p.bytes)
+				HIP_TRY(h, hipMemcpyAsync(pin ? pin + at : p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
+			at += (p.bytes + 15) & ~(size_t)15;
+		}
+		HIP_SYNC(h, s);
+		at = 0;
+		for (const FetchPart& p : parts) {
+			if (pin && p.bytes)
+				memcpy(p.dst, pin + at, p.bytes);
+			at += (p.bytes + 15) & ~(size_t)15;
+		}
+		return XTN_OK;
+	}
+	char* to[2] = {nullptr, nullptr};  // where a half's bytes go
+	size_t len[2] = {0, 0};
+	int half = 0;
+	auto drain = [&](int b) -> int {
+		if (!to[b])
+			return XTN_OK;
+		HIP_TRY(h, hipEventSynchronize(h->dl_ev[b]));
+		memcpy(to[b], pin + b * DL_HALF, len[b]);
+		to[b] = nullptr;
+		return XTN_OK;
+	};
+	for (const FetchPart& p : parts)
+		for (size_t off = 0; off < p.bytes; off += DL_HALF, half ^= 1) {
+			TRY(drain(half));
+			len[half] = std::min(DL_HALF, p.bytes - off);
+			to[half] = static_cast<char*>(p.dst) + off;
+			HIP_TRY(h, hipMemcpyAsync(pin + half * DL_HALF, static_cast<const char*>(p.src) + off, len[half],
+			                          hipMemcpyDeviceToHost, s));
+			HIP_TRY(h, hipEventRecord(h->dl_ev[half], s));
+		}
+	TRY(drain(half));
+	TRY(drain(half ^ 1));
+	++h->stats.n_syncs;
 	return XTN_OK;
 }
+
+int read_ctrs(xtn_handle* h, RunCtrs* out) { return fetch(h, {{out, h->ctrs.p, sizeof(RunCtrs)}}, h->stream); }
 
 double now_ms() {
 	using namespace std::chrono;
@@ -552,11 +619,7 @@ int zero_ctl(xtn_handle* h, bool counters, bool tail) {
 	return XTN_OK;
 }
 
-int read_head(xtn_handle* h, CtlHead* out) {
-	HIP_TRY(h, hipMemcpyAsync(out, h->ctrs.p, sizeof(CtlHead), hipMemcpyDeviceToHost, h->stream));
-	HIP_SYNC(h, h->stream);
-	return XTN_OK;
-}
+int read_head(xtn_handle* h, CtlHead* out) { return fetch(h, {{out, h->ctrs.p, sizeof(CtlHead)}}, h->stream); }
 
 // Global path for one bucket that does not fit the LDS tile: sort the
 // segment by the run bits, list its runs, emit the pairs of every run whose
@@ -1181,8 +1244,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	const bool v_known = V > 0;
 	if (!v_known) {
 		TRY(issue_pack());
-		HIP_TRY(h, hipMemcpyAsync(&V, h->voff.as<uint64_t>() + nseq, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-		HIP_SYNC(h, s);
+		TRY(fetch(h, {{&V, h->voff.as<uint64_t>() + nseq, sizeof(uint64_t)}}, s));
 	}
 	st.n_variants = (int64_t)V;
 
@@ -1957,9 +2019,7 @@ int overlap_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callba
 	HIP_LAUNCH_CHECK(h);
 	TRY(scan_excl<uint32_t>(h, h->flags.as<uint32_t>(), h->pos.as<uint32_t>(), n, h->pos.as<uint32_t>() + n));
 	uint32_t U = 0, ctl[2] = {0, 0};
-	HIP_TRY(h, hipMemcpyAsync(&U, h->pos.as<uint32_t>() + n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-	HIP_TRY(h, hipMemcpyAsync(ctl, h->scalar.p, sizeof(ctl), hipMemcpyDeviceToHost, s));
-	HIP_SYNC(h, s);
+	TRY(fetch(h, {{&U, h->pos.as<uint32_t>() + n, sizeof(uint32_t)}, {ctl, h->scalar.p, sizeof(ctl)}}, s));
 	if (ctl[1] != 0xFFFFFFFFu)
 		return fail(h, XTN_ERR_ARG, "negative repertoire index at row %u", ctl[1]);
 	const int32_t R = (int32_t)ctl[0];
@@ -2008,8 +2068,7 @@ int overlap_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callba
 	TRY(scan_excl<uint32_t>(h, h->ov_present.as<uint32_t>(), h->pos.as<uint32_t>(), RR,
 	                        h->pos.as<uint32_t>() + RR));
 	uint32_t nout = 0;
-	HIP_TRY(h, hipMemcpyAsync(&nout, h->pos.as<uint32_t>() + RR, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-	HIP_SYNC(h, s);
+	TRY(fetch(h, {{&nout, h->pos.as<uint32_t>() + RR, sizeof(uint32_t)}}, s));
 	TRY(ensure(h, h->out_pairs, sizeof(int2) * (size_t)std::max<uint32_t>(nout, 1)));
 	TRY(ensure(h, h->ov_cnt, sizeof(unsigned long long) * (size_t)std::max<uint32_t>(nout, 1)));
 	k_matrix_emit<<<grid_for(RR, 256), 256, 0, s>>>(h->ov_present.as<uint32_t>(), h->pos.as<uint32_t>(),
@@ -2018,11 +2077,8 @@ int overlap_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callba
 	HIP_LAUNCH_CHECK(h);
 	std::vector<xtn_int2> hp(std::max<uint32_t>(nout, 1));
 	std::vector<uint64_t> hv(std::max<uint32_t>(nout, 1));
-	if (nout) {
-		HIP_TRY(h, hipMemcpyAsync(hp.data(), h->out_pairs.p, sizeof(xtn_int2) * nout, hipMemcpyDeviceToHost, s));
-		HIP_TRY(h, hipMemcpyAsync(hv.data(), h->ov_cnt.p, sizeof(uint64_t) * nout, hipMemcpyDeviceToHost, s));
-	}
-	HIP_SYNC(h, s);
+	TRY(fetch(h, {{hp.data(), h->out_pairs.p, sizeof(xtn_int2) * nout}, {hv.data(), h->ov_cnt.p, sizeof(uint64_t) * nout}},
+	          s));
 	collect_profile(h);
 	st.n_sequences = U;
 	st.n_output = nout;
@@ -2126,7 +2182,9 @@ void xtn_close(xtn_handle* h) {
 		(void)hipHostFree(h->pin);
 	if (h->out_pin)
 		(void)hipHostFree(h->out_pin);
-	for (hipEvent_t e : h->pin_ev)
+	if (h->dl_pin)
+		(void)hipHostFree(h->dl_pin);
+	for (hipEvent_t e : {h->pin_ev[0], h->pin_ev[1], h->dl_ev[0], h->dl_ev[1]})
 		if (e)
 			(void)hipEventDestroy(e);
 	if (h->graph_exec)
@@ -2329,11 +2387,8 @@ int xtn_copy_nn_output(xtn_handle* h, xtn_int2* pairs, int8_t* distances, int64_
 	const int64_t n = std::min<int64_t>(cap, h->out_len);
 	if (n <= 0)
 		return XTN_OK;
-	HIP_TRY(h, hipMemcpyAsync(pairs, h->out_pairs.p, sizeof(xtn_int2) * (size_t)n,
-	                          hipMemcpyDeviceToHost, h->stream));
-	HIP_TRY(h, hipMemcpyAsync(distances, h->out_dist.p, (size_t)n, hipMemcpyDeviceToHost, h->stream));
-	HIP_SYNC(h, h->stream);
-	return XTN_OK;
+	return fetch(h, {{pairs, h->out_pairs.p, sizeof(xtn_int2) * (size_t)n}, {distances, h->out_dist.p, (size_t)n}},
+	             h->stream);
 }
 
 int xtn_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callback, void* user) {
@@ -2424,12 +2479,9 @@ static int copy_output(xtn_handle* h, std::vector<xtn_int2>& pairs, std::vector<
 	const int64_t n = h->out_len;
 	pairs.resize((size_t)std::max<int64_t>(n, 1));
 	dist.resize((size_t)std::max<int64_t>(n, 1));
-	if (n > 0) {
-		HIP_TRY(h, hipMemcpyAsync(pairs.data(), h->out_pairs.p, sizeof(xtn_int2) * (size_t)n,
-		                          hipMemcpyDeviceToHost, h->stream));
-		HIP_TRY(h, hipMemcpyAsync(dist.data(), h->out_dist.p, (size_t)n, hipMemcpyDeviceToHost, h->stream));
-		HIP_SYNC(h, h->stream);
-	}
+	if (n > 0)
+		TRY(fetch(h, {{pairs.data(), h->out_pairs.p, sizeof(xtn_int2) * (size_t)n}, {dist.data(), h->out_dist.p, (size_t)n}},
+		          h->stream));
 	return XTN_OK;
 }
 
@@ -3179,12 +3231,10 @@ int serve_query(xtn_server* sv, xtn_handle* w, const ServeRequest& rq, ServeResu
 	const int64_t nout = (int64_t)head.n_out;
 	res->pairs.resize((size_t)nout);
 	res->dist.resize((size_t)nout);
-	if (nout) {
-		HIP_TRY(w, hipMemcpyAsync(res->pairs.data(), w->out_pairs.p, sizeof(xtn_int2) * (size_t)nout,
-		                          hipMemcpyDeviceToHost, s));
-		HIP_TRY(w, hipMemcpyAsync(res->dist.data(), w->out_dist.p, (size_t)nout, hipMemcpyDeviceToHost, s));
-		HIP_SYNC(w, s);
-	}
+	if (nout)
+		TRY(fetch(w, {{res->pairs.data(), w->out_pairs.p, sizeof(xtn_int2) * (size_t)nout},
+		              {res->dist.data(), w->out_dist.p, (size_t)nout}},
+		          s));
 	return XTN_OK;
 }
 
