@@ -44,6 +44,8 @@ using namespace xtn;
 
 namespace {
 
+constexpr int DEFAULT_BUCKET_TARGET = 2200;  // mean records per bucket
+
 struct DBuf {
 	void* p = nullptr;
 	size_t cap = 0;
@@ -121,7 +123,7 @@ struct xtn_handle {
 	bool graph_coarse = false;   // the graph's generator does the coarse pass
 	// engine parameters the autotuner chooses (xtn_set_tuning / xtn_autotune)
 	int tune_cap = 3072;      // bucket kernel instantiation: 2048, 3072 or 4096 records
-	int tune_target = 2200;   // mean records per bucket
+	int tune_target = DEFAULT_BUCKET_TARGET;  // mean records per bucket
 	int tune_sort_nt = 512;   // threads of a pair-sort tile: 256, 512 or 1024
 	int tune_sort_tile = 4096;  // keys of a pair-sort tile: 4096 or 8192
 	int tune_select_nt = 256;   // threads of a select tile (8 candidates each): 256 or 512
@@ -869,14 +871,12 @@ struct Grouping {
 
 // ---- tiles and bins of one chunk (xtn_tiles.hpp)
 
-// groups of four records that a thread of the bin kernel holds
-constexpr int bin_groups(int d) { return d <= 2 ? 18 : 9; }
-
 struct TilePlan {
 	uint32_t tile = 0;  // records between the starts of two tiles
 	int64_t ntiles = 0;
 	int bin_bits = 0;
 	int idx_bits = 0;
+	int bin_nt = BIN_NT, bin_groups = 18;  // the bin kernel's instantiation
 };
 
 // the tiling of V records of n sequences
@@ -903,19 +903,42 @@ TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
 	// four of them), and enough of them that bin and record leave 11 keys per
 	// record: two records meet by chance once in 20 or so.
 	const double key_bits = std::log2((double)V) + 3.5;
-	for (p.bin_bits = 6; (1 << p.bin_bits) < TL_BINS_MAX; ++p.bin_bits) {
-		const double lambda = (double)tile / (1 << p.bin_bits);
-		double q = 0, w = std::exp(-lambda);
-		if (lambda > 200)
-			q = lambda / 4 + 0.375;
-		else
-			for (int k = 1; k < 400; ++k) {
-				w *= lambda / k;
-				q += w * ((k + 3) / 4);
-			}
-		if (q * (double)p.ntiles <= 0.965 * BIN_NT * bin_groups(d) && p.bin_bits + 32 - tl_len_bits(d) - p.idx_bits >= key_bits)
+	auto bins_for = [&](int nt, int groups) {
+		for (int bits = 6; (1 << bits) <= TL_BINS_MAX; ++bits) {
+			const double lambda = (double)tile / (1 << bits);
+			double q = 0, w = std::exp(-lambda);
+			if (lambda > 200)
+				q = lambda / 4 + 0.375;
+			else
+				for (int k = 1; k < 400; ++k) {
+					w *= lambda / k;
+					q += w * ((k + 3) / 4);
+				}
+			if (q * (double)p.ntiles <= 0.965 * nt * groups && bits + 32 - tl_len_bits(d) - p.idx_bits >= key_bits)
+				return bits;
+		}
+		return 0;
+	};
+	// The narrow form first; where its bins would leave runs of fewer than six
+	// records, the wide one over half as many (at 1.15M CDR3s, d = 2: columns
+	// 29 us and bins 656 us against 51 and 660; at 50 000, d = 4, 24 and 599
+	// against 44 and 629); at distances 3 and 4 then the wide one of 18 groups,
+	// whose list still takes a fifth of the records.
+	const struct {
+		int nt, groups;
+	} forms[] = {{BIN_NT, d <= 2 ? 18 : 9}, {BIN_WIDE_NT, d <= 2 ? 18 : 9}, {BIN_WIDE_NT, 18}};
+	for (const auto& f : forms) {
+		const int bits = bins_for(f.nt, f.groups);
+		if (!bits || (p.bin_bits && bits >= p.bin_bits))
+			continue;
+		p.bin_bits = bits;
+		p.bin_nt = f.nt;
+		p.bin_groups = f.groups;
+		if ((double)tile / (1 << bits) >= 6.0)
 			break;
 	}
+	if (!p.bin_bits)
+		p.ntiles = 0;  // more records than the bins take
 	return p;
 }
 
@@ -1078,7 +1101,6 @@ int regroup_exact(xtn_handle* h, Grouping& g) {
 }
 
 int issue_buckets(xtn_handle* h, Grouping& g, uint32_t lo, uint32_t hi, int64_t pcap) {
-	const bool ranged = lo > 0 || (int64_t)hi < g.nseq;
 	if (g.tiles) {
 		BinArgs& bn = g.bn;
 		bn.pairs = h->pairs.as<uint64_t>();
@@ -1087,15 +1109,17 @@ int issue_buckets(xtn_handle* h, Grouping& g, uint32_t lo, uint32_t hi, int64_t 
 		bn.id_hi = hi;
 		StageScope sg(h, "pairs");
 		ProfScope ps(h, "bins", (double)g.nrec * 4.0);
-		const unsigned grid = (unsigned)std::min<int64_t>(bn.nb, (int64_t)h->n_cu * BIN_PER_CU);
+		const unsigned grid = (unsigned)std::min<int64_t>(bn.nb, (int64_t)h->n_cu * BIN_WIDE_NT / bn.nt);
 		typedef void (*BinFn)(BinArgs);
 		static const BinFn fns[2][2][2] = {
-		    {{k_bins<18, false, false>, k_bins<18, true, false>}, {k_bins<18, false, true>, k_bins<18, true, true>}},
-		    {{k_bins<9, false, false>, k_bins<9, true, false>}, {k_bins<9, false, true>, k_bins<9, true, true>}}};
-		fns[bin_groups(bn.distance) == 9][h->bin_parts][ranged]<<<grid, BIN_NT, 0, h->stream>>>(bn);
+		    {{k_bins<BIN_NT, 18, false>, k_bins<BIN_NT, 18, true>}, {k_bins<BIN_NT, 9, false>, k_bins<BIN_NT, 9, true>}},
+		    {{k_bins<BIN_WIDE_NT, 18, false>, k_bins<BIN_WIDE_NT, 18, true>},
+		     {k_bins<BIN_WIDE_NT, 9, false>, k_bins<BIN_WIDE_NT, 9, true>}}};
+		fns[bn.nt == BIN_WIDE_NT][bn.groups == 9][h->bin_parts]<<<grid, bn.nt, 0, h->stream>>>(bn);
 		HIP_LAUNCH_CHECK(h);
 		return XTN_OK;
 	}
+	const bool ranged = lo > 0 || (int64_t)hi < g.nseq;
 	BucketArgs& ba = g.ba;
 	ba.pairs = h->pairs.as<uint64_t>();
 	ba.pcap = pcap;
@@ -1248,6 +1272,17 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	}
 	st.n_variants = (int64_t)V;
 
+	// Enough records at distances 1 to 4: tiles ordered by bin (xtn_tiles.hpp),
+	// until a bound there is outgrown. One chunk then holds about 4e8 records,
+	// 2.8 times what the buckets take; a smaller bucket target keeps cutting
+	// chunks as before.
+	const int64_t bucket_records = (int64_t)65536 * h->tune_target;
+	auto tiles_wanted = [&]() {
+		return d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && (int64_t)V < (int64_t)INT32_MAX && !h->no_alloc &&
+		       h->cfg.max_records_per_chunk <= 0 && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
+		       !h->coarse_off && !h->tail_safe &&
+		       ((int64_t)V <= bucket_records || h->tune_target >= DEFAULT_BUCKET_TARGET);
+	};
 	// chunk plan: the records of one chunk (plus the sort buffer and the
 	// bucket regions, ~40 B per record in all) must fit the HBM budget, and
 	// its buckets must stay near the target record count
@@ -1263,6 +1298,12 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		budget = std::min<int64_t>(budget, (int64_t)65536 * h->tune_target);
 	}
 	budget = std::max<int64_t>(budget, 1 << 16);
+	// (a tiled record takes ~8 B with its share of the bin starts)
+	const TilePlan tplan =
+	    tiles_wanted() && (double)V * 8.0 <= (double)free_b * 0.6 ? plan_tiles((int64_t)V, nseq, d, h->n_cu) : TilePlan{};
+	auto use_tiles = [&]() { return tplan.ntiles > 0 && tiles_wanted(); };
+	if (use_tiles())
+		budget = (int64_t)V;
 	int pbits = 0;
 	while (((int64_t)V >> pbits) > budget && pbits < 12)
 		++pbits;
@@ -1293,14 +1334,6 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	ga.part_bits = pbits;
 	ga.V = (int64_t)V;
 	ga.set_of = set_of;
-	// one chunk of enough records at distances 1 to 4: tiles ordered by bin
-	// (xtn_tiles.hpp), until a bound there is outgrown
-	auto use_tiles = [&]() {
-		return nparts == 1 && d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && !h->no_alloc &&
-		       h->cfg.max_records_per_chunk <= 0 && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
-		       !h->coarse_off && !h->tail_safe;
-	};
-	const TilePlan tplan = use_tiles() ? plan_tiles((int64_t)V, nseq, d, h->n_cu) : TilePlan{};
 	// packing (unless done above to learn V) and the generator's tile table
 	bool prologue_done = false;
 	auto prologue = [&]() -> int {
@@ -1517,6 +1550,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			bn.ntiles = tplan.ntiles;
 			bn.cpitch = cpitch;
 			bn.nb = nbins;
+			bn.nt = tplan.bin_nt;
+			bn.groups = tplan.bin_groups;
 			bn.lb = tplan.idx_bits;
 			bn.len_bits = tl_len_bits(d);
 			bn.key_low = std::max(bn.lb + bn.len_bits, tplan.bin_bits);
@@ -1798,6 +1833,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				// the run kernels take by their long runs): the run again with
 				// the separate pass, which these sequences keep from now on
 				h->coarse_off = true;
+				if ((int64_t)V > bucket_records)  // the chunks of the separate pass
+					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
 				grouped = false;
 				prologue_done = false;
 				continue;
@@ -1831,6 +1868,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				// host-checked tail from now on, and the round is redone
 				// (packing included, whose offsets share the flag)
 				h->tail_safe = true;
+				if ((int64_t)V > bucket_records && nparts == 1)
+					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
 				grouped = false;
 				prologue_done = false;
 				continue;

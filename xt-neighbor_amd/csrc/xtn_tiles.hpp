@@ -466,8 +466,9 @@ __global__ __launch_bounds__(256) void k_tile_cols(const uint16_t* __restrict__ 
 
 // threads of a bin's workgroup, two workgroups per CU (one's loads and
 // barriers under the other's work: 430 us against 476 at 1M CDR3s, d = 2, for
-// one of 1024 threads over half as many bins)
-constexpr int BIN_NT = 512, BIN_PER_CU = 2;
+// one of 1024 threads over half as many bins); the wide form takes the records
+// that the narrow one would need too many bins for
+constexpr int BIN_NT = 512, BIN_WIDE_NT = 1024;
 
 struct BinArgs {
 	const uint32_t* rec;     // the tiles
@@ -476,6 +477,7 @@ struct BinArgs {
 	const uint64_t* pk;
 	int64_t ntiles, cpitch;
 	int32_t nb;
+	int32_t nt, groups;      // the instantiation: BIN_NT or BIN_WIDE_NT threads, 18 or 9 groups each
 	int32_t lb;              // index bits of a record
 	int32_t len_bits;        // length bits above them
 	int32_t key_low;         // lowest key bit of a record (above it the key's bits below the bin; zeros may lie
@@ -548,7 +550,7 @@ __device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint3
 
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// Bins over resident workgroups. BIN_NT threads hold QPT groups of four records
+// Bins over resident workgroups. NT threads hold QPT groups of four records
 // each.
 //   1. the runs of the bin (k_tile_cols' row and the next one) are listed as
 //      groups of up to four records, and every group is loaded into
@@ -567,15 +569,15 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // QPT 18: bins of up to 36864 slots, an eighth of whose records may be
 // listed; QPT 9 (distances 3 and 4, where a neighbouring pair shares hundreds
 // of variants): half as many slots and a list for half of their records.
-template <int QPT, bool RANGED, bool PARTS>
-__global__ __launch_bounds__(BIN_NT, 4) void k_bins(BinArgs a) {
-	constexpr int NT = BIN_NT;
-	constexpr int B1 = 18, B2 = 16, HBITS = QPT == 18 ? 12 : 11;
-	static_assert(QPT == 18 || QPT == 9, "bitmaps of 7 bits or more and a quarter of that per record");
+template <int NT, int QPT, bool PARTS>
+__global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
+	constexpr int X = NT / BIN_NT;  // the wide form: everything twice, one workgroup per CU
+	constexpr int B1 = 17 + X, B2 = 15 + X, HBITS = (QPT == 18 ? 11 : 10) + X;
+	static_assert((X == 1 || X == 2) && (QPT == 18 || QPT == 9), "bitmaps of 7 bits or more and a quarter of that per record");
 	constexpr int QCAP = NT * QPT;
-	constexpr int SVC = QPT == 18 ? (1 << B1) / 8 / 6 / 64 * 64 : 7168;  // records listed in step 3
+	constexpr int SVC = QPT == 18 ? (1 << B1) / 8 / 6 / 64 * 64 : 7168 * X;  // records listed in step 3
 	constexpr int HEADS = 1 << HBITS;
-	constexpr int PLC = QPT == 18 ? (QCAP * 4 - HEADS * 4 - SVC * 2) / 4 : 1024;
+	constexpr int PLC = QPT == 18 ? (QCAP * 4 - HEADS * 4 - SVC * 2) / 4 : 1024 * X;
 	static_assert(PLC >= NT, "room for pairs beside the lists");
 	__shared__ union {
 		uint32_t bm1[(1 << B1) / 32];
@@ -596,7 +598,7 @@ __global__ __launch_bounds__(BIN_NT, 4) void k_bins(BinArgs a) {
 	__shared__ uint32_t s_tmp[NT / WAVE + 1];
 	__shared__ unsigned long long s_base;
 	__shared__ uint32_t s_nsv, s_npl;
-	static_assert(sizeof(u1) + sizeof(u2) + sizeof(s_bm2) <= 79 * 1024, "two workgroups per CU");
+	static_assert(sizeof(u1) + sizeof(u2) + sizeof(s_bm2) <= 79 * 1024 * X, "two workgroups per CU");
 	const int t = threadIdx.x;
 	const int lane = lane_id();
 	const int G = (int)gridDim.x;
@@ -776,7 +778,7 @@ __global__ __launch_bounds__(BIN_NT, 4) void k_bins(BinArgs a) {
 			if (x == y)
 				return false;
 			const uint32_t lo = x < y ? x : y, hi = x < y ? y : x;
-			if (RANGED && (lo < a.id_lo || lo >= a.id_hi))
+			if (lo < a.id_lo || lo >= a.id_hi)
 				return false;
 			*p = ((uint64_t)lo << a.idb) | hi;
 			return tile_pair(a.pk, lo, hi, (ri >> a.lb) & ((1u << a.len_bits) - 1u), a.len_bits,
