@@ -101,3 +101,47 @@ def test_tiled_sets_and_rounds(d):
                 a, b = int(cuts[k]), int(cuts[k + 1])
                 inside = want[(want[:, 0] >= a) & (want[:, 1] < b)] - np.array([a, a, 0])
                 assert np.array_equal(got.get(k, np.zeros((0, 3), np.int64)), inside), k
+
+
+def test_replays_keep_their_distance():
+    # a captured run of one distance, runs of others, and the captured one again
+    # (few candidates at every distance, so that the pair buffer's size stays)
+    long = random_seqs(np.random.default_rng(130), 3_500, 13, 17)
+    chars, offsets = xtn.encode(long + [s[:k % 9] + "AC"[k % 2] + s[k % 9 + k % 3:] for k, s in enumerate(long)])
+    want = {d: oracle.nn_port_mt(chars, offsets, d, 0, THREADS)[0].astype(np.int64) for d in (2, 3, 4)}
+    back = 0  # replays right after another distance's run
+    with xtn.Engine(distance=2) as eng:
+        eng.set_sequences(chars=chars, offsets=offsets)
+        for d in (4, 3, 2):  # every buffer is there from here on: graphs stay valid
+            assert np.array_equal(search(eng, d, 0)[0], want[d])
+        for first, other in [(2, 3), (3, 2), (3, 4), (4, 2)]:
+            for k, d in enumerate((first, first, first, other, first, first)):
+                got, st = search(eng, d, 0)
+                assert np.array_equal(got, want[d]), (first, other, d, st)
+                back += st["graph_replays"] if k == 4 else 0
+    assert back >= 1
+
+
+@pytest.mark.parametrize("d,n", [(1, 120_000), (2, 24_000), (3, 8_000)])
+def test_replays_with_other_rows_of_the_same_shape(d, n):
+    # the same counts and buffers, so the same graph: rows all apart, then rows
+    # of which each has one copy (the bins' lists run over) or many (more equal
+    # pairs than records)
+    def rows(copies):
+        base = random_seqs(np.random.default_rng(140 + copies), n // copies, 15, 15)
+        seqs = [s for s in base for _ in range(copies)]
+        return xtn.encode([seqs[i] for i in np.random.default_rng(copies).permutation(n)])
+
+    inputs = {c: rows(c) for c in (1, 2, 8)}
+    want = {c: oracle.nn_port_mt(*inputs[c], d, 0, THREADS)[0].astype(np.int64) for c in inputs}
+    with xtn.Engine(distance=d) as eng:
+        eng.set_sequences(chars=inputs[1][0], offsets=inputs[1][1])
+        for _ in range(3):
+            got, st = search(eng, d, 0)
+            assert np.array_equal(got, want[1])
+        assert st["graph_replays"] == 1
+        for c in (2, 1, 8, 2, 1):
+            eng.set_sequences(chars=inputs[c][0], offsets=inputs[c][1])
+            for _ in range(2):
+                got, st = search(eng, d, 0)
+                assert np.array_equal(got, want[c]), (c, st)

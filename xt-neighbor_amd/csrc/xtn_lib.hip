@@ -85,8 +85,9 @@ struct xtn_handle {
 	DBuf recs_all, recs_part;  // chunked runs: every record once, then ordered by part
 	DBuf seg_cur, seg_ctl;  // the generator's coarse pass: sub-range cursors, digit tiling
 	DBuf tile_rec, tile_offs, tile_cols;  // tiles ordered by bin, their bin starts by tile and by bin
-	DBuf del_sets_d;  // the deletion sets of distance del_sets_of (xtn_tiles.hpp)
-	int del_sets_of = 0;
+	DBuf del_sets_d;  // the deletion sets of distances 2, 3 and 4, one after another (xtn_tiles.hpp): written
+	                  // once, since a captured run reads its distance's
+	bool del_sets_set = false;
 	DBuf pk, voff, recs, recs_alt, hist, scan_tmp, runs_small, runs_big, big_pre, pairs, pairs_alt,
 	    flags, pos, dist, out_pairs, out_dist, ctrs, part_hist, scalar;
 	// overlap-mode workspaces
@@ -1298,6 +1299,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		budget = std::min<int64_t>(budget, (int64_t)65536 * h->tune_target);
 	}
 	budget = std::max<int64_t>(budget, 1 << 16);
+	const int64_t sorted_budget = budget;  // a chunk of the other layouts
 	// (a tiled record takes ~8 B with its share of the bin starts)
 	const TilePlan tplan =
 	    tiles_wanted() && (double)V * 8.0 <= (double)free_b * 0.6 ? plan_tiles((int64_t)V, nseq, d, h->n_cu) : TilePlan{};
@@ -1522,16 +1524,25 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			TRY(ensure(h, h->tile_rec, sizeof(uint32_t) * (size_t)(tplan.ntiles * TL_CAP + 4)));
 			TRY(ensure(h, h->tile_offs, sizeof(uint16_t) * (size_t)(tplan.ntiles * pitch)));
 			TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
-			if (d >= 2 && h->del_sets_of != d) {
-				static const std::vector<uint32_t> sets[TL_MAX_D - 1] = {del_sets(2), del_sets(3), del_sets(4)};
-				const std::vector<uint32_t>& v = sets[d - 2];
-				TRY(ensure(h, h->del_sets_d, sizeof(uint32_t) * (size_t)tl_sets(TL_MAX_D)));
-				HIP_TRY(h, hipMemcpyAsync(h->del_sets_d.p, v.data(), sizeof(uint32_t) * v.size(),
+			if (d >= 2 && !h->del_sets_set) {
+				static const std::vector<uint32_t> sets = [] {
+					std::vector<uint32_t> all;
+					for (int k = 2; k <= TL_MAX_D; ++k) {
+						const std::vector<uint32_t> one = del_sets(k);
+						all.insert(all.end(), one.begin(), one.end());
+					}
+					return all;
+				}();
+				TRY(ensure(h, h->del_sets_d, sizeof(uint32_t) * sets.size()));
+				HIP_TRY(h, hipMemcpyAsync(h->del_sets_d.p, sets.data(), sizeof(uint32_t) * sets.size(),
 				                          hipMemcpyHostToDevice, s));
-				h->del_sets_of = d;
+				h->del_sets_set = true;
 			}
 			TileArgs& ta = g.ta;
 			ta.del = h->del_sets_d.as<uint32_t>();
+			for (int k = 2; k < d; ++k)
+				ta.del += tl_sets(k);
+			ta.n = nseq;
 			ta.pk = h->pk.as<uint64_t>();
 			ta.voff = h->voff.as<uint64_t>();
 			ta.first = h->tseq.as<uint32_t>();
@@ -1776,8 +1787,9 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				sig.select_nt = h->tune_select_nt;
 				sig.low = h->tail_full ? 0 : h->tune_low;
 				sig.coarse = h->coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
-				sig.pad = h->bin_parts ? 1 : 0;
+				sig.pad = (h->bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0);
 			}
+			const bool tiled = use_tiles();  // also of a replay, which plans nothing
 			bool via_graph = false;
 			if (graph_ok && h->graph_exec && sig == h->graph_sig) {
 				HIP_TRY(h, hipGraphLaunch(h->graph_exec, s));
@@ -1826,20 +1838,20 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			}
 			TRY(read_head(h, &head));
 			n_written = std::max<int64_t>(n_written, (int64_t)head.rc.n_records);
-			if (head.rc.coarse_ovf || (g1.tiles && head.rc.pairs_small > V)) {
+			if (head.rc.coarse_ovf || (tiled && head.rc.pairs_small > V)) {
 				// a sub-range of the generator's coarse pass overflowed and lost
 				// records, or the tiles and bins outgrew a bound or met more
 				// equal pairs than records (many copies of some strings, which
 				// the run kernels take by their long runs): the run again with
 				// the separate pass, which these sequences keep from now on
 				h->coarse_off = true;
-				if ((int64_t)V > bucket_records)  // the chunks of the separate pass
+				if ((int64_t)V > sorted_budget)  // the chunks of the separate pass
 					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
 				grouped = false;
 				prologue_done = false;
 				continue;
 			}
-			if (g1.tiles && head.rc.n_big) {
+			if (tiled && head.rc.n_big) {
 				// bins listed more records than fit: the run again with the bins
 				// in parts, which these sequences keep from now on
 				h->bin_parts = true;
@@ -1868,7 +1880,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				// host-checked tail from now on, and the round is redone
 				// (packing included, whose offsets share the flag)
 				h->tail_safe = true;
-				if ((int64_t)V > bucket_records && nparts == 1)
+				if ((int64_t)V > sorted_budget && nparts == 1)
 					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
 				grouped = false;
 				prologue_done = false;

@@ -100,7 +100,7 @@ struct TileArgs {
 	const uint64_t* pk;
 	const uint64_t* voff;
 	const uint32_t* first;   // first sequence of each tile, [ntiles] = n
-	const uint32_t* del;     // the deletion sets (del_sets)
+	const uint32_t* del;     // the deletion sets of the distance (del_sets)
 	uint32_t* out;           // TL_CAP slots per tile
 	uint16_t* offs;          // a row of `pitch` per tile: the start of each bin, then the tile's total
 	unsigned long long* ovf;
@@ -108,6 +108,7 @@ struct TileArgs {
 	int32_t bin_bits;        // 6..13
 	int32_t lb;              // index bits of a record
 	int32_t sets;            // the prefixes carry query sets
+	uint32_t n;              // sequences
 };
 
 // A record: key bits below the bin, the low bits of the variant's length, the
@@ -223,8 +224,8 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 	const uint32_t s0 = a.first[tile], s1 = a.first[tile + 1];
 	const int cnt = (int)(s1 - s0);
 	const int most = SEQS < (1 << a.lb) - 1 ? SEQS : (1 << a.lb) - 1;
-	if (cnt <= 0 || cnt > most) {  // uniform
-		tile_refuse(a, row, nb, cnt > most);
+	if (cnt <= 0 || cnt > most || s1 > a.n) {  // uniform (past n: a packing that gave up left the table undone)
+		tile_refuse(a, row, nb, cnt > 0);
 		return;
 	}
 	const uint64_t v0 = a.voff[s0];
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles1(TileArgs a) {
 	uint16_t* const row = a.offs + tile * a.pitch;
 	const uint32_t s0 = a.first[tile], s1 = a.first[tile + 1];
 	const int cnt = (int)(s1 - s0);
-	if (cnt <= 0 || cnt > (1 << a.lb) - 1) {  // uniform
+	if (cnt <= 0 || cnt > (1 << a.lb) - 1 || s1 > a.n) {  // uniform
 		tile_refuse(a, row, nb, cnt > 0);
 		return;
 	}
