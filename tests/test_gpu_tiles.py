@@ -105,9 +105,9 @@ def test_tiled_sets_and_rounds(d):
 
 def test_replays_keep_their_distance():
     # a captured run of one distance, runs of others, and the captured one again
-    # (few candidates at every distance, so that the pair buffer's size stays)
-    long = random_seqs(np.random.default_rng(130), 3_500, 13, 17)
-    chars, offsets = xtn.encode(long + [s[:k % 9] + "AC"[k % 2] + s[k % 9 + k % 3:] for k, s in enumerate(long)])
+    # (few candidates at every distance, so that the plan for them stays)
+    long = random_seqs(np.random.default_rng(130), 7_000, 13, 17)
+    chars, offsets = xtn.encode(long + [s[:k] + "AC"[k % 2] + s[k + k % 3:] for k, s in enumerate(long[:8])])
     want = {d: oracle.nn_port_mt(chars, offsets, d, 0, THREADS)[0].astype(np.int64) for d in (2, 3, 4)}
     back = 0  # replays right after another distance's run
     with xtn.Engine(distance=2) as eng:

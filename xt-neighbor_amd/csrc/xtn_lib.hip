@@ -582,6 +582,12 @@ double now_ms() {
 
 constexpr int KEY_BITS = 32;             // hash bits that order records into runs
 constexpr int64_t TILES_MIN_RECORDS = 600000;  // fewer records of a chunk take the sorted layout
+// The one-workgroup tail (k_tail_small) is taken for at most this many
+// candidates in the run before or, with none to go by, for at most this many
+// records. Each thousand candidates take its one CU 7 us; at 5499 it is 20 us
+// ahead of the passes, and towards its capacity of 8192 they meet.
+constexpr int64_t SMALL_TAIL_EXPECTED = 6000;
+constexpr uint64_t SMALL_TAIL_RECORDS = 200000;
 
 // device control block: the counters of the candidate search, then the
 // tail's block
@@ -699,6 +705,7 @@ struct TailPlan {
 	int passes = 0;    // 8-bit LSD digits over the pair bits from low_bits up to 2 * idb
 	int low_bits = 0;  // > 0: the select ranks the bits below in LDS (k_select_grouped)
 	int64_t sort_tiles = 0, sel_tiles = 0;
+	bool small = false;  // k_tail_small instead of all of these
 };
 
 // LSD passes of the next candidate sort over 2 * idb pair bits: the sort
@@ -714,6 +721,7 @@ int tail_passes(const xtn_handle* h, int idb) {
 // look-back state
 int tail_prepare(xtn_handle* h, int64_t pcap, int idb, int64_t out_keep, TailPlan* tp) {
 	tp->pcap = pcap;
+	tp->small = false;
 	tp->passes = tail_passes(h, idb);
 	tp->low_bits = std::max(0, 2 * idb - 8 * tp->passes);
 	const int64_t sort_tile = h->tune_sort_tile, sel_tile = (int64_t)h->tune_select_nt * SL_IT;
@@ -738,6 +746,31 @@ int issue_tail(xtn_handle* h, const TailPlan& tp, int idb, const uint32_t* seq_m
 	hipStream_t s = h->stream;
 	CtlBlock* cb = ctl_block(h);
 	const unsigned long long* n_dev = &cb->rc.n_cand;
+	SelectArgs sa{};
+	sa.n_dev = n_dev;
+	sa.cap = tp.pcap;
+	sa.idb = idb;
+	sa.distance = h->cfg.distance;
+	sa.measure = h->cfg.measure;
+	sa.row_base = row_base;
+	sa.low_bits = tp.low_bits;
+	sa.chars = h->chars.as<uint8_t>();
+	sa.offs = h->offs.as<uint32_t>();
+	sa.seq_map = seq_map;
+	sa.set_of = set_of;
+	sa.chars_b = chars_b;
+	sa.offs_b = offs_b;
+	sa.out_pairs = h->out_pairs.as<int2>() + out_off;
+	sa.out_dist = h->out_dist.as<int8_t>() + out_off;
+	sa.ctl = &cb->tc;
+	sa.spin_limit = h->spin_limit;
+	if (tp.small) {
+		sa.keys = h->pairs.as<uint64_t>();
+		ProfScope ps(h, "tail_small", 8.0 * (double)h->last_pairs);
+		small_tail_kernel(h->cfg.distance, h->cfg.measure)<<<1, TS_NT, 0, s>>>(sa, (2 * idb + 7) / 8);
+		HIP_LAUNCH_CHECK(h);
+		return XTN_OK;
+	}
 	uint32_t* state = h->tail_state.as<uint32_t>();
 	const int64_t nsort = (int64_t)tp.passes * tp.sort_tiles * RS_BINS;
 	// profile byte counts: the candidates of the previous run (the count of
@@ -768,26 +801,8 @@ int issue_tail(xtn_handle* h, const TailPlan& tp, int idb, const uint32_t* seq_m
 		HIP_LAUNCH_CHECK(h);
 		std::swap(a, b);
 	}
-	SelectArgs sa{};
 	sa.keys = a;
-	sa.n_dev = n_dev;
-	sa.cap = tp.pcap;
-	sa.idb = idb;
-	sa.distance = h->cfg.distance;
-	sa.measure = h->cfg.measure;
-	sa.row_base = row_base;
-	sa.low_bits = tp.low_bits;
-	sa.chars = h->chars.as<uint8_t>();
-	sa.offs = h->offs.as<uint32_t>();
-	sa.seq_map = seq_map;
-	sa.set_of = set_of;
-	sa.chars_b = chars_b;
-	sa.offs_b = offs_b;
-	sa.out_pairs = h->out_pairs.as<int2>() + out_off;
-	sa.out_dist = h->out_dist.as<int8_t>() + out_off;
-	sa.ctl = &cb->tc;
 	sa.state = reinterpret_cast<uint64_t*>(state + nsort);
-	sa.spin_limit = h->spin_limit;
 	{
 		// candidates read once, the unique ones' two strings and offsets, the
 		// kept triples written
@@ -1747,6 +1762,9 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			}
 			TRY(checked_candidates(h, g1, lo, hi_id, pmax, &pcap, &n_pairs, &split));
 		} else if (nparts == 1) {
+			const bool small = h->tune_low == 0 && (h->last_pairs > 0 && !h->no_alloc
+			                                            ? h->last_pairs <= SMALL_TAIL_EXPECTED
+			                                            : V <= SMALL_TAIL_RECORDS);
 			// everything issued, one readback: the whole run of a single
 			// round is a graph once it has run the same way before
 			auto issue_all = [&]() -> int {
@@ -1760,6 +1778,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 					grouped = true;
 				}
 				TRY(tail_prepare(h, pcap, idb, out_total, &tp));
+				tp.small = small;
 				TRY(issue_buckets(h, g1, lo, hi_id, pcap));
 				StageScope sg(h, "verify");
 				TRY(issue_tail(h, tp, idb, seq_map, row_base, set_of, out_total));
@@ -1787,7 +1806,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				sig.select_nt = h->tune_select_nt;
 				sig.low = h->tail_full ? 0 : h->tune_low;
 				sig.coarse = h->coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
-				sig.pad = (h->bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0);
+				sig.pad = (h->bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0);
 			}
 			const bool tiled = use_tiles();  // also of a replay, which plans nothing
 			bool via_graph = false;
@@ -1859,6 +1878,14 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				grouped = false;
 				prologue_done = false;
 				continue;
+			}
+			if (small && !head.error && (int64_t)head.rc.n_cand > TS_CAP && (int64_t)head.rc.n_cand <= pcap &&
+			    head.rc.append == 0) {
+				// too many for the one workgroup: the tail over the candidates as
+				// they lie (a later run goes by their count)
+				TRY(tail_prepare(h, pcap, idb, out_total, &tp));
+				TRY(issue_tail(h, tp, idb, seq_map, row_base, set_of, out_total));
+				TRY(read_head(h, &head));
 			}
 			const bool clean =
 			    !head.error && !head.overflow && (int64_t)head.rc.n_cand <= pcap && head.rc.append == 0;
@@ -3247,10 +3274,12 @@ int serve_query(xtn_server* sv, xtn_handle* w, const ServeRequest& rq, ServeResu
 	CtlHead head{};
 	TailPlan tp;
 	bool grown = false;
+	bool small = (double)V * (w->serve_ratio > 0 ? ratio : 0.02) <= (double)SMALL_TAIL_EXPECTED;
 	w->tail_full = false;
 	for (;;) {
 		TRY(ensure(w, w->pairs, sizeof(uint64_t) * (size_t)pcap));
 		TRY(tail_prepare(w, pcap, idb, 0, &tp));
+		tp.small = small;
 		TRY(zero_ctl(w, true, true));
 		k_match<<<grid_for(V, MATCH_NT), MATCH_NT, 0, s>>>(w->recs.as<uint64_t>(), V, sv->index, sv->dir,
 		                                                   sv->dir_bits, idb, w->pairs.as<uint64_t>(), pcap,
@@ -3268,6 +3297,10 @@ int serve_query(xtn_server* sv, xtn_handle* w, const ServeRequest& rq, ServeResu
 			pcap = (int64_t)head.rc.n_cand + (int64_t)head.rc.n_cand / 4;
 			pcap = std::min<int64_t>(pcap, (int64_t)LB_VAL);
 			grown = true;
+			continue;
+		}
+		if (small && (int64_t)head.rc.n_cand > TS_CAP) {
+			small = false;
 			continue;
 		}
 		if (!head.overflow)

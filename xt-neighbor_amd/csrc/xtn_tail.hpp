@@ -730,6 +730,112 @@ __global__ __launch_bounds__(NT) void k_select_grouped(SelectArgs a) {
 	select_emit<NT, R>(a, tile, ntiles, s_k, s_d, nu, s_cc, &s_excl);
 }
 
+// The whole tail of up to TS_CAP candidates in one workgroup: sorted in LDS by
+// the passes of k_onesweep (keys in registers between them), the first of
+// each value verified a pair per lane, the kept ones written in order. Bound
+// by latency: a few thousand candidates are no work for the chip, and the
+// passes' launches, gaps and look-backs cost more than the one CU's time (a
+// resident run at d = 1: 3000 CDR3s, 1026 candidates: 21 us against six
+// launches of 61, the run 93 us against 117; 17 000, 5499: 51 against 81, the
+// run 129 against 149). The candidates are spread over all waves, so that a
+// pass is as few dependent rounds as they allow. More candidates than TS_CAP
+// write nothing (the host sees their count).
+constexpr int TS_NT = 1024;
+constexpr int TS_IT = 8;
+constexpr int TS_CAP = TS_NT * TS_IT;
+
+template <int D>
+__global__ __launch_bounds__(TS_NT) void k_tail_small(SelectArgs a, int passes) {
+	__shared__ uint64_t s_k[TS_CAP];
+	__shared__ uint32_t s_cnt[TS_NT / WAVE][RS_BINS];
+	__shared__ uint32_t s_dpre[RS_BINS];
+	__shared__ uint32_t s_scan[TS_NT / WAVE + 1];
+	__shared__ int8_t s_d[TS_CAP];
+	__shared__ uint32_t s_cc[TS_IT * TS_NT / WAVE + 1];
+	const int t = threadIdx.x;
+	const int lane = lane_id();
+	const int w = t / WAVE;
+	const int64_t n64 = tail_count(a.n_dev, a.cap);
+	if (n64 > TS_CAP || n64 < (int64_t)*a.n_dev)  // uniform
+		return;
+	const int n = (int)n64;
+	const int seg = (n + TS_NT - 1) / TS_NT * WAVE;  // positions of a wave, <= TS_IT * WAVE
+	const int wrem = n - w * seg;
+	const int w_valid = wrem <= 0 ? 0 : (wrem < seg ? wrem : seg);
+	uint64_t k[TS_IT];
+#pragma unroll
+	for (int r = 0; r < TS_IT; ++r)
+		k[r] = r * WAVE + lane < w_valid ? a.keys[w * seg + r * WAVE + lane] : 0ull;
+	for (int p = 0; p < passes; ++p) {
+		uint32_t lp[TS_IT];
+		rank_tile_g<TS_NT, TS_IT>(k, w_valid, 8 * p, lp, s_cnt, s_dpre, s_scan);
+#pragma unroll
+		for (int r = 0; r < TS_IT; ++r)
+			if (lp[r] != 0xFFFFFFFFu)
+				s_k[lp[r]] = k[r];
+		__syncthreads();
+#pragma unroll
+		for (int r = 0; r < TS_IT; ++r)
+			k[r] = r * WAVE + lane < w_valid ? s_k[w * seg + r * WAVE + lane] : 0ull;
+	}
+	__syncthreads();
+	// the first of each value, in rows of TS_NT positions
+	uint32_t uflags = 0;
+#pragma unroll
+	for (int r = 0; r < TS_IT; ++r) {
+		const int q = r * TS_NT + t;
+		k[r] = q < n ? s_k[q] : 0ull;
+		if (q < n && (q == 0 || s_k[q - 1] != k[r]))
+			uflags |= 1u << r;
+	}
+	uint32_t pos[TS_IT];
+	const uint32_t nu = striped_rank<TS_NT, TS_IT>(uflags, pos, s_cc);  // (its barriers end the reads above)
+#pragma unroll
+	for (int r = 0; r < TS_IT; ++r)
+		if (uflags & (1u << r))
+			s_k[pos[r]] = k[r];
+	__syncthreads();
+	select_verify<D, TS_NT>(a, s_k, s_d, nu);
+	uint32_t kflags = 0;
+#pragma unroll
+	for (int r = 0; r < TS_IT; ++r) {
+		const uint32_t q = (uint32_t)(r * TS_NT + t);
+		if (q < nu && s_d[q] >= 0)
+			kflags |= 1u << r;
+	}
+	const uint32_t nk = striped_rank<TS_NT, TS_IT>(kflags, pos, s_cc);
+	if (t == 0) {
+		a.ctl->n_unique = nu;
+		a.ctl->n_out = nk;
+	}
+	const uint64_t idmask = (1ull << a.idb) - 1ull;
+#pragma unroll
+	for (int r = 0; r < TS_IT; ++r)
+		if (kflags & (1u << r)) {
+			const uint32_t q = (uint32_t)(r * TS_NT + t);
+			const uint64_t p = s_k[q];
+			a.out_pairs[pos[r]] = make_int2((int)(p >> a.idb), (int)(p & idmask));
+			a.out_dist[pos[r]] = s_d[q];
+		}
+}
+
+typedef void (*SmallTailFn)(SelectArgs, int);
+inline SmallTailFn small_tail_kernel(int distance, int measure) {
+	if (measure == 1)
+		return k_tail_small<1>;
+	switch (distance) {
+	case 1: return k_tail_small<1>;
+	case 2: return k_tail_small<2>;
+	case 3: return k_tail_small<3>;
+	case 4: return k_tail_small<4>;
+	case 5: return k_tail_small<5>;
+	case 6: return k_tail_small<6>;
+	case 7: return k_tail_small<7>;
+	case 8: return k_tail_small<8>;
+	default: return k_tail_small<0>;
+	}
+}
+
 // the select kernel of a run: the band of its distance (Hamming needs none),
 // NT threads per tile, over fully sorted or grouped candidates
 typedef void (*SelectFn)(SelectArgs);
