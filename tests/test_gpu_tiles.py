@@ -83,6 +83,37 @@ def test_tiled_search_matches_oracle(name, make, d, measure, tiled):
         assert np.array_equal(got, want)
 
 
+def fifteens(seed, n):
+    # 15 residues each, a third of the rows a substitution away from another
+    seqs = random_seqs(np.random.default_rng(seed), n - n // 3, 15, 15)
+    return xtn.encode(seqs + [s[:k % 15] + "W" + s[k % 15 + 1:] for k, s in enumerate(seqs[:n // 3])])
+
+
+@pytest.mark.parametrize("name,make,d,measure,tiled", [
+    # 16 variants each: 4080, 4096 and 4112 records around the fewest that are tiled
+    ("fewest", lambda: fifteens(201, 255), 1, 0, 0),
+    ("fewest", lambda: fifteens(202, 256), 1, 1, 1),
+    ("fewest", lambda: fifteens(203, 257), 1, 0, 1),
+    ("fewest", lambda: xtn.synth_nn(204, 41, planted=0.3, max_edits=2), 2, 0, None),
+    ("fewest", lambda: xtn.synth_nn(205, 9, planted=0.3, max_edits=2), 3, 0, None),
+    ("fewest", lambda: xtn.synth_nn(206, 3, planted=0.3, max_edits=2), 4, 1, None),
+    # bins in number up to two per CU, then the forms of more slots
+    ("more bins", lambda: xtn.synth_nn(207, 17_001, planted=0.3, max_edits=1), 1, 0, 1),
+    ("more bins", lambda: xtn.synth_nn(208, 2_003, 15.0, 2.5, 6, 30, planted=0.3, max_edits=2), 2, 0, 1),
+    ("few slots", lambda: xtn.synth_nn(209, 19_009, planted=0.3, max_edits=2), 2, 1, 1),
+    ("few slots", lambda: xtn.synth_nn(210, 2_311, planted=0.3, max_edits=2), 3, 0, 1),
+    ("few slots", lambda: xtn.synth_nn(211, 1_000, planted=0.3, max_edits=2), 4, 0, 1),
+    ("mixed lengths", lambda: mixed_lengths(212, 400), 3, 1, None),
+    ("mixed lengths", lambda: mixed_lengths(213, 4_000), 1, 0, None),
+    ("short strings", lambda: xtn.synth_nn(214, 3_000, 6.0, 0.0, 6, 6, planted=0.2, max_edits=1), 2, 0, None),
+    ("twice", lambda: repeated(215, 700, 2), 2, 0, None),
+    ("copies", lambda: repeated(216, 40, 60), 1, 0, 0),
+    ("one row", lambda: xtn.encode(["CASSLGTDTQYF"] * 500), 1, 0, 0),
+])
+def test_tiled_small_inputs(name, make, d, measure, tiled):
+    test_tiled_search_matches_oracle(name, make, d, measure, tiled)
+
+
 @pytest.mark.parametrize("d", [1, 2, 3])
 def test_tiled_sets_and_rounds(d):
     n = {1: 60_000, 2: 30_000, 3: 8_000}[d]

@@ -581,7 +581,11 @@ double now_ms() {
 // ----------------------------------------------------------- NN pipeline --
 
 constexpr int KEY_BITS = 32;             // hash bits that order records into runs
-constexpr int64_t TILES_MIN_RECORDS = 600000;  // fewer records of a chunk take the sorted layout
+// Fewer records of a chunk take the sorted layout. Both sides, resident runs:
+// 4827 records (300 CDR3s, d = 1) 54 us in tiles against 79 sorted, 160 003
+// 84 against 114, 1 594 140 146 against 200; below about 2500 the sorted layout
+// is one bucket without a pass, 52 us against 62 for 721.
+constexpr int64_t TILES_MIN_RECORDS = 4096;
 // The one-workgroup tail (k_tail_small) is taken for at most this many
 // candidates in the run before or, with none to go by, for at most this many
 // records. Each thousand candidates take its one CU 7 us; at 5499 it is 20 us
@@ -919,8 +923,11 @@ TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
 	// four of them), and enough of them that bin and record leave 11 keys per
 	// record: two records meet by chance once in 20 or so.
 	const double key_bits = std::log2((double)V) + 3.5;
+	// a bin for every resident workgroup of the narrow form (two per CU)
+	// while they keep 512 records or more
+	const int min_bits = std::max(6, std::min(9, bits_for(V / 512) - 1));
 	auto bins_for = [&](int nt, int groups) {
-		for (int bits = 6; (1 << bits) <= TL_BINS_MAX; ++bits) {
+		for (int bits = min_bits; (1 << bits) <= TL_BINS_MAX; ++bits) {
 			const double lambda = (double)tile / (1 << bits);
 			double q = 0, w = std::exp(-lambda);
 			if (lambda > 200)
@@ -935,6 +942,12 @@ TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
 		}
 		return 0;
 	};
+	// The form of few slots where the fewest bins suffice.
+	if (bins_for(BIN_NT, 3) == min_bits) {
+		p.bin_bits = min_bits;
+		p.bin_groups = 3;
+		return p;
+	}
 	// The narrow form first; where its bins would leave runs of fewer than six
 	// records, the wide one over half as many (at 1.15M CDR3s, d = 2: columns
 	// 29 us and bins 656 us against 51 and 660; at 50 000, d = 4, 24 and 599
@@ -971,6 +984,8 @@ constexpr int COARSE_SUB_BITS = 6;
 int issue_grouping(xtn_handle* h, Grouping& g) {
 	hipStream_t s = h->stream;
 	BucketArgs& ba = g.ba;
+	if (g.tiles && g.bn.groups == 3)
+		return XTN_OK;  // the bins read the tiles' rows
 	if (g.tiles) {
 		StageScope sg(h, "sort");
 		ProfScope ps(h, "tile_cols", 4.0 * (double)g.bn.nb * (double)g.bn.ntiles);
@@ -1131,7 +1146,9 @@ int issue_buckets(xtn_handle* h, Grouping& g, uint32_t lo, uint32_t hi, int64_t 
 		    {{k_bins<BIN_NT, 18, false>, k_bins<BIN_NT, 18, true>}, {k_bins<BIN_NT, 9, false>, k_bins<BIN_NT, 9, true>}},
 		    {{k_bins<BIN_WIDE_NT, 18, false>, k_bins<BIN_WIDE_NT, 18, true>},
 		     {k_bins<BIN_WIDE_NT, 9, false>, k_bins<BIN_WIDE_NT, 9, true>}}};
-		fns[bn.nt == BIN_WIDE_NT][bn.groups == 9][h->bin_parts]<<<grid, bn.nt, 0, h->stream>>>(bn);
+		const BinFn fn = bn.groups == 3 ? k_bins<BIN_NT, 3, false>
+		                                : fns[bn.nt == BIN_WIDE_NT][bn.groups == 9][h->bin_parts];
+		fn<<<grid, bn.nt, 0, h->stream>>>(bn);
 		HIP_LAUNCH_CHECK(h);
 		return XTN_OK;
 	}
@@ -1365,8 +1382,10 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			TRY(ensure(h, h->pack_state, sizeof(uint64_t) * (size_t)nb));
 			TRY(ensure(h, h->tseq, sizeof(uint32_t) * (size_t)(ntiles + 1)));
 			StageScope sg(h, "generate");
-			k_fill_u64<<<grid_for(nb, 256), 256, 0, s>>>(h->pack_state.as<unsigned long long>(), nb, 0ull);
-			HIP_LAUNCH_CHECK(h);
+			if (nb > 1) {  // (one workgroup looks at no state)
+				k_fill_u64<<<grid_for(nb, 256), 256, 0, s>>>(h->pack_state.as<unsigned long long>(), nb, 0ull);
+				HIP_LAUNCH_CHECK(h);
+			}
 			ProfScope ps(h, "pack", (double)nseq * (16.0 + 16.0 + 8.0));
 			k_pack_scan<<<(unsigned)nb, PK_NT, 0, s>>>(h->chars.as<uint8_t>(), h->offs.as<uint32_t>(), seq_map, row_base,
 			                                         set_of, nseq, d, h->pk.as<uint64_t>(), h->voff.as<uint64_t>(),
@@ -1538,7 +1557,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			// slots, with room for the 16-byte read at the end of the last run
 			TRY(ensure(h, h->tile_rec, sizeof(uint32_t) * (size_t)(tplan.ntiles * TL_CAP + 4)));
 			TRY(ensure(h, h->tile_offs, sizeof(uint16_t) * (size_t)(tplan.ntiles * pitch)));
-			TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
+			if (tplan.bin_groups > 3)
+				TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
 			if (d >= 2 && !h->del_sets_set) {
 				static const std::vector<uint32_t> sets = [] {
 					std::vector<uint32_t> all;
@@ -1575,6 +1595,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			bn.pk = ta.pk;
 			bn.ntiles = tplan.ntiles;
 			bn.cpitch = cpitch;
+			bn.offs = ta.offs;
+			bn.pitch = pitch;
 			bn.nb = nbins;
 			bn.nt = tplan.bin_nt;
 			bn.groups = tplan.bin_groups;

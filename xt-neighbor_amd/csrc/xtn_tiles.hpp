@@ -477,8 +477,10 @@ struct BinArgs {
 	const uint32_t* first;
 	const uint64_t* pk;
 	int64_t ntiles, cpitch;
+	const uint16_t* offs;    // the tiles' own rows, `pitch` apart (groups 3, which has no cols)
+	int32_t pitch;
 	int32_t nb;
-	int32_t nt, groups;      // the instantiation: BIN_NT or BIN_WIDE_NT threads, 18 or 9 groups each
+	int32_t nt, groups;      // the instantiation: BIN_NT or BIN_WIDE_NT threads, 18, 9 or 3 groups each
 	int32_t lb;              // index bits of a record
 	int32_t len_bits;        // length bits above them
 	int32_t key_low;         // lowest key bit of a record (above it the key's bits below the bin; zeros may lie
@@ -488,7 +490,7 @@ struct BinArgs {
 	uint32_t id_lo, id_hi;   // only pairs whose smaller id lies in [id_lo, id_hi)
 	uint64_t* pairs;
 	int64_t pcap;
-	RunCtrs* ctr;            // n_cand; pairs_small: record pairs of equal key; n_big set when a bin lists more
+	RunCtrs* ctr;            // n_cand; n_records (groups 3); pairs_small: record pairs of equal key; n_big set when a bin lists more
 	                         // records than fit, coarse_ovf when it outgrows another bound
 };
 
@@ -570,13 +572,20 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // QPT 18: bins of up to 36864 slots, an eighth of whose records may be
 // listed; QPT 9 (distances 3 and 4, where a neighbouring pair shares hundreds
 // of variants): half as many slots and a list for half of their records.
+// QPT 3: bins of up to 6144 slots of a small input, where the time is latency:
+// less to clear and fewer rounds, every record may be listed, and the runs
+// come from the tiles' own rows, a tile per thread (a few hundred lines per
+// bin instead of a transposing launch). 160 003 records (10 000 CDR3s, d = 1):
+// 15 us, with 18 groups 21 beside 7 of k_tile_cols.
 template <int NT, int QPT, bool PARTS>
 __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 	constexpr int X = NT / BIN_NT;  // the wide form: everything twice, one workgroup per CU
-	constexpr int B1 = 17 + X, B2 = 15 + X, HBITS = (QPT == 18 ? 11 : 10) + X;
-	static_assert((X == 1 || X == 2) && (QPT == 18 || QPT == 9), "bitmaps of 7 bits or more and a quarter of that per record");
+	constexpr bool FEW = QPT == 3;
+	constexpr int B1 = FEW ? 16 : 17 + X, B2 = B1 - 2, HBITS = (QPT == 18 ? 11 : 10) + X;
+	static_assert((X == 1 || X == 2) && (QPT == 18 || QPT == 9 || FEW), "bitmaps of 7 bits or more and a quarter of that per record");
+	static_assert(!FEW || !PARTS, "every record fits the list");
 	constexpr int QCAP = NT * QPT;
-	constexpr int SVC = QPT == 18 ? (1 << B1) / 8 / 6 / 64 * 64 : 7168 * X;  // records listed in step 3
+	constexpr int SVC = QPT == 18 ? (1 << B1) / 8 / 6 / 64 * 64 : FEW ? QCAP * 4 : 7168 * X;  // records listed in step 3
 	constexpr int HEADS = 1 << HBITS;
 	constexpr int PLC = QPT == 18 ? (QCAP * 4 - HEADS * 4 - SVC * 2) / 4 : 1024 * X;
 	static_assert(PLC >= NT, "room for pairs beside the lists");
@@ -624,27 +633,44 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		if (t == 0)
 			s_nsv = s_npl = 0;
 		// 1. eight tiles per thread and round
+		constexpr int TR = FEW ? 1 : 8;
 		uint32_t nq = 0;
-		const uint16_t* const r0 = a.cols + (int64_t)b * a.cpitch;
-		for (int64_t tb = 0; tb < a.ntiles; tb += NT * 8) {
-			const int64_t tile0 = tb + t * 8;
-			uint4 x = make_uint4(0u, 0u, 0u, 0u), y = x;
-			if (tile0 < a.cpitch) {
-				x = *reinterpret_cast<const uint4*>(r0 + tile0);
-				y = *reinterpret_cast<const uint4*>(r0 + a.cpitch + tile0);
-			}
-			const uint32_t xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w};
-			uint32_t st[8], n[8], q = 0;
+		const uint16_t* const r0 = FEW ? a.offs + b : a.cols + (int64_t)b * a.cpitch;
+		if (FEW && b == 0) {
+			uint32_t c = 0;
+			for (int64_t tile = t; tile < a.ntiles; tile += NT)
+				c += a.offs[tile * a.pitch + a.nb];
+			uint32_t tot;
+			block_excl_scan<NT>(c, s_tmp, &tot);
+			if (t == 0)
+				atomicAdd(&a.ctr->n_records, (unsigned long long)tot);
+		}
+		for (int64_t tb = 0; tb < a.ntiles; tb += NT * TR) {
+			const int64_t tile0 = tb + t * TR;
+			uint32_t st[TR], n[TR], q = 0;
+			if constexpr (FEW) {
+				const bool in = tile0 < a.ntiles;
+				st[0] = in ? r0[tile0 * a.pitch] : 0u;
+				n[0] = in ? r0[tile0 * a.pitch + 1] - st[0] : 0u;
+				q = (n[0] + 3) / 4;
+			} else {
+				uint4 x = make_uint4(0u, 0u, 0u, 0u), y = x;
+				if (tile0 < a.cpitch) {
+					x = *reinterpret_cast<const uint4*>(r0 + tile0);
+					y = *reinterpret_cast<const uint4*>(r0 + a.cpitch + tile0);
+				}
+				const uint32_t xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
-			for (int j = 0; j < 8; ++j) {
-				st[j] = (xs[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
-				n[j] = ((ys[j / 2] >> (16 * (j & 1))) & 0xFFFFu) - st[j];
-				q += (n[j] + 3) / 4;
+				for (int j = 0; j < TR; ++j) {
+					st[j] = (xs[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
+					n[j] = ((ys[j / 2] >> (16 * (j & 1))) & 0xFFFFu) - st[j];
+					q += (n[j] + 3) / 4;
+				}
 			}
 			uint32_t tot;
 			uint32_t pos = nq + block_excl_scan<NT>(q, s_tmp, &tot);
 #pragma unroll
-			for (int j = 0; j < 8; ++j) {
+			for (int j = 0; j < TR; ++j) {
 				uint32_t at = ((uint32_t)(tile0 + j) << TL_CAP_BITS) + st[j];
 				for (uint32_t left = n[j]; left > 0;) {
 					const uint32_t c = left < 4u ? left : 4u;
