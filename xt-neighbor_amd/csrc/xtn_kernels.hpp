@@ -2147,4 +2147,13 @@ __global__ void k_fill_u64(unsigned long long* p, int64_t n, unsigned long long 
 		p[i] = v;
 }
 
+// two ranges of words cleared by one launch
+__global__ void k_clear_u64(unsigned long long* p, int64_t n, unsigned long long* q, int64_t m) {
+	const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n)
+		p[i] = 0ull;
+	else if (i < n + m)
+		q[i - n] = 0ull;
+}
+
 }  // namespace xtn

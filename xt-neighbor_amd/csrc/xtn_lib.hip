@@ -131,6 +131,8 @@ struct xtn_handle {
 	int tune_low = 0;           // pair bits left unsorted for the select's in-group ranking: 0, 8, 16, 24
 	int tune_coarse_sep = 0;    // 1: the records' first ordering pass as a pass of its own (tuned)
 	bool tail_full = false;     // a group outgrew the select's window: full sorts until new sequences
+	bool groups_off = false;    // a group of ids got more candidates than fit: the tail's passes until new
+	                            // sequences
 	bool bin_parts = false;     // a bin listed more records than fit: bins in parts until new sequences
 	bool coarse_off = false;    // a sub-range of the generator's coarse pass overflowed: the separate
 	                            // pass until new sequences
@@ -710,6 +712,8 @@ struct TailPlan {
 	int low_bits = 0;  // > 0: the select ranks the bits below in LDS (k_select_grouped)
 	int64_t sort_tiles = 0, sel_tiles = 0;
 	bool small = false;  // k_tail_small instead of all of these
+	int groups = 0;      // > 0: k_tail_count, k_tail_split and k_tail_group over up to as many groups
+	TailGroups tg{};
 };
 
 // LSD passes of the next candidate sort over 2 * idb pair bits: the sort
@@ -726,6 +730,7 @@ int tail_passes(const xtn_handle* h, int idb) {
 int tail_prepare(xtn_handle* h, int64_t pcap, int idb, int64_t out_keep, TailPlan* tp) {
 	tp->pcap = pcap;
 	tp->small = false;
+	tp->groups = 0;
 	tp->passes = tail_passes(h, idb);
 	tp->low_bits = std::max(0, 2 * idb - 8 * tp->passes);
 	const int64_t sort_tile = h->tune_sort_tile, sel_tile = (int64_t)h->tune_select_nt * SL_IT;
@@ -741,6 +746,29 @@ int tail_prepare(xtn_handle* h, int64_t pcap, int idb, int64_t out_keep, TailPla
 	return XTN_OK;
 }
 
+// The tail in up to `groups` groups of the ids [lo, hi); its workspace, the
+// search counters and the tail's block cleared by one launch.
+int tail_groups(xtn_handle* h, int groups, uint32_t lo, uint32_t hi, TailPlan* tp) {
+	tp->groups = groups;
+	// look-back words, fill, counts, infos
+	const int bits = tail_stretch_bits(tp->pcap);
+	const int64_t words = (int64_t)groups * (1 + TG_PITCH / 2) + (1 << bits) / 2;
+	TRY(ensure(h, h->tail_state, sizeof(uint64_t) * (size_t)(words + groups)));
+	uint64_t* p = h->tail_state.as<uint64_t>() + groups;
+	tp->tg.fill = reinterpret_cast<uint32_t*>(p);
+	p += (int64_t)groups * TG_PITCH / 2;
+	tp->tg.count = reinterpret_cast<uint32_t*>(p);
+	p += (1 << bits) / 2;
+	tp->tg.info = reinterpret_cast<TailGroup*>(p);
+	tp->tg.id0 = lo;
+	tp->tg.shift = std::max(0, bits_for((int64_t)(hi - lo) - 1) - bits);
+	const int64_t head = (int64_t)(sizeof(CtlBlock) / 8);
+	k_clear_u64<<<grid_for(head + words, 256), 256, 0, h->stream>>>(ctr_field(h, 0), head,
+	                                                                h->tail_state.as<unsigned long long>(), words);
+	HIP_LAUNCH_CHECK(h);
+	return XTN_OK;
+}
+
 // the tail's launches over the candidates in `pairs` (count: the search
 // counter), outputs written from out_pairs[out_off]; the tail block must be
 // zero (zero_ctl)
@@ -750,6 +778,9 @@ int issue_tail(xtn_handle* h, const TailPlan& tp, int idb, const uint32_t* seq_m
 	hipStream_t s = h->stream;
 	CtlBlock* cb = ctl_block(h);
 	const unsigned long long* n_dev = &cb->rc.n_cand;
+	// profile byte counts: the candidates of the previous run (the count of
+	// this one is only on the device)
+	const double cand = (double)h->last_pairs;
 	SelectArgs sa{};
 	sa.n_dev = n_dev;
 	sa.cap = tp.pcap;
@@ -770,16 +801,37 @@ int issue_tail(xtn_handle* h, const TailPlan& tp, int idb, const uint32_t* seq_m
 	sa.spin_limit = h->spin_limit;
 	if (tp.small) {
 		sa.keys = h->pairs.as<uint64_t>();
-		ProfScope ps(h, "tail_small", 8.0 * (double)h->last_pairs);
-		small_tail_kernel(h->cfg.distance, h->cfg.measure)<<<1, TS_NT, 0, s>>>(sa, (2 * idb + 7) / 8);
+		ProfScope ps(h, "tail_small", 8.0 * cand);
+		sa.state = h->tail_state.as<uint64_t>();
+		block_tail_kernels(h->cfg.distance, h->cfg.measure).small<<<1, TS_NT, 0, s>>>(sa, (2 * idb + 7) / 8);
+		HIP_LAUNCH_CHECK(h);
+		return XTN_OK;
+	}
+	if (tp.groups > 0) {
+		const unsigned g = grid_for(tp.pcap, TG_CAP);
+		const bool fine = tail_stretch_bits(tp.pcap) == 14;
+		{
+			ProfScope ps(h, "tail_count", 8.0 * cand);
+			(fine ? k_tail_count<14> : k_tail_count<12>)<<<std::min(g, 64u), TG_NT, 0, s>>>(h->pairs.as<uint64_t>(), n_dev,
+			                                                                           tp.pcap, idb, tp.tg);
+			HIP_LAUNCH_CHECK(h);
+		}
+		{
+			ProfScope ps(h, "tail_split", 16.0 * cand);
+			(fine ? k_tail_split<14, 1024> : k_tail_split<12, TG_NT>)<<<fine ? grid_for(tp.pcap, 1024 * TG_IT) : g,
+			                                                          fine ? 1024 : TG_NT, 0, s>>>(
+			    h->pairs.as<uint64_t>(), n_dev, tp.pcap, idb, tp.tg, h->pairs_alt.as<uint64_t>(), &cb->tc.overflow);
+			HIP_LAUNCH_CHECK(h);
+		}
+		sa.keys = h->pairs_alt.as<uint64_t>();
+		sa.state = h->tail_state.as<uint64_t>();
+		ProfScope ps(h, "tail_group", 8.0 * cand + 40.0 * (double)h->last_unique + 9.0 * (double)h->last_out);
+		block_tail_kernels(h->cfg.distance, h->cfg.measure).group<<<tp.groups, TG_NT, 0, s>>>(sa, tp.tg);
 		HIP_LAUNCH_CHECK(h);
 		return XTN_OK;
 	}
 	uint32_t* state = h->tail_state.as<uint32_t>();
 	const int64_t nsort = (int64_t)tp.passes * tp.sort_tiles * RS_BINS;
-	// profile byte counts: the candidates of the previous run (the count of
-	// this one is only on the device)
-	const double cand = (double)h->last_pairs;
 	{
 		ProfScope ps(h, "tail_hist", 8.0 * cand);
 		const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(tp.sort_tiles, 256));
@@ -1787,11 +1839,23 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			const bool small = h->tune_low == 0 && (h->last_pairs > 0 && !h->no_alloc
 			                                            ? h->last_pairs <= SMALL_TAIL_EXPECTED
 			                                            : V <= SMALL_TAIL_RECORDS);
+			// (from distance 4 on one id alone brings thousands of candidates,
+			// which no group holds, once there are some hundred thousand)
+			int groups = !small && h->tune_low == 0 && !h->no_alloc && !h->groups_off && (d < 4 || pcap <= TG_FINE / 2)
+			                 ? (int)tail_groups_max(pcap)
+			                 : 0;
+			if (groups > TG_MAX)
+				groups = 0;
 			// everything issued, one readback: the whole run of a single
 			// round is a graph once it has run the same way before
 			auto issue_all = [&]() -> int {
 				// counters first: the generator's coarse pass may flag an overflow
-				TRY(zero_ctl(h, true, true));
+				TRY(tail_prepare(h, pcap, idb, out_total, &tp));
+				tp.small = small;
+				if (groups)
+					TRY(tail_groups(h, groups, lo, hi_id, &tp));
+				else
+					TRY(zero_ctl(h, true, true));
 				if (!grouped) {
 					TRY(prologue());
 					TRY(plan_chunk((int64_t)V, g1));
@@ -1799,8 +1863,6 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 					TRY(issue_grouping(h, g1));
 					grouped = true;
 				}
-				TRY(tail_prepare(h, pcap, idb, out_total, &tp));
-				tp.small = small;
 				TRY(issue_buckets(h, g1, lo, hi_id, pcap));
 				StageScope sg(h, "verify");
 				TRY(issue_tail(h, tp, idb, seq_map, row_base, set_of, out_total));
@@ -1828,7 +1890,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				sig.select_nt = h->tune_select_nt;
 				sig.low = h->tail_full ? 0 : h->tune_low;
 				sig.coarse = h->coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
-				sig.pad = (h->bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0);
+				sig.pad = (h->bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0) | (groups ? 8 : 0);
 			}
 			const bool tiled = use_tiles();  // also of a replay, which plans nothing
 			bool via_graph = false;
@@ -1901,14 +1963,19 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				prologue_done = false;
 				continue;
 			}
-			if (small && !head.error && (int64_t)head.rc.n_cand > TS_CAP && (int64_t)head.rc.n_cand <= pcap &&
-			    head.rc.append == 0) {
-				// too many for the one workgroup: the tail over the candidates as
-				// they lie (a later run goes by their count)
+			if (!head.error && (int64_t)head.rc.n_cand <= pcap && head.rc.append == 0 &&
+			    ((small && (int64_t)head.rc.n_cand > TS_CAP) || (groups && head.overflow))) {
+				// too many for the one workgroup (a later run goes by their count)
+				// or for one of the groups (the passes until new sequences): the
+				// passes over the candidates as they lie
+				h->groups_off = h->groups_off || groups > 0;
+				TRY(zero_ctl(h, false, true));
 				TRY(tail_prepare(h, pcap, idb, out_total, &tp));
 				TRY(issue_tail(h, tp, idb, seq_map, row_base, set_of, out_total));
 				TRY(read_head(h, &head));
 			}
+			if (groups)
+				head.overflow = 0;  // not the select's
 			const bool clean =
 			    !head.error && !head.overflow && (int64_t)head.rc.n_cand <= pcap && head.rc.append == 0;
 			if (head.overflow)
@@ -2464,6 +2531,7 @@ int xtn_set_sequences(xtn_handle* h, const char* chars, const uint32_t* offsets,
 	h->tail_full = false;
 	h->coarse_off = false;
 	h->bin_parts = false;
+	h->groups_off = false;
 	return XTN_OK;
 }
 

@@ -5,9 +5,11 @@
 // The reference does this as sort_int2 + unique (xtn_inner.cu:138-142,
 // cub.cu:116-124, 156-163), cal_distance (kernel.cu:359-392) and the flag
 // compaction of postprocessing (xtn_inner.cu:147-165), each a separate device
-// call with host round trips in between. Here it is P + 2 launches with no
-// host involvement, all sized by a capacity and reading the actual candidate
-// count from device memory:
+// call with host round trips in between. Here a few thousand candidates take
+// one workgroup (k_tail_small), a few million three launches over groups of
+// neighbouring ids (k_tail_count, k_tail_split, k_tail_group), and what fits
+// neither P + 2 launches, none with host involvement, all sized by a capacity
+// and reading the actual candidate count from device memory. The last form:
 //
 //   k_tail_hist    one read of the candidates: the global count of every
 //                  8-bit digit of every LSD pass (P x 256 counters); also
@@ -730,109 +732,275 @@ __global__ __launch_bounds__(NT) void k_select_grouped(SelectArgs a) {
 	select_emit<NT, R>(a, tile, ntiles, s_k, s_d, nu, s_cc, &s_excl);
 }
 
-// The whole tail of up to TS_CAP candidates in one workgroup: sorted in LDS by
-// the passes of k_onesweep (keys in registers between them), the first of
-// each value verified a pair per lane, the kept ones written in order. Bound
+// The tail in groups of neighbouring smaller ids: k_tail_count counts the
+// candidates of a few thousand stretches of ids, k_tail_split cuts the stretches into
+// groups of about tail_group(n) candidates and gathers each, k_tail_group
+// sorts, verifies and writes a group in LDS. Three launches that read the
+// candidates four times, instead of a histogram, four to six passes over all
+// of them and the select, whose launches and look-backs are most of the time
+// up to a million candidates. Resident runs: 32 412 candidates (100 000 CDR3s,
+// d = 1) 39 us against 102 in seven launches, the run 94 against 147; 883 066
+// (1M, d = 2) 83 against 143, the run 892 against 936; 1.62M (5M, d = 1) 173
+// against 247; 2.66M (3M, d = 2) 195 against 255. A group that gets more
+// candidates than TG_CAP (one id, or a stretch of ids, with thousands of
+// neighbours) raises overflow, and the host takes the passes over the
+// candidates as they lie.
+constexpr int TG_NT = 512;
+constexpr int TG_IT = 8;
+constexpr int TG_CAP = TG_NT * TG_IT;
+constexpr int64_t TG_FINE = 524288;  // candidates from which the stretches are finer
+// log2 of the stretches: ids are rarely even in neighbours (ten times the mean
+// at the low ids of rows copied from earlier ones), so that a stretch has to
+// hold a small part of a group (883 066 candidates: 78 us in 4096 stretches, 83 in
+// 16 384; 1.62M outgrow a group of the former)
+constexpr int tail_stretch_bits(int64_t cap) { return cap <= TG_FINE ? 12 : 14; }
+constexpr int TG_MAX = 4096;  // groups at most
+
+// log2 of a group's candidates: half its capacity, less where that would leave
+// CUs without one
+__host__ __device__ constexpr int tail_group_bits(int64_t n) { return n <= 131072 ? 9 : n <= 262144 ? 10 : 11; }
+inline int64_t tail_groups_max(int64_t cap) {  // of up to cap candidates
+	return cap <= 131072 ? (cap >> 9) + 1 : std::max<int64_t>(257, (cap >> 11) + 1);
+}
+
+struct TailGroup {
+	uint32_t start;        // its first candidate
+	uint16_t first, last;  // its stretches
+};
+
+// workspace of the groups (fill and count zeroed before)
+struct TailGroups {
+	TailGroup* info;
+	uint32_t* fill;   // candidates placed so far, TG_PITCH words apart: a line each, since their atomics serialise
+	uint32_t* count;  // per stretch
+	uint32_t id0;     // the first id
+	int32_t shift;    // ids of a stretch
+};
+constexpr int TG_PITCH = 16;
+
+template <int BITS>
+__global__ __launch_bounds__(TG_NT) void k_tail_count(const uint64_t* __restrict__ keys,
+                                                    const unsigned long long* __restrict__ n_dev, int64_t cap, int idb,
+                                                    TailGroups g) {
+	constexpr int BINS = 1 << BITS;
+	__shared__ uint32_t s_cnt[BINS];
+	const int t = threadIdx.x;
+	const int64_t n = tail_count(n_dev, cap);
+	if ((int64_t)blockIdx.x * TG_CAP >= n)  // uniform
+		return;
+	for (int i = t; i < BINS; i += TG_NT)
+		s_cnt[i] = 0;
+	__syncthreads();
+	for (int64_t base = (int64_t)blockIdx.x * TG_CAP; base < n; base += (int64_t)gridDim.x * TG_CAP) {
+		uint64_t k[TG_IT];
+#pragma unroll
+		for (int r = 0; r < TG_IT; ++r)
+			k[r] = base + r * TG_NT + t < n ? keys[base + r * TG_NT + t] : ~0ull;  // no candidate has all bits set
+#pragma unroll
+		for (int r = 0; r < TG_IT; ++r)
+			if (k[r] != ~0ull)
+				atomicAdd(&s_cnt[((uint32_t)(k[r] >> idb) - g.id0) >> g.shift], 1u);
+	}
+	__syncthreads();
+	for (int i = t; i < BINS; i += TG_NT)
+		if (s_cnt[i])
+			atomicAdd(&g.count[i], s_cnt[i]);
+}
+
+// Every workgroup scans the stretches' counts by itself (16 KB from L2) rather
+// than wait for one that does; the first writes the groups down.
+template <int BITS, int NT>
+__global__ __launch_bounds__(NT) void k_tail_split(const uint64_t* __restrict__ keys,
+                                                    const unsigned long long* __restrict__ n_dev, int64_t cap, int idb,
+                                                    TailGroups g, uint64_t* __restrict__ out,
+                                                    uint32_t* __restrict__ overflow) {
+	constexpr int BINS = 1 << BITS;
+	__shared__ uint32_t s_start[BINS];
+	__shared__ uint32_t s_cnt[TG_MAX];
+	__shared__ uint32_t s_gst[TG_MAX];
+	__shared__ uint32_t s_tmp[NT / WAVE + 1];
+	constexpr int PER = BINS / NT;
+	const int t = threadIdx.x;
+	const int64_t n = tail_count(n_dev, cap);
+	const int64_t base = (int64_t)blockIdx.x * (NT * TG_IT);
+	if (base >= n)  // uniform
+		return;
+	const int gb = tail_group_bits(n);
+	const int ng = (int)(n >> gb) + 1;  // <= TG_MAX
+	uint64_t k[TG_IT];
+#pragma unroll
+	for (int r = 0; r < TG_IT; ++r)
+		k[r] = base + r * NT + t < n ? keys[base + r * NT + t] : ~0ull;
+	uint32_t c[PER], sum = 0;
+	int heavy = 0;
+#pragma unroll
+	for (int j = 0; j < PER; ++j) {
+		c[j] = g.count[t * PER + j];
+		sum += c[j];
+		heavy |= c[j] > (uint32_t)TG_CAP;
+	}
+	for (int i = t; i < ng; i += NT)
+		s_cnt[i] = 0;
+	if (__syncthreads_or(heavy)) {  // no cut makes its group fit
+		if (t == 0 && blockIdx.x == 0)
+			atomicOr(overflow, 1u);
+		return;
+	}
+	uint32_t run = block_excl_scan<NT>(sum, s_tmp, (uint32_t*)nullptr);
+#pragma unroll
+	for (int j = 0; j < PER; ++j) {
+		s_start[t * PER + j] = run;
+		run += c[j];
+	}
+	__syncthreads();
+	// a stretch is in the group its first candidate falls in; start <= n
+	for (int i = t; i < BINS; i += NT) {
+		const uint32_t s = s_start[i], q = s >> gb;
+		if (i == 0 || s_start[i - 1] >> gb != q) {
+			s_gst[q] = s;
+			if (blockIdx.x == 0) {
+				g.info[q].start = s;
+				g.info[q].first = (uint16_t)i;
+			}
+		}
+		if (blockIdx.x == 0 && (i == BINS - 1 || s_start[i + 1] >> gb != q))
+			g.info[q].last = (uint16_t)i;
+	}
+	uint32_t at[TG_IT], gr[TG_IT];
+#pragma unroll
+	for (int r = 0; r < TG_IT; ++r) {
+		const bool in = k[r] != ~0ull;
+		gr[r] = in ? s_start[((uint32_t)(k[r] >> idb) - g.id0) >> g.shift] >> gb : 0u;
+		at[r] = in ? atomicAdd(&s_cnt[gr[r]], 1u) : 0u;
+	}
+	__syncthreads();
+	for (int i = t; i < ng; i += NT)
+		if (s_cnt[i])
+			s_cnt[i] = s_gst[i] + atomicAdd(&g.fill[i * TG_PITCH], s_cnt[i]);
+	__syncthreads();
+#pragma unroll
+	for (int r = 0; r < TG_IT; ++r)
+		if (k[r] != ~0ull)
+			out[s_cnt[gr[r]] + at[r]] = k[r];
+}
+
+// n <= NT * IT candidates from keys: sorted in LDS by the passes of k_onesweep
+// (keys in registers between them; lo is taken off each key meanwhile), the
+// first of each value verified a pair per lane, the kept ones written in order
+// after those of the tiles before. The candidates are spread over all waves,
+// so that a pass is as few dependent rounds as they allow.
+template <int D, int NT, int IT>
+__device__ __forceinline__ void tail_block(const SelectArgs& a, const uint64_t* __restrict__ keys, int n, uint64_t lo,
+                                           int passes, int64_t tile, int64_t ntiles) {
+	__shared__ uint64_t s_k[NT * IT];
+	__shared__ uint32_t s_cnt[NT / WAVE][RS_BINS];
+	__shared__ uint32_t s_dpre[RS_BINS];
+	__shared__ uint32_t s_scan[NT / WAVE + 1];
+	__shared__ int8_t s_d[NT * IT];
+	__shared__ uint32_t s_cc[IT * NT / WAVE + 1];
+	__shared__ uint32_t s_excl;
+	const int t = threadIdx.x;
+	const int lane = lane_id();
+	const int w = t / WAVE;
+	uint32_t nu = 0;
+	if (n > 0) {  // uniform
+		const int seg = (n + NT - 1) / NT * WAVE;  // positions of a wave, <= IT * WAVE
+		const int wrem = n - w * seg;
+		const int w_valid = wrem <= 0 ? 0 : (wrem < seg ? wrem : seg);
+		uint64_t k[IT];
+#pragma unroll
+		for (int r = 0; r < IT; ++r)
+			k[r] = r * WAVE + lane < w_valid ? keys[w * seg + r * WAVE + lane] - lo : 0ull;
+		for (int p = 0; p < passes; ++p) {
+			uint32_t lp[IT];
+			rank_tile_g<NT, IT>(k, w_valid, 8 * p, lp, s_cnt, s_dpre, s_scan);
+#pragma unroll
+			for (int r = 0; r < IT; ++r)
+				if (lp[r] != 0xFFFFFFFFu)
+					s_k[lp[r]] = k[r];
+			__syncthreads();
+#pragma unroll
+			for (int r = 0; r < IT; ++r)
+				k[r] = r * WAVE + lane < w_valid ? s_k[w * seg + r * WAVE + lane] : 0ull;
+		}
+		__syncthreads();
+		// the first of each value, in rows of NT positions
+		uint32_t uflags = 0;
+#pragma unroll
+		for (int r = 0; r < IT; ++r) {
+			const int q = r * NT + t;
+			k[r] = q < n ? s_k[q] : 0ull;
+			if (q < n && (q == 0 || s_k[q - 1] != k[r]))
+				uflags |= 1u << r;
+		}
+		uint32_t pos[IT];
+		nu = striped_rank<NT, IT>(uflags, pos, s_cc);  // (its barriers end the reads above)
+#pragma unroll
+		for (int r = 0; r < IT; ++r)
+			if (uflags & (1u << r))
+				s_k[pos[r]] = k[r] + lo;
+		__syncthreads();
+		select_verify<D, NT>(a, s_k, s_d, nu);
+	}
+	select_emit<NT, IT>(a, tile, ntiles, s_k, s_d, nu, s_cc, &s_excl);
+}
+
+template <int D>
+__global__ __launch_bounds__(TG_NT) void k_tail_group(SelectArgs a, TailGroups g) {
+	const int64_t b = blockIdx.x;
+	uint32_t n = g.fill[b * TG_PITCH];
+	if (n > (uint32_t)TG_CAP) {  // uniform
+		if (threadIdx.x == 0)
+			atomicOr(&a.ctl->overflow, 1u);
+		n = 0;  // the groups after this one wait on its counts all the same
+	}
+	TailGroup q{};
+	if (n > 0)
+		q = g.info[b];
+	const uint64_t lo = (uint64_t)(g.id0 + ((uint32_t)q.first << g.shift)) << a.idb;
+	const uint32_t span = ((uint32_t)(q.last - q.first + 1) << g.shift) - 1u;  // the largest id - lo's
+	const int bits = a.idb + 32 - __clz((int)(span | 1u));
+	tail_block<D, TG_NT, TG_IT>(a, a.keys + q.start, (int)n, lo, (bits + 7) / 8, b, gridDim.x);
+}
+
+// The whole tail of up to TS_CAP candidates in one workgroup and launch. Bound
 // by latency: a few thousand candidates are no work for the chip, and the
 // passes' launches, gaps and look-backs cost more than the one CU's time (a
 // resident run at d = 1: 3000 CDR3s, 1026 candidates: 21 us against six
 // launches of 61, the run 93 us against 117; 17 000, 5499: 51 against 81, the
-// run 129 against 149). The candidates are spread over all waves, so that a
-// pass is as few dependent rounds as they allow. More candidates than TS_CAP
-// write nothing (the host sees their count).
+// run 129 against 149). More candidates than TS_CAP write nothing (the host
+// sees their count).
 constexpr int TS_NT = 1024;
 constexpr int TS_IT = 8;
 constexpr int TS_CAP = TS_NT * TS_IT;
 
 template <int D>
 __global__ __launch_bounds__(TS_NT) void k_tail_small(SelectArgs a, int passes) {
-	__shared__ uint64_t s_k[TS_CAP];
-	__shared__ uint32_t s_cnt[TS_NT / WAVE][RS_BINS];
-	__shared__ uint32_t s_dpre[RS_BINS];
-	__shared__ uint32_t s_scan[TS_NT / WAVE + 1];
-	__shared__ int8_t s_d[TS_CAP];
-	__shared__ uint32_t s_cc[TS_IT * TS_NT / WAVE + 1];
-	const int t = threadIdx.x;
-	const int lane = lane_id();
-	const int w = t / WAVE;
-	const int64_t n64 = tail_count(a.n_dev, a.cap);
-	if (n64 > TS_CAP || n64 < (int64_t)*a.n_dev)  // uniform
+	const int64_t n = tail_count(a.n_dev, a.cap);
+	if (n > TS_CAP || n < (int64_t)*a.n_dev)  // uniform
 		return;
-	const int n = (int)n64;
-	const int seg = (n + TS_NT - 1) / TS_NT * WAVE;  // positions of a wave, <= TS_IT * WAVE
-	const int wrem = n - w * seg;
-	const int w_valid = wrem <= 0 ? 0 : (wrem < seg ? wrem : seg);
-	uint64_t k[TS_IT];
-#pragma unroll
-	for (int r = 0; r < TS_IT; ++r)
-		k[r] = r * WAVE + lane < w_valid ? a.keys[w * seg + r * WAVE + lane] : 0ull;
-	for (int p = 0; p < passes; ++p) {
-		uint32_t lp[TS_IT];
-		rank_tile_g<TS_NT, TS_IT>(k, w_valid, 8 * p, lp, s_cnt, s_dpre, s_scan);
-#pragma unroll
-		for (int r = 0; r < TS_IT; ++r)
-			if (lp[r] != 0xFFFFFFFFu)
-				s_k[lp[r]] = k[r];
-		__syncthreads();
-#pragma unroll
-		for (int r = 0; r < TS_IT; ++r)
-			k[r] = r * WAVE + lane < w_valid ? s_k[w * seg + r * WAVE + lane] : 0ull;
-	}
-	__syncthreads();
-	// the first of each value, in rows of TS_NT positions
-	uint32_t uflags = 0;
-#pragma unroll
-	for (int r = 0; r < TS_IT; ++r) {
-		const int q = r * TS_NT + t;
-		k[r] = q < n ? s_k[q] : 0ull;
-		if (q < n && (q == 0 || s_k[q - 1] != k[r]))
-			uflags |= 1u << r;
-	}
-	uint32_t pos[TS_IT];
-	const uint32_t nu = striped_rank<TS_NT, TS_IT>(uflags, pos, s_cc);  // (its barriers end the reads above)
-#pragma unroll
-	for (int r = 0; r < TS_IT; ++r)
-		if (uflags & (1u << r))
-			s_k[pos[r]] = k[r];
-	__syncthreads();
-	select_verify<D, TS_NT>(a, s_k, s_d, nu);
-	uint32_t kflags = 0;
-#pragma unroll
-	for (int r = 0; r < TS_IT; ++r) {
-		const uint32_t q = (uint32_t)(r * TS_NT + t);
-		if (q < nu && s_d[q] >= 0)
-			kflags |= 1u << r;
-	}
-	const uint32_t nk = striped_rank<TS_NT, TS_IT>(kflags, pos, s_cc);
-	if (t == 0) {
-		a.ctl->n_unique = nu;
-		a.ctl->n_out = nk;
-	}
-	const uint64_t idmask = (1ull << a.idb) - 1ull;
-#pragma unroll
-	for (int r = 0; r < TS_IT; ++r)
-		if (kflags & (1u << r)) {
-			const uint32_t q = (uint32_t)(r * TS_NT + t);
-			const uint64_t p = s_k[q];
-			a.out_pairs[pos[r]] = make_int2((int)(p >> a.idb), (int)(p & idmask));
-			a.out_dist[pos[r]] = s_d[q];
-		}
+	tail_block<D, TS_NT, TS_IT>(a, a.keys, (int)n, 0ull, passes, 0, 1);
 }
 
 typedef void (*SmallTailFn)(SelectArgs, int);
-inline SmallTailFn small_tail_kernel(int distance, int measure) {
+typedef void (*GroupTailFn)(SelectArgs, TailGroups);
+struct BlockTailFns {
+	SmallTailFn small;
+	GroupTailFn group;
+};
+inline BlockTailFns block_tail_kernels(int distance, int measure) {
 	if (measure == 1)
-		return k_tail_small<1>;
+		return {k_tail_small<1>, k_tail_group<1>};
 	switch (distance) {
-	case 1: return k_tail_small<1>;
-	case 2: return k_tail_small<2>;
-	case 3: return k_tail_small<3>;
-	case 4: return k_tail_small<4>;
-	case 5: return k_tail_small<5>;
-	case 6: return k_tail_small<6>;
-	case 7: return k_tail_small<7>;
-	case 8: return k_tail_small<8>;
-	default: return k_tail_small<0>;
+	case 1: return {k_tail_small<1>, k_tail_group<1>};
+	case 2: return {k_tail_small<2>, k_tail_group<2>};
+	case 3: return {k_tail_small<3>, k_tail_group<3>};
+	case 4: return {k_tail_small<4>, k_tail_group<4>};
+	case 5: return {k_tail_small<5>, k_tail_group<5>};
+	case 6: return {k_tail_small<6>, k_tail_group<6>};
+	case 7: return {k_tail_small<7>, k_tail_group<7>};
+	case 8: return {k_tail_small<8>, k_tail_group<8>};
+	default: return {k_tail_small<0>, k_tail_group<0>};
 	}
 }
 
