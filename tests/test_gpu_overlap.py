@@ -127,3 +127,19 @@ def test_cli_overlap_airr(tmp_path):
                         "-N", "2", "-o", str(out2)], capture_output=True, env=env, timeout=120)
     assert r.returncode == 0, r.stderr
     assert out2.read_bytes() == read_golden("expected_airr_overlap_d1.txt")
+
+
+@pytest.mark.parametrize("copies,distinct", [(3, 30_000), (1, 70_000), (40, 1_500)])
+def test_rows_whose_hashes_meet(engine, copies, distinct):
+    # some strings share the hash bits that order the rows (24 of them up to
+    # half a million rows: about 27 pairs among 30 000), and their copies come
+    # mixed
+    rng = np.random.default_rng(copies)
+    chars, offsets = xtn.synth_nn(70 + copies, distinct, planted=0.2, max_edits=1)
+    seqs = xtn.decode(chars, offsets) * copies
+    seqs = [seqs[i] for i in rng.permutation(len(seqs))]
+    freq = rng.integers(1, 100, len(seqs)).tolist()
+    rep = np.sort(rng.integers(0, 7, len(seqs))).tolist()
+    got = run(engine, seqs, freq=freq, rep=rep, d=1)
+    want = oracle.overlap(*xtn.encode(seqs), freq, rep, 1, 0)
+    assert got.tolist() == want.tolist()

@@ -91,7 +91,7 @@ struct xtn_handle {
 	DBuf pk, voff, recs, recs_alt, hist, scan_tmp, runs_small, runs_big, big_pre, pairs, pairs_alt,
 	    flags, pos, dist, out_pairs, out_dist, ctrs, part_hist, scalar;
 	// overlap-mode workspaces
-	DBuf ov_keys, ov_keys_alt, ov_vals, ov_vals_alt, ov_info, ov_leader, ov_ustart, ov_umap,
+	DBuf ov_keys, ov_keys_alt, ov_vals, ov_info, ov_leader, ov_ustart, ov_umap,
 	    ov_cnt, ov_matrix, ov_present;
 
 	int64_t out_len = 0;
@@ -2147,20 +2147,21 @@ int overlap_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callba
 	TRY(ensure(h, h->scalar, sizeof(uint64_t)));
 	HIP_TRY(h, hipMemcpyAsync(h->ov_keys_alt.p, info, sizeof(xtn_seq_info) * (size_t)n, hipMemcpyHostToDevice, s));
 	k_fill_u64<<<1, 256, 0, s>>>(h->scalar.as<unsigned long long>(), 1, 0xFFFFFFFF00000000ull);
-	k_split_info<<<grid_for(n, 256), 256, 0, s>>>(h->ov_keys_alt.as<int32_t>(), n, h->ov_info.as<int32_t>(),
+	k_split_info<<<std::min(grid_for(n, 256), (unsigned)SI_GRID), 256, 0, s>>>(h->ov_keys_alt.as<int32_t>(), n, h->ov_info.as<int32_t>(),
 	                                               h->ov_info.as<int32_t>() + n, h->scalar.as<uint32_t>());
 	HIP_LAUNCH_CHECK(h);
 	const int32_t* freq_d = h->ov_info.as<int32_t>();
 	const int32_t* rep_d = freq_d + n;
 
-	// exact duplicates: hash sort, leaders, stable sort by leader position
+	// exact duplicates: hash sort, then the runs of equal hash bits by string.
+	// 24 hash bits, a pass less than 32, up to half a million rows: the runs
+	// that mix strings are then a few thousand at most.
 	const int idb = bits_for(std::max(n - 1, 1));
-	const int K = std::min(32, 64 - idb);
+	const int K = std::min(n <= 1 << 19 ? 24 : 32, 64 - idb);
 	const int rs = 64 - K;
 	TRY(ensure(h, h->ov_keys, sizeof(uint64_t) * (size_t)n));
 	TRY(ensure(h, h->ov_keys_alt, sizeof(uint64_t) * (size_t)n));
 	TRY(ensure(h, h->ov_vals, sizeof(uint32_t) * (size_t)n));
-	TRY(ensure(h, h->ov_vals_alt, sizeof(uint32_t) * (size_t)n));
 	{
 		ProfScope ps(h, "ov_hash", (double)n * 28.0);
 		k_hash_rows<<<grid_for(n, 256), 256, 0, s>>>(h->chars.as<uint8_t>(), h->offs.as<uint32_t>(), n, idb,
@@ -2175,8 +2176,6 @@ int overlap_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callba
 		                                            h->ov_keys_alt.as<uint64_t>(), h->ov_vals.as<uint32_t>());
 		HIP_LAUNCH_CHECK(h);
 	}
-	TRY(radix_sort(h, h->ov_keys_alt, h->ov_keys, &h->ov_vals, &h->ov_vals_alt, n, 0, bits_for(n),
-	               "ov_sort_leader"));
 	const uint64_t* lead = h->ov_keys_alt.as<uint64_t>();
 	const uint32_t* rows = h->ov_vals.as<uint32_t>();
 
@@ -2334,7 +2333,7 @@ void xtn_close(xtn_handle* h) {
 	                &h->scan_tmp, &h->runs_small, &h->runs_big, &h->big_pre, &h->pairs,
 	                &h->pairs_alt, &h->flags, &h->pos, &h->dist, &h->out_pairs, &h->out_dist,
 	                &h->ctrs, &h->part_hist, &h->scalar, &h->ov_keys, &h->ov_keys_alt, &h->ov_vals,
-	                &h->ov_vals_alt, &h->ov_info, &h->ov_leader, &h->ov_ustart, &h->ov_umap,
+	                &h->ov_info, &h->ov_leader, &h->ov_ustart, &h->ov_umap,
 	                &h->ov_cnt, &h->ov_matrix, &h->ov_present, &h->bstart, &h->ovf, &h->set_of,
 	                &h->set_offs, &h->tseq, &h->tail_state, &h->pack_state};
 	for (DBuf* b : bufs)

@@ -3,11 +3,10 @@
 // Flow on the device:
 //   k_hash_rows        64-bit hash of every full string, row id in the low bits
 //   radix sort         equal hashes adjacent, rows ascending inside (stable)
-//   k_leaders          inside each run of equal hash bits, every row points at
-//                      the first row with an identical string (exact compare)
-//   radix sort (k,v)   by leader position: duplicates contiguous, rows
-//                      ascending (the stable full-string sort of
-//                      xtn_overlap_inner.cu:57-73 gives the same groups)
+//   k_leaders          inside each run of equal hash bits, identical strings
+//                      brought together (exact compare), rows ascending (the
+//                      stable full-string sort of xtn_overlap_inner.cu:57-73
+//                      gives the same groups)
 //   k_group_flags/_starts  group starts, one representative row per group
 //   k_exact_term       f_a*f_b into (rep_a, rep_b) for a <= b of a group
 //                      (init_overlap_output, kernel.cu:565-584)
@@ -34,20 +33,26 @@ constexpr int OV_LDS_REPS = 64;  // R <= 64: per-workgroup LDS copy of the matri
 // The caller's rows ({frequency, repertoire, original_index}, 12 bytes each)
 // split into a frequency and a repertoire array, with the repertoire count
 // (largest index + 1) into ctl[0] and the first row holding a negative
-// repertoire index into ctl[1] (ctl zeroed / all ones beforehand); one
-// atomic per wave for each.
+// repertoire index into ctl[1] (ctl zeroed / all ones beforehand). Bound by
+// the row stream once the atomics on the two addresses are few: one per
+// workgroup of a grid-stride grid of SI_GRID, and only by one that would move
+// the bound (a stale read costs an atomic more, never a wrong bound). One per
+// wave took 104 us for 575 928 rows, 11 this way.
+constexpr int SI_GRID = 256;
 __global__ __launch_bounds__(256) void k_split_info(const int32_t* __restrict__ rows, int32_t n,
                                                     int32_t* __restrict__ freq, int32_t* __restrict__ rep,
                                                     uint32_t* __restrict__ ctl) {
-	const int32_t i = blockIdx.x * 256 + threadIdx.x;
-	int32_t r = 0;
-	if (i < n) {
-		freq[i] = rows[3 * (int64_t)i];
-		r = rows[3 * (int64_t)i + 1];
+	__shared__ uint32_t s_top[256 / WAVE], s_bad[256 / WAVE];
+	uint32_t top = 0, bad = 0xFFFFFFFFu;
+	for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+		const int32_t r = rows[3 * i + 1];
+		freq[i] = rows[3 * i];
 		rep[i] = r;
+		if (r >= 0)
+			top = (uint32_t)r + 1u > top ? (uint32_t)r + 1u : top;
+		else
+			bad = (uint32_t)i < bad ? (uint32_t)i : bad;
 	}
-	uint32_t top = i < n && r >= 0 ? (uint32_t)r + 1u : 0u;
-	uint32_t bad = i < n && r < 0 ? (uint32_t)i : 0xFFFFFFFFu;
 #pragma unroll
 	for (int o = WAVE / 2; o > 0; o >>= 1) {
 		const uint32_t t2 = (uint32_t)__shfl_xor((int)top, o);
@@ -55,9 +60,16 @@ __global__ __launch_bounds__(256) void k_split_info(const int32_t* __restrict__ 
 		top = t2 > top ? t2 : top;
 		bad = b2 < bad ? b2 : bad;
 	}
-	// atomics on one address serialise: a wave only updates a bound it
-	// would move (a stale read costs one atomic more, never a wrong bound)
 	if ((threadIdx.x & (WAVE - 1)) == 0) {
+		s_top[threadIdx.x / WAVE] = top;
+		s_bad[threadIdx.x / WAVE] = bad;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		for (int w = 1; w < 256 / WAVE; ++w) {
+			top = s_top[w] > top ? s_top[w] : top;
+			bad = s_bad[w] < bad ? s_bad[w] : bad;
+		}
 		if (top && top > __hip_atomic_load(&ctl[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
 			atomicMax(&ctl[0], top);
 		if (bad != 0xFFFFFFFFu && bad < __hip_atomic_load(&ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -100,9 +112,13 @@ __device__ __forceinline__ bool same_string(const uint8_t* __restrict__ chars,
 	return true;
 }
 
-// One thread per run head of equal (rec >> rs): walks its run in order and
-// gives every element the sorted position of the first element holding the
-// same string. key_out[e] = leader position, val_out[e] = row.
+// One thread per run head of equal (rec >> rs): walks its run and lays it out
+// with identical strings together, the groups in the order of their first
+// rows and the rows of a group ascending. key_out[e] = the position of its
+// group's first row, val_out[e] = row. Runs of one string, nearly all, are in
+// order as they come; one that mixes strings is ordered here, group by group,
+// instead of by a sort of all rows by group (107 us of radix passes for
+// 575 928 rows).
 __global__ __launch_bounds__(256) void k_leaders(const uint64_t* __restrict__ recs, int32_t n, int rs,
                                                  int idb, const uint8_t* __restrict__ chars,
                                                  const uint32_t* __restrict__ offs,
@@ -119,12 +135,14 @@ __global__ __launch_bounds__(256) void k_leaders(const uint64_t* __restrict__ re
 	while (end < n && (recs[end] >> rs) == cur)
 		++end;
 	const uint32_t head_row = (uint32_t)(recs[i] & mask);
+	bool mixed = false;
 	for (int32_t e = i; e < end; ++e) {
 		const uint32_t row = (uint32_t)(recs[e] & mask);
 		int32_t lead = i;
 		if (e != i && !same_string(chars, offs, row, head_row)) {
 			// a different string with the same hash bits: first earlier
 			// element of this run with the same string, else itself
+			mixed = true;
 			lead = e;
 			for (int32_t p = i + 1; p < e; ++p)
 				if (key_out[p] == (uint64_t)p && same_string(chars, offs, row, (uint32_t)(recs[p] & mask))) {
@@ -135,6 +153,18 @@ __global__ __launch_bounds__(256) void k_leaders(const uint64_t* __restrict__ re
 		key_out[e] = (uint64_t)lead;
 		val_out[e] = row;
 	}
+	if (!mixed)
+		return;
+	int32_t q = i;
+	for (int32_t p = i; p < end; ++p) {
+		if (key_out[p] != (uint64_t)p)
+			continue;
+		for (int32_t e = p; e < end; ++e)
+			if (key_out[e] == (uint64_t)p)
+				val_out[q++] = (uint32_t)(recs[e] & mask);
+	}
+	for (q = i + 1; q < end; ++q)  // (key_out[i] = i)
+		key_out[q] = same_string(chars, offs, val_out[q], val_out[q - 1]) ? key_out[q - 1] : (uint64_t)q;
 }
 
 __global__ __launch_bounds__(256) void k_group_flags(const uint64_t* __restrict__ keys, int32_t n,
