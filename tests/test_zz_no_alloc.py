@@ -101,3 +101,27 @@ def test_noalloc_limits():
     # and it still works after the rejected calls
     st, got = noalloc(lib, hip, chars, offsets, 1, 0, 1 << 20)
     assert st == 0 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n,d,measure", [(2, 1, 0), (255, 1, 0), (300, 1, 1), (1000, 1, 0), (30_000, 1, 0), (60, 2, 1),
+                                         (8_000, 2, 0), (15, 3, 0), (1_500, 3, 1), (5, 4, 0), (200, 4, 0), (420, 4, 0),
+                                         (20, 5, 0)])
+def test_noalloc_tiles_at_the_scratch_sizes(n, d, measure):
+    # from a few rows to nearly the records that the scratch holds; rows that
+    # come many times (which leave the tiles) and others between, so that each
+    # call finds what another left
+    lib = xtn.load_library()
+    hip = hip_runtime()
+    for chars, offsets in (xtn.synth_nn(63, n, planted=0.3, max_edits=min(d, 2)),
+                           xtn.encode(xtn.decode(*xtn.synth_nn(64, max(2, n // 8), planted=0.3, max_edits=1)) * (6 if d == 1 else 3)),
+                           xtn.synth_nn(65, max(2, n // 2), 9.0, 3.0, 2, 30, planted=0.3, max_edits=1)):
+        st, got = noalloc(lib, hip, chars, offsets, d, measure, 1 << 20)
+        assert st == 0
+        want = resident(chars, offsets, d, measure)
+        assert np.array_equal(got, want)
+
+
+def test_noalloc_still_refuses_more_candidates_than_its_scratch():
+    chars, offsets = xtn.encode(xtn.decode(*xtn.synth_nn(64, 1000, planted=0.3, max_edits=1)) * 6)
+    st, _ = noalloc(xtn.load_library(), hip_runtime(), chars, offsets, 2, 0, 1 << 20)
+    assert st == 6

@@ -85,9 +85,6 @@ struct xtn_handle {
 	DBuf recs_all, recs_part;  // chunked runs: every record once, then ordered by part
 	DBuf seg_cur, seg_ctl;  // the generator's coarse pass: sub-range cursors, digit tiling
 	DBuf tile_rec, tile_offs, tile_cols;  // tiles ordered by bin, their bin starts by tile and by bin
-	DBuf del_sets_d;  // the deletion sets of distances 2, 3 and 4, one after another (xtn_tiles.hpp): written
-	                  // once, since a captured run reads its distance's
-	bool del_sets_set = false;
 	DBuf pk, voff, recs, recs_alt, hist, scan_tmp, runs_small, runs_big, big_pre, pairs, pairs_alt,
 	    flags, pos, dist, out_pairs, out_dist, ctrs, part_hist, scalar;
 	// overlap-mode workspaces
@@ -946,9 +943,14 @@ struct Grouping {
 struct TilePlan {
 	uint32_t tile = 0;  // records between the starts of two tiles
 	int64_t ntiles = 0;
+	int slot_bits = 0;  // of a tile's slots
 	int bin_bits = 0;
 	int idx_bits = 0;
 	int bin_nt = BIN_NT, bin_groups = 18;  // the bin kernel's instantiation
+	int pitch() const { return ((1 << bin_bits) + 64 + 63) / 64 * 64; }
+	// slots, with room for the 16-byte read at the end of the last run
+	size_t rec_bytes() const { return sizeof(uint32_t) * ((size_t)(ntiles << slot_bits) + 4); }
+	size_t offs_bytes() const { return sizeof(uint16_t) * (size_t)(ntiles * pitch()); }
 };
 
 // the tiling of V records of n sequences
@@ -966,6 +968,7 @@ TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
 	TilePlan p;
 	p.tile = (uint32_t)tile;
 	p.ntiles = (V + tile - 1) / tile;
+	p.slot_bits = bits_for(tile + (int64_t)host_variant_count(MAX_PREFIX, d) - 1);
 	// index bits for twice the average tile's sequences (at distance 4 a
 	// short string has a tenth or less of the average's variants, so that
 	// the few sequences of a tile vary more)
@@ -1363,8 +1366,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	// chunks as before.
 	const int64_t bucket_records = (int64_t)65536 * h->tune_target;
 	auto tiles_wanted = [&]() {
-		return d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && (int64_t)V < (int64_t)INT32_MAX && !h->no_alloc &&
-		       h->cfg.max_records_per_chunk <= 0 && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
+		return d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && (int64_t)V < (int64_t)INT32_MAX &&
+		       (h->no_alloc ? (int64_t)V <= h->cfg.max_records_per_chunk : h->cfg.max_records_per_chunk <= 0) && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
 		       !h->coarse_off && !h->tail_safe &&
 		       ((int64_t)V <= bucket_records || h->tune_target >= DEFAULT_BUCKET_TARGET);
 	};
@@ -1385,8 +1388,11 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	budget = std::max<int64_t>(budget, 1 << 16);
 	const int64_t sorted_budget = budget;  // a chunk of the other layouts
 	// (a tiled record takes ~8 B with its share of the bin starts)
-	const TilePlan tplan =
+	TilePlan tplan =
 	    tiles_wanted() && (double)V * 8.0 <= (double)free_b * 0.6 ? plan_tiles((int64_t)V, nseq, d, h->n_cu) : TilePlan{};
+	if (h->no_alloc && (tplan.bin_groups != 3 || tplan.rec_bytes() > h->tile_rec.cap ||
+	                    tplan.offs_bytes() > h->tile_offs.cap || 4 * (size_t)(tplan.ntiles + 1) > h->tseq.cap))
+		tplan = TilePlan{};  // more than the slices of the static scratch hold
 	auto use_tiles = [&]() { return tplan.ntiles > 0 && tiles_wanted(); };
 	if (use_tiles())
 		budget = (int64_t)V;
@@ -1605,31 +1611,14 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		if (use_tiles()) {
 			g.tiles = true;
 			const int64_t cpitch = (tplan.ntiles + 63) / 64 * 64;
-			const int nbins = 1 << tplan.bin_bits, pitch = (nbins + 64 + 63) / 64 * 64;
-			// slots, with room for the 16-byte read at the end of the last run
-			TRY(ensure(h, h->tile_rec, sizeof(uint32_t) * (size_t)(tplan.ntiles * TL_CAP + 4)));
-			TRY(ensure(h, h->tile_offs, sizeof(uint16_t) * (size_t)(tplan.ntiles * pitch)));
+			const int nbins = 1 << tplan.bin_bits, pitch = tplan.pitch();
+			TRY(ensure(h, h->tile_rec, tplan.rec_bytes()));
+			TRY(ensure(h, h->tile_offs, tplan.offs_bytes()));
 			if (tplan.bin_groups > 3)
 				TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
-			if (d >= 2 && !h->del_sets_set) {
-				static const std::vector<uint32_t> sets = [] {
-					std::vector<uint32_t> all;
-					for (int k = 2; k <= TL_MAX_D; ++k) {
-						const std::vector<uint32_t> one = del_sets(k);
-						all.insert(all.end(), one.begin(), one.end());
-					}
-					return all;
-				}();
-				TRY(ensure(h, h->del_sets_d, sizeof(uint32_t) * sets.size()));
-				HIP_TRY(h, hipMemcpyAsync(h->del_sets_d.p, sets.data(), sizeof(uint32_t) * sets.size(),
-				                          hipMemcpyHostToDevice, s));
-				h->del_sets_set = true;
-			}
 			TileArgs& ta = g.ta;
-			ta.del = h->del_sets_d.as<uint32_t>();
-			for (int k = 2; k < d; ++k)
-				ta.del += tl_sets(k);
 			ta.n = nseq;
+			ta.slot_bits = tplan.slot_bits;
 			ta.pk = h->pk.as<uint64_t>();
 			ta.voff = h->voff.as<uint64_t>();
 			ta.first = h->tseq.as<uint32_t>();
@@ -1649,6 +1638,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			bn.cpitch = cpitch;
 			bn.offs = ta.offs;
 			bn.pitch = pitch;
+			bn.slot_bits = tplan.slot_bits;
 			bn.nb = nbins;
 			bn.nt = tplan.bin_nt;
 			bn.groups = tplan.bin_groups;
@@ -2328,7 +2318,7 @@ void xtn_close(xtn_handle* h) {
 		return;
 	(void)hipSetDevice(h->cfg.device);
 	(void)hipStreamSynchronize(h->stream);
-	DBuf* bufs[] = {&h->del_sets_d, &h->tile_rec, &h->tile_offs, &h->tile_cols, &h->recs_all, &h->recs_part, &h->seg_cur, &h->seg_ctl, &h->bcount, &h->ctl, &h->chars, &h->offs, &h->pk, &h->voff,
+	DBuf* bufs[] = {&h->tile_rec, &h->tile_offs, &h->tile_cols, &h->recs_all, &h->recs_part, &h->seg_cur, &h->seg_ctl, &h->bcount, &h->ctl, &h->chars, &h->offs, &h->pk, &h->voff,
 	                &h->recs, &h->recs_alt, &h->hist,
 	                &h->scan_tmp, &h->runs_small, &h->runs_big, &h->big_pre, &h->pairs,
 	                &h->pairs_alt, &h->flags, &h->pos, &h->dist, &h->out_pairs, &h->out_dist,
@@ -3139,7 +3129,7 @@ bool carve_scratch(xtn_handle* h, uint8_t* base) {
 	take(h->pk, 16 * NA_MAX_SEQS);
 	take(h->voff, 8 * (NA_MAX_SEQS + 1));
 	take(h->pack_state, 8 * (NA_MAX_SEQS / 256 + 1));
-	take(h->tseq, 4 * (NA_MAX_RECORDS / GEN_TILE + 2));
+	take(h->tseq, 4 * (NA_MAX_RECORDS / 2048 + 2));  // (a tile of either record layout holds 2048 records or more)
 	take(h->recs, 8 * NA_MAX_RECORDS);
 	take(h->recs_alt, 8 * NA_MAX_RECORDS);
 	take(h->hist, 4 * RS_BINS * rtiles);
@@ -3160,6 +3150,10 @@ bool carve_scratch(xtn_handle* h, uint8_t* base) {
 	take(h->tail_state, 4 * (4 * sort_tiles * RS_BINS + 2 * sel_tiles));  // 2 * idb <= 32 bits: 4 passes
 	take(h->pos, 4 * (NA_MAX_PAIRS / SEL_TILE + NA_MAX_PAIRS / SEL_NT + 4));
 	take(h->dist, NA_MAX_PAIRS);
+	// tiles where the other layout has its records and its runs, which they replace
+	h->tile_rec.p = h->recs.p;
+	h->tile_rec.cap = h->recs.cap + h->recs_alt.cap;
+	h->tile_offs = h->runs_small;
 	return off <= NA_SCRATCH_BYTES;
 }
 

@@ -41,7 +41,7 @@ namespace xtn {
 
 constexpr int TL_NT = 1024;
 constexpr int TL_CAP_BITS = 15;
-constexpr int TL_CAP = 1 << TL_CAP_BITS;  // record slots of a tile
+constexpr int TL_CAP = 1 << TL_CAP_BITS;  // records of a tile, at most
 constexpr int TL_IT = TL_CAP / TL_NT;     // records of a thread
 constexpr int TL_BINS_MAX = 8192;
 constexpr uint32_t TL_NONE = 0xFFFFFFFFu;  // no record (a tile's last index is never used)
@@ -100,8 +100,7 @@ struct TileArgs {
 	const uint64_t* pk;
 	const uint64_t* voff;
 	const uint32_t* first;   // first sequence of each tile, [ntiles] = n
-	const uint32_t* del;     // the deletion sets of the distance (del_sets)
-	uint32_t* out;           // TL_CAP slots per tile
+	uint32_t* out;           // 2^slot_bits slots per tile
 	uint16_t* offs;          // a row of `pitch` per tile: the start of each bin, then the tile's total
 	unsigned long long* ovf;
 	int32_t pitch;
@@ -109,6 +108,7 @@ struct TileArgs {
 	int32_t lb;              // index bits of a record
 	int32_t sets;            // the prefixes carry query sets
 	uint32_t n;              // sequences
+	int32_t slot_bits;       // a tile's slots, at most TL_CAP
 };
 
 // A record: key bits below the bin, the low bits of the variant's length, the
@@ -119,31 +119,38 @@ __device__ __forceinline__ uint32_t tile_record(uint32_t h, int bin_bits, uint32
 	return ((h << bin_bits) & ~(((LM + 1u) << lb) - 1u)) | ((len & LM) << lb) | idx;
 }
 
-// The deletion sets of at most d positions, ordered by their largest position
-// as c_del_tables is: positions ascending, five bits each from bit 0, NO_DEL
-// above the real ones, the number of deletions from bit 25.
-inline std::vector<uint32_t> del_sets(int d) {
-	std::vector<uint32_t> r;
-	auto put = [&](const int* q, int m) {
-		uint32_t e = (uint32_t)m << 25;
-		for (int k = 0; k < TL_MAX_D; ++k)
-			e |= (uint32_t)(k < m ? q[k] : NO_DEL) << (5 * k);
-		r.push_back(e);
-	};
-	put(nullptr, 0);
-	for (int top = 0; top < MAX_PREFIX; ++top)
-		for (uint32_t below = 0; below < 1u << top; ++below) {
-			if (__builtin_popcount(below) >= d)
-				continue;
-			int q[TL_MAX_D], m = 0;
-			for (int i = 0; i < top; ++i)
-				if ((below >> i) & 1u)
-					q[m++] = i;
-			q[m++] = top;
-			put(q, m);
-		}
-	return r;
+// The deletion sets of at most 2, 3 and 4 positions, ordered by their largest
+// position as c_del_tables is: positions ascending, five bits each from bit 0,
+// NO_DEL above the real ones, the number of deletions from bit 25. In global
+// memory: each workgroup copies its distance's to LDS once.
+struct TileDelSets {
+	uint32_t d2[DEL_SETS2], d3[DEL_SETS3], d4[DEL_SETS4];
+};
+
+constexpr uint32_t tile_del_entry(int m, int a, int b, int c, int d) {
+	return (uint32_t)a | ((uint32_t)b << 5) | ((uint32_t)c << 10) | ((uint32_t)d << 15) | ((uint32_t)m << 25);
 }
+
+constexpr TileDelSets make_tile_del_sets() {
+	TileDelSets t{};
+	constexpr int N = NO_DEL;
+	t.d2[0] = t.d3[0] = t.d4[0] = tile_del_entry(0, N, N, N, N);
+	int q2 = 1, q3 = 1, q4 = 1;
+	for (int m = 0; m < MAX_PREFIX; ++m) {
+		t.d2[q2++] = t.d3[q3++] = t.d4[q4++] = tile_del_entry(1, m, N, N, N);
+		for (int k = 0; k < m; ++k) {
+			t.d2[q2++] = t.d3[q3++] = t.d4[q4++] = tile_del_entry(2, k, m, N, N);
+			for (int j = 0; j < k; ++j) {
+				t.d3[q3++] = t.d4[q4++] = tile_del_entry(3, j, k, m, N);
+				for (int i = 0; i < j; ++i)
+					t.d4[q4++] = tile_del_entry(4, i, j, k, m);
+			}
+		}
+	}
+	return t;
+}
+
+__device__ const TileDelSets g_tile_del_sets = make_tile_del_sets();
 
 // the bins' counts (16 bits each, two to a word) turned into their starts,
 // also written to the tile's row; returns the total
@@ -190,7 +197,7 @@ __device__ __forceinline__ void tile_refuse(const TileArgs& a, uint16_t* row, in
 }
 
 // Distances 2 to 4. The deletion sets of a prefix come in the order of
-// their largest position (del_sets), a thread takes consecutive records,
+// their largest position, a thread takes consecutive records,
 // and the record's rank inside its bin comes from the same LDS atomic that
 // counts it; the records stay in registers until the tables are dead and
 // the ordered tile takes their LDS. At distance 4 the colex unranking this
@@ -230,7 +237,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 	}
 	const uint64_t v0 = a.voff[s0];
 	const uint32_t total = (uint32_t)(a.voff[s1] - v0);
-	if (total > (uint32_t)TL_CAP) {  // uniform; the tiling rules it out
+	if (total > 1u << a.slot_bits) {  // uniform; the tiling rules it out
 		tile_refuse(a, row, nb, true);
 		return;
 	}
@@ -238,8 +245,9 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 		s_cnt[i] = 0;
 	for (int i = t; i < MAX_PREFIX * 32; i += TL_NT)
 		(&u.s.terms[0][0])[i] = (&c_tile_terms.t[0][0])[i];
+	const uint32_t* const del = D == 2 ? g_tile_del_sets.d2 : D == 3 ? g_tile_del_sets.d3 : g_tile_del_sets.d4;
 	for (int i = t; i < NSETS; i += TL_NT)
-		u.s.del[i] = a.del[i];
+		u.s.del[i] = del[i];
 	__syncthreads();
 	for (int i = t; i < cnt; i += TL_NT) {
 		const uint64_t lo = a.pk[2 * (int64_t)(s0 + i)];
@@ -340,7 +348,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 		if (at[it] != TL_NONE)
 			u.rec[c16[at[it] >> 16] + (at[it] & 0xFFFFu)] = rec[it];
 	__syncthreads();
-	tile_out(u.rec, a.out + tile * TL_CAP, kept);
+	tile_out(u.rec, a.out + (tile << a.slot_bits), kept);
 }
 
 // Distance 1: a thread takes whole sequences and steps the key from one
@@ -362,7 +370,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles1(TileArgs a) {
 		tile_refuse(a, row, nb, cnt > 0);
 		return;
 	}
-	if (a.voff[s1] - a.voff[s0] > (uint64_t)TL_CAP) {  // uniform; the tiling rules it out
+	if (a.voff[s1] - a.voff[s0] > 1ull << a.slot_bits) {  // uniform; the tiling rules it out
 		tile_refuse(a, row, nb, true);
 		return;
 	}
@@ -410,7 +418,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles1(TileArgs a) {
 		s_rec[pos] = tile_record<1>(h, a.bin_bits, len, a.lb, idx);
 	});
 	__syncthreads();
-	tile_out(s_rec, a.out + tile * TL_CAP, total);
+	tile_out(s_rec, a.out + (tile << a.slot_bits), total);
 }
 
 // first[b] = the first sequence whose records start at or after b * tile (b <=
@@ -479,6 +487,7 @@ struct BinArgs {
 	int64_t ntiles, cpitch;
 	const uint16_t* offs;    // the tiles' own rows, `pitch` apart (groups 3, which has no cols)
 	int32_t pitch;
+	int32_t slot_bits;       // a tile's
 	int32_t nb;
 	int32_t nt, groups;      // the instantiation: BIN_NT or BIN_WIDE_NT threads, 18, 9 or 3 groups each
 	int32_t lb;              // index bits of a record
@@ -671,7 +680,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 			uint32_t pos = nq + block_excl_scan<NT>(q, s_tmp, &tot);
 #pragma unroll
 			for (int j = 0; j < TR; ++j) {
-				uint32_t at = ((uint32_t)(tile0 + j) << TL_CAP_BITS) + st[j];
+				uint32_t at = ((uint32_t)(tile0 + j) << a.slot_bits) + st[j];
 				for (uint32_t left = n[j]; left > 0;) {
 					const uint32_t c = left < 4u ? left : 4u;
 					if (pos < (uint32_t)QCAP)
@@ -765,7 +774,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		for (int k = 0; k < QPT; ++k) {
 			if (((hit[k * 4 / 32] >> (k * 4 % 32)) & 15u) == 0u)
 				continue;
-			const uint16_t tile = (uint16_t)(u2.list[k * NT + t] >> (TL_CAP_BITS + 2));
+			const uint16_t tile = (uint16_t)(u2.list[k * NT + t] >> (a.slot_bits + 2));
 #pragma unroll
 			for (int j = 0; j < 4; ++j)
 				if ((hit[(k * 4 + j) / 32] >> ((k * 4 + j) % 32)) & 1u) {
