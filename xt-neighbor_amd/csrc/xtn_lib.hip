@@ -586,11 +586,14 @@ constexpr int KEY_BITS = 32;             // hash bits that order records into ru
 // is one bucket without a pass, 52 us against 62 for 721.
 constexpr int64_t TILES_MIN_RECORDS = 4096;
 // The one-workgroup tail (k_tail_small) is taken for at most this many
-// candidates in the run before or, with none to go by, for at most this many
+// candidates in the run before, or with none to go by for at most this many
 // records. Each thousand candidates take its one CU 7 us; at 5499 it is 20 us
-// ahead of the passes, and towards its capacity of 8192 they meet.
+// ahead of the passes, at about 4400 the groups' three launches (k_tail_group)
+// have caught up. The run before may have been of other rows, so a run of more
+// than SMALL_TAIL_MAX records, where the tail matters less and ten thousands of
+// candidates are usual, goes by its own size.
 constexpr int64_t SMALL_TAIL_EXPECTED = 6000;
-constexpr uint64_t SMALL_TAIL_RECORDS = 200000;
+constexpr uint64_t SMALL_TAIL_RECORDS = 200000, SMALL_TAIL_MAX = 4000000;
 
 // device control block: the counters of the candidate search, then the
 // tail's block
@@ -1827,7 +1830,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			TRY(checked_candidates(h, g1, lo, hi_id, pmax, &pcap, &n_pairs, &split));
 		} else if (nparts == 1) {
 			const bool small = h->tune_low == 0 && (h->last_pairs > 0 && !h->no_alloc
-			                                            ? h->last_pairs <= SMALL_TAIL_EXPECTED
+			                                            ? h->last_pairs <= SMALL_TAIL_EXPECTED && V <= SMALL_TAIL_MAX
 			                                            : V <= SMALL_TAIL_RECORDS);
 			// (from distance 4 on one id alone brings thousands of candidates,
 			// which no group holds, once there are some hundred thousand)
