@@ -548,7 +548,7 @@ def main():
     progress(f"{args.workload}: {step_s * 1e3:.3f} ms per step")
     kernels = ["tiles", "tile_cols", "bins", "gen", "gen_coarse", "sort_rec_hist", "sort_rec_scatter", "region", "bucket", "runs", "pairs_small",
                "pairs_big",
-               "sort_seg_hist", "sort_seg_scatter", "tail_hist", "sort_pairs", "select", "pack", "scan",
+               "sort_seg_hist", "sort_seg_scatter", "tail_small", "tail_count", "tail_split", "tail_group", "tail_hist", "sort_pairs", "select", "pack", "scan",
                "gen_count"]
     prof = {k: eng.kernel_profile(k) for k in kernels}
     # the library prices the record-path launches at the V records of the

@@ -113,7 +113,8 @@ typedef struct {
 	int64_t n_candidates;  /* candidate pairs i != j emitted from runs (with
 	                          multiplicity; the copies a sequence's repeated
 	                          variants would add are not there when the
-	                          generator's coarse pass left them out) */
+	                          generator left those out, nor, in tiles, those
+	                          of a pair within one edit beyond its first) */
 	int64_t n_unique;      /* unique candidate pairs verified (U) */
 	int64_t n_output;      /* pairs (NN) or repertoire entries (overlap) out */
 	double ms_total;       /* device pipeline wall time */
@@ -125,21 +126,25 @@ typedef struct {
 	int64_t n_launches;    /* kernel launches of the last call */
 	int64_t n_syncs;       /* host waits on the device of the last call */
 	int64_t graph_replays; /* runs issued as one captured graph launch */
-	int64_t tail_passes;   /* 8-bit LSD passes of the last candidate sort: fewer
+	int64_t tail_passes;   /* 8-bit LSD passes that sort the candidates where
+	                          they are sorted as one (not where a workgroup
+	                          or groups of neighbouring ids take them): fewer
 	                          than the pair bits need when the select ranks
 	                          the low bits of each group in LDS, all of them
 	                          after a group outgrew the select's window on
 	                          this handle */
-	int64_t coarse_in_generator; /* 1: the generator ordered the records by their
-	                                top 8 hash bits itself; 0: a separate pass did
-	                                (always after a sub-range of the generator's
-	                                pass overflowed on this handle, until new
-	                                sequences) */
+	int64_t coarse_in_generator; /* 1: the generator ordered the records itself, into
+	                                tiles ordered by bin or by their top 8 hash
+	                                bits; 0: a separate pass did (always after
+	                                the generator's order outgrew a bound, or
+	                                met more equal pairs than records, on this
+	                                handle, until new sequences) */
 	int64_t n_records;     /* deletion records written: n_variants less the
 	                          repeated variants of a sequence (deleting any
 	                          residue of a run of equal ones gives the same
-	                          string), which the generator's coarse pass
-	                          leaves out; n_variants on the separate pass */
+	                          string) where the generator orders the records
+	                          and leaves them out; n_variants on the separate
+	                          pass */
 } xtn_stats;
 
 /* fills *cfg with defaults: distance 1, Levenshtein, device 0 */
