@@ -23,11 +23,11 @@
 #include <stdint.h>
 #include <type_traits>
 
+#include "xtn_plan.hpp"
 #include "xtn_prims.hpp"
 
 namespace xtn {
 
-constexpr int MAX_PREFIX = 18;      // xtn.h:8 MAX_COMPRESSED_LENGTH
 constexpr int PK_SET_SHIFT = 26;    // packed high word: 26 residue bits, then the set id
 constexpr uint32_t PK_SET_MASK = (1u << 30) - 1u;
 constexpr uint64_t PK_HI_MASK = (1ull << 56) - 1ull;  // residues + set, without the length byte
@@ -126,6 +126,25 @@ __global__ __launch_bounds__(256) void k_pack(const uint8_t* __restrict__ chars,
 	if (i >= n)
 		return;
 	vcount[i] = pack_one(chars, offs, seq_map, row_base, set_of, i, distance, pk);
+}
+
+// The sequences of each prefix length (counts[0..18], zeroed before), of which
+// V and the tiles follow, where the host doesn't hold the lengths.
+__global__ __launch_bounds__(256) void k_len_counts(const uint32_t* __restrict__ offs,
+                                                    const uint32_t* __restrict__ seq_map, uint32_t row_base, int32_t n,
+                                                    unsigned long long* __restrict__ counts) {
+	__shared__ uint32_t s_c[MAX_PREFIX + 1];
+	if (threadIdx.x <= MAX_PREFIX)
+		s_c[threadIdx.x] = 0;
+	__syncthreads();
+	for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+		const uint32_t o = seq_map ? seq_map[i] : row_base + (uint32_t)i;
+		const uint32_t len = offs[o + 1] - offs[o];
+		atomicAdd(&s_c[len < (uint32_t)MAX_PREFIX ? len : (uint32_t)MAX_PREFIX], 1u);
+	}
+	__syncthreads();
+	if (threadIdx.x <= MAX_PREFIX && s_c[threadIdx.x])
+		atomicAdd(&counts[threadIdx.x], (unsigned long long)s_c[threadIdx.x]);
 }
 
 // ---------------------------------------------------------- generation --

@@ -102,8 +102,6 @@ struct xtn_handle {
 	int64_t last_pairs = 0;
 	int64_t last_unique = 0, last_out = 0;  // the previous run's unique candidates and outputs
 	                                         // (byte counts of the output select's profile)
-	// host copy of the prefix lengths, and per-row prefix sums of the
-	// variant counts for one distance: V of any row range without a readback
 	int n_cu = 256;
 	// the single-chunk run captured as a graph: replayed while a run's
 	// signature (sizes, pointers, the allocation generation) matches
@@ -149,9 +147,10 @@ struct xtn_handle {
 	uint32_t spin_limit = LB_SPIN_LIMIT;  // XTN_LOOKBACK_SPIN_LIMIT overrides (tests of the fallback)
 	size_t free_cache = 0;   // hipMemGetInfo's free bytes, re-read after an allocation
 	bool free_valid = false;
+	// host copy of the prefix lengths and their counts: V and the tiles of any
+	// row range without a readback
 	std::vector<uint8_t> prefix_len;
-	std::vector<uint64_t> vprefix;
-	int vprefix_d = 0;
+	std::vector<uint32_t> len_cum;  // rows of each prefix length before every LEN_BLOCK rows (range_lengths)
 };
 
 namespace {
@@ -258,24 +257,46 @@ int grow_keep(xtn_handle* h, DBuf& b, size_t bytes, size_t keep) {
 	return XTN_OK;
 }
 
-int bits_for(int64_t maxval) {
-	int b = 1;
-	while (b < 62 && (1ll << b) <= maxval)
-		++b;
-	return b;
+// The lengths of rows [r0, r0 + n): the counts before every LEN_BLOCK rows,
+// made once for a handle's rows, and the rows at the two ends one by one.
+constexpr int64_t LEN_BLOCK = 1024;
+
+void add_lengths(const uint8_t* len, int64_t n, LenCounts* out) {
+	uint32_t c[4][MAX_PREFIX + 1] = {};  // (four: neighbours are often alike)
+	int64_t i = 0;
+	for (; i + 4 <= n; i += 4)
+		for (int k = 0; k < 4; ++k)
+			++c[k][len[i + k]];
+	for (; i < n; ++i)
+		++c[0][len[i]];
+	for (int L = 0; L <= MAX_PREFIX; ++L)
+		out->c[L] += (int64_t)c[0][L] + c[1][L] + c[2][L] + c[3][L];
 }
 
-// sum_{k <= min(d, L)} C(L, k) for the 18-residue prefix of a len-residue
-// sequence (the count k_pack computes on the device)
-uint64_t host_variant_count(uint32_t len, int d) {
-	const int L = len < 18 ? (int)len : 18;
-	const int m = d < L ? d : L;
-	uint64_t c = 1, total = 1;
-	for (int j = 1; j <= m; ++j) {
-		c = c * (uint64_t)(L - j + 1) / (uint64_t)j;
-		total += c;
+LenCounts range_lengths(xtn_handle* h, int64_t r0, int64_t n) {
+	LenCounts out;
+	const uint8_t* len = h->prefix_len.data();
+	const int64_t b0 = (r0 + LEN_BLOCK - 1) / LEN_BLOCK, b1 = (r0 + n) / LEN_BLOCK;
+	if (b1 <= b0 + 1) {
+		add_lengths(len + r0, n, &out);
+		return out;
 	}
-	return total;
+	constexpr int W = MAX_PREFIX + 1;
+	if (h->len_cum.empty()) {
+		const int64_t blocks = (int64_t)h->prefix_len.size() / LEN_BLOCK;
+		h->len_cum.assign((size_t)((blocks + 1) * W), 0);
+		LenCounts all;
+		for (int64_t b = 0; b < blocks; ++b) {
+			add_lengths(len + b * LEN_BLOCK, LEN_BLOCK, &all);
+			for (int L = 0; L < W; ++L)
+				h->len_cum[(size_t)((b + 1) * W + L)] = (uint32_t)all.c[L];
+		}
+	}
+	add_lengths(len + r0, b0 * LEN_BLOCK - r0, &out);
+	add_lengths(len + b1 * LEN_BLOCK, r0 + n - b1 * LEN_BLOCK, &out);
+	for (int L = 0; L < W; ++L)
+		out.c[L] += (int64_t)h->len_cum[(size_t)(b1 * W + L)] - h->len_cum[(size_t)(b0 * W + L)];
+	return out;
 }
 
 inline unsigned grid_for(int64_t n, int per_block) {
@@ -941,94 +962,6 @@ struct Grouping {
 	BinArgs bn{};
 };
 
-// ---- tiles and bins of one chunk (xtn_tiles.hpp)
-
-struct TilePlan {
-	uint32_t tile = 0;  // records between the starts of two tiles
-	int64_t ntiles = 0;
-	int slot_bits = 0;  // of a tile's slots
-	int bin_bits = 0;
-	int idx_bits = 0;
-	int bin_nt = BIN_NT, bin_groups = 18;  // the bin kernel's instantiation
-	int pitch() const { return ((1 << bin_bits) + 64 + 63) / 64 * 64; }
-	// slots, with room for the 16-byte read at the end of the last run
-	size_t rec_bytes() const { return sizeof(uint32_t) * ((size_t)(ntiles << slot_bits) + 4); }
-	size_t offs_bytes() const { return sizeof(uint16_t) * (size_t)(ntiles * pitch()); }
-};
-
-// the tiling of V records of n sequences
-TilePlan plan_tiles(int64_t V, int32_t n, int d, int n_cu) {
-	// a tile holds the sequences starting in its stretch of `tile` records,
-	// so up to one sequence's variants more, and no more sequences than its
-	// tables (half of that on average, for uneven lengths)
-	const int64_t most = TL_CAP - (int64_t)host_variant_count(MAX_PREFIX, d);
-	const double avg = (double)V / n;
-	int64_t tile = std::min<int64_t>(most, (int64_t)(0.5 * tl_seqs(d) * avg));
-	// whole rounds of one workgroup per CU
-	const int64_t rounds = (V + n_cu * tile - 1) / (n_cu * tile);
-	tile = std::max<int64_t>(std::min<int64_t>(tile, (V + n_cu * rounds - 1) / (n_cu * rounds)), 2048);
-	tile = std::min(tile, most);
-	TilePlan p;
-	p.tile = (uint32_t)tile;
-	p.ntiles = (V + tile - 1) / tile;
-	p.slot_bits = bits_for(tile + (int64_t)host_variant_count(MAX_PREFIX, d) - 1);
-	// index bits for twice the average tile's sequences (at distance 4 a
-	// short string has a tenth or less of the average's variants, so that
-	// the few sequences of a tile vary more)
-	p.idx_bits = d >= 4 ? tl_idx_bits(d) : std::min(bits_for((int64_t)(2.0 * (double)tile / avg) + 1), tl_idx_bits(d));
-	// The fewest bins whose runs fit the bin kernel's registers (a run, the
-	// records that one tile has for one bin, is Poisson and takes a group per
-	// four of them), and enough of them that bin and record leave 11 keys per
-	// record: two records meet by chance once in 20 or so.
-	const double key_bits = std::log2((double)V) + 3.5;
-	// a bin for every resident workgroup of the narrow form (two per CU)
-	// while they keep 512 records or more
-	const int min_bits = std::max(6, std::min(9, bits_for(V / 512) - 1));
-	auto bins_for = [&](int nt, int groups) {
-		for (int bits = min_bits; (1 << bits) <= TL_BINS_MAX; ++bits) {
-			const double lambda = (double)tile / (1 << bits);
-			double q = 0, w = std::exp(-lambda);
-			if (lambda > 200)
-				q = lambda / 4 + 0.375;
-			else
-				for (int k = 1; k < 400; ++k) {
-					w *= lambda / k;
-					q += w * ((k + 3) / 4);
-				}
-			if (q * (double)p.ntiles <= 0.965 * nt * groups && bits + 32 - tl_len_bits(d) - p.idx_bits >= key_bits)
-				return bits;
-		}
-		return 0;
-	};
-	// The form of few slots where the fewest bins suffice.
-	if (bins_for(BIN_NT, 3) == min_bits) {
-		p.bin_bits = min_bits;
-		p.bin_groups = 3;
-		return p;
-	}
-	// The narrow form first; where its bins would leave runs of fewer than six
-	// records, the wide one over half as many (at 1.15M CDR3s, d = 2: columns
-	// 29 us and bins 656 us against 51 and 660; at 50 000, d = 4, 24 and 599
-	// against 44 and 629); at distances 3 and 4 then the wide one of 18 groups,
-	// whose list still takes a fifth of the records.
-	const struct {
-		int nt, groups;
-	} forms[] = {{BIN_NT, d <= 2 ? 18 : 9}, {BIN_WIDE_NT, d <= 2 ? 18 : 9}, {BIN_WIDE_NT, 18}};
-	for (const auto& f : forms) {
-		const int bits = bins_for(f.nt, f.groups);
-		if (!bits || (p.bin_bits && bits >= p.bin_bits))
-			continue;
-		p.bin_bits = bits;
-		p.bin_nt = f.nt;
-		p.bin_groups = f.groups;
-		if ((double)tile / (1 << bits) >= 6.0)
-			break;
-	}
-	if (!p.bin_bits)
-		p.ntiles = 0;  // more records than the bins take
-	return p;
-}
-
 // sub-ranges per coarse digit in the generator's coarse pass: a generator
 // tile takes the one of its index mod 64 (tiles of one sub-range run on one
 // XCD), so each slot cursor sees 1/16384 of the tiles' claims (same-address
@@ -1329,20 +1262,24 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	TRY(ensure(h, h->pk, sizeof(uint64_t) * 2 * (size_t)nseq));
 	TRY(ensure(h, h->voff, sizeof(uint64_t) * ((size_t)nseq + 1)));
 	TRY(ensure(h, h->ctrs, sizeof(CtlBlock)));
-	uint64_t V = 0;
-	if (!seq_map && (int64_t)row_base + nseq <= (int64_t)h->prefix_len.size()) {
-		// the closed form the device scan sums
-		if (h->vprefix_d != d || h->vprefix.size() != h->prefix_len.size() + 1) {
-			uint64_t per[19];
-			for (int L = 0; L <= 18; ++L)
-				per[L] = host_variant_count((uint32_t)L, d);
-			h->vprefix.assign(h->prefix_len.size() + 1, 0);
-			for (size_t i = 0; i < h->prefix_len.size(); ++i)
-				h->vprefix[i + 1] = h->vprefix[i] + per[h->prefix_len[i]];
-			h->vprefix_d = d;
-		}
-		V = h->vprefix[row_base + nseq] - h->vprefix[row_base];
+	// the sequences by length give the number of records (the closed form the
+	// device scan sums) and the tiles
+	LenCounts lens;
+	const bool v_known = !seq_map && (int64_t)row_base + nseq <= (int64_t)h->prefix_len.size();
+	if (v_known) {
+		lens = range_lengths(h, row_base, nseq);
+	} else {
+		unsigned long long* counts = nullptr;
+		TRY(ensure(h, h->part_hist, sizeof(lens.c)));
+		counts = h->part_hist.as<unsigned long long>();
+		k_fill_u64<<<1, 256, 0, s>>>(counts, MAX_PREFIX + 1, 0ull);
+		HIP_LAUNCH_CHECK(h);
+		k_len_counts<<<std::min(grid_for(nseq, 256), 256u), 256, 0, s>>>(h->offs.as<uint32_t>(), seq_map, row_base, nseq,
+		                                                                counts);
+		HIP_LAUNCH_CHECK(h);
+		TRY(fetch(h, {{lens.c, counts, sizeof(lens.c)}}, s));
 	}
+	const uint64_t V = (uint64_t)lens.records(d, 0);
 	auto issue_pack = [&]() -> int {
 		StageScope sg(h, "generate");
 		{
@@ -1356,11 +1293,6 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		                        h->voff.as<uint64_t>() + nseq));
 		return XTN_OK;
 	};
-	const bool v_known = V > 0;
-	if (!v_known) {
-		TRY(issue_pack());
-		TRY(fetch(h, {{&V, h->voff.as<uint64_t>() + nseq, sizeof(uint64_t)}}, s));
-	}
 	st.n_variants = (int64_t)V;
 
 	// Enough records at distances 1 to 4: tiles ordered by bin (xtn_tiles.hpp),
@@ -1390,9 +1322,9 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	}
 	budget = std::max<int64_t>(budget, 1 << 16);
 	const int64_t sorted_budget = budget;  // a chunk of the other layouts
-	// (a tiled record takes ~8 B with its share of the bin starts)
-	TilePlan tplan =
-	    tiles_wanted() && (double)V * 8.0 <= (double)free_b * 0.6 ? plan_tiles((int64_t)V, nseq, d, h->n_cu) : TilePlan{};
+	TilePlan tplan = tiles_wanted() ? plan_tiles(lens, nseq, d, h->n_cu) : TilePlan{};
+	if ((double)tplan.rec_bytes() + (double)tplan.offs_bytes() + (double)tplan.cols_bytes() > (double)free_b * 0.6)
+		tplan = TilePlan{};
 	if (h->no_alloc && (tplan.bin_groups != 3 || tplan.rec_bytes() > h->tile_rec.cap ||
 	                    tplan.offs_bytes() > h->tile_offs.cap || 4 * (size_t)(tplan.ntiles + 1) > h->tseq.cap))
 		tplan = TilePlan{};  // more than the slices of the static scratch hold
@@ -1429,12 +1361,13 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	ga.part_bits = pbits;
 	ga.V = (int64_t)V;
 	ga.set_of = set_of;
-	// packing (unless done above to learn V) and the generator's tile table
+	// packing and the generator's tile table (several chunks, and a handle
+	// whose look-back once gave up, pack and scan by launches of their own)
 	bool prologue_done = false;
 	auto prologue = [&]() -> int {
 		if (prologue_done)
 			return XTN_OK;
-		if (v_known && nparts == 1 && !h->tail_safe) {
+		if (nparts == 1 && !h->tail_safe) {
 			// packing, offsets and tile table in one launch (its look-back
 			// shares the error flag the single-chunk run reads at its end)
 			const int64_t nb = (nseq + PK_SEQ - 1) / PK_SEQ;
@@ -1448,24 +1381,15 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				HIP_LAUNCH_CHECK(h);
 			}
 			ProfScope ps(h, "pack", (double)nseq * (16.0 + 16.0 + 8.0));
-			k_pack_scan<<<(unsigned)nb, PK_NT, 0, s>>>(h->chars.as<uint8_t>(), h->offs.as<uint32_t>(), seq_map, row_base,
-			                                         set_of, nseq, d, h->pk.as<uint64_t>(), h->voff.as<uint64_t>(),
-			                                         h->tseq.as<uint32_t>(), tl ? tplan.tile : 0u,
-			                                         h->pack_state.as<uint64_t>(), LB_SPIN_LIMIT,
-			                                         &ctl_block(h)->tc.error);
+			(tl ? k_pack_scan<true> : k_pack_scan<false>)<<<(unsigned)nb, PK_NT, 0, s>>>(
+			    h->chars.as<uint8_t>(), h->offs.as<uint32_t>(), seq_map, row_base, set_of, nseq, d,
+			    h->pk.as<uint64_t>(), h->voff.as<uint64_t>(), h->tseq.as<uint32_t>(), tplan.tile, tplan.least,
+			    h->pack_state.as<uint64_t>(), LB_SPIN_LIMIT, &ctl_block(h)->tc.error);
 			HIP_LAUNCH_CHECK(h);
 			ga.tile_seq = h->tseq.as<uint32_t>();
 		} else {
-			if (v_known)
-				TRY(issue_pack());
-			if (use_tiles()) {
-				TRY(ensure(h, h->tseq, sizeof(uint32_t) * (size_t)(tplan.ntiles + 1)));
-				k_tile_first<<<grid_for(nseq, 256), 256, 0, s>>>(h->voff.as<uint64_t>(), nseq, tplan.tile,
-				                                                 (uint32_t)tplan.ntiles, h->tseq.as<uint32_t>());
-				HIP_LAUNCH_CHECK(h);
-			} else {
-				TRY(tile_seq_table(h, s, nseq, V, &ga.tile_seq));
-			}
+			TRY(issue_pack());
+			TRY(tile_seq_table(h, s, nseq, V, &ga.tile_seq));
 		}
 		prologue_done = true;
 		return XTN_OK;
@@ -1613,12 +1537,12 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		g.nseq = nseq;
 		if (use_tiles()) {
 			g.tiles = true;
-			const int64_t cpitch = (tplan.ntiles + 63) / 64 * 64;
+			const int64_t cpitch = tplan.cpitch();
 			const int nbins = 1 << tplan.bin_bits, pitch = tplan.pitch();
 			TRY(ensure(h, h->tile_rec, tplan.rec_bytes()));
 			TRY(ensure(h, h->tile_offs, tplan.offs_bytes()));
 			if (tplan.bin_groups > 3)
-				TRY(ensure(h, h->tile_cols, sizeof(uint16_t) * (size_t)((nbins + 1) * cpitch)));
+				TRY(ensure(h, h->tile_cols, tplan.cols_bytes()));
 			TileArgs& ta = g.ta;
 			ta.n = nseq;
 			ta.slot_bits = tplan.slot_bits;
@@ -2518,8 +2442,7 @@ int xtn_set_sequences(xtn_handle* h, const char* chars, const uint32_t* offsets,
 	h->n_chars = total;
 	h->out_len = 0;
 	h->prefix_len.swap(plen);
-	h->vprefix.clear();
-	h->vprefix_d = 0;
+	h->len_cum.clear();
 	h->tail_full = false;
 	h->coarse_off = false;
 	h->bin_parts = false;

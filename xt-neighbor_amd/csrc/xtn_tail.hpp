@@ -1041,40 +1041,45 @@ inline SelectFn select_kernel(int distance, int measure, int nt, bool grouped) {
 // then writes its offset and records the generator tiles whose first record
 // it holds (tile_seq, as k_tile_seq); the last one writes voff[n] = V and
 // tile_seq[ceil(V / GEN_TILE)], since it holds record V - 1 (every sequence
-// has at least one variant, itself). With own_tile > 0 the table is
-// k_tile_first's over tiles of that many records instead. The waits are on lower-numbered
+// has at least one variant, itself). TILED: the table holds the first sequence
+// of each tile of plan_tiles instead, the one whose weights before it reach
+// the multiple of own_tile, and the number of sequences after the last; a
+// sequence weighs its records, or `least`, and the weights are summed in the
+// upper half of the same words (21 us at 1M CDR3s, as without). The waits are on lower-numbered
 // workgroups, which each XCD dispatches first; a wait past spin_limit
 // raises *error and the host redoes the run.
 constexpr int PK_NT = 1024;
 constexpr int PK_PER = 2;                // consecutive sequences per thread
 constexpr int PK_SEQ = PK_NT * PK_PER;  // sequences per workgroup: a short look-back chain
 
+template <bool TILED>
 __global__ __launch_bounds__(PK_NT) void k_pack_scan(const uint8_t* __restrict__ chars,
                                                    const uint32_t* __restrict__ offs,
                                                    const uint32_t* __restrict__ seq_map, uint32_t row_base,
                                                    const uint32_t* __restrict__ set_of, int32_t n, int distance,
                                                    uint64_t* __restrict__ pk, uint64_t* __restrict__ voff,
                                                    uint32_t* __restrict__ tile_seq, uint32_t own_tile,
-                                                   uint64_t* __restrict__ state, uint32_t spin_limit,
+                                                   uint32_t least, uint64_t* __restrict__ state, uint32_t spin_limit,
                                                    uint32_t* __restrict__ error) {
-	__shared__ uint32_t s_tmp[PK_NT / WAVE + 1];
+	__shared__ uint64_t s_tmp[PK_NT / WAVE + 1];
 	__shared__ uint64_t s_prefix;
 	const int t = threadIdx.x;
 	const int32_t i0 = blockIdx.x * PK_SEQ + PK_PER * t;
 	uint32_t c[PK_PER];
-	uint32_t csum = 0;
+	uint64_t csum = 0;  // the records, and above 31 bits the weights (a tiling's sums are below 2^31)
+	auto weight = [&](uint32_t r) -> uint64_t { return TILED ? (uint64_t)(r > least ? r : least) << LB2_SHIFT : 0ull; };
 #pragma unroll
 	for (int u = 0; u < PK_PER; ++u) {
 		const int32_t i = i0 + u;
 		c[u] = i < n ? pack_one(chars, offs, seq_map, row_base, set_of, i, distance, pk) : 0u;
-		csum += c[u];
+		csum += i < n ? c[u] + weight(c[u]) : 0ull;
 	}
-	uint32_t tot;
-	const uint32_t ex = block_excl_scan<PK_NT>(csum, s_tmp, &tot);  // <= PK_SEQ * 2^18
+	uint64_t tot;
+	const uint64_t ex = block_excl_scan<PK_NT>(csum, s_tmp, &tot);
 	const int64_t b = blockIdx.x;
 	if (t < WAVE) {
 		if (t == 0)
-			lb_store64(state + b, (b == 0 ? LB2_INC : LB2_AGG) | (uint64_t)tot);
+			lb_store64(state + b, (b == 0 ? LB2_INC : LB2_AGG) | tot);
 		const uint64_t prefix = b == 0 ? 0ull : lookback_wave(state, b, spin_limit, error);
 		if (t == 0) {
 			if (b > 0)
@@ -1084,6 +1089,9 @@ __global__ __launch_bounds__(PK_NT) void k_pack_scan(const uint8_t* __restrict__
 	}
 	__syncthreads();
 	uint64_t o = s_prefix + ex;
+	uint32_t w = (uint32_t)(o >> LB2_SHIFT);
+	if constexpr (TILED)
+		o &= (1ull << LB2_SHIFT) - 1ull;
 #pragma unroll
 	for (int u = 0; u < PK_PER; ++u) {
 		const int32_t i = i0 + u;
@@ -1091,16 +1099,18 @@ __global__ __launch_bounds__(PK_NT) void k_pack_scan(const uint8_t* __restrict__
 			return;
 		const uint64_t e = o + c[u];
 		voff[i] = o;
-		if (own_tile) {  // V < 2^31
-			for (uint32_t bt = (uint32_t)o / own_tile + 1; bt * own_tile <= (uint32_t)e; ++bt)
+		if constexpr (TILED) {
+			const uint32_t we = w + (uint32_t)(weight(c[u]) >> LB2_SHIFT);
+			for (uint32_t bt = w / own_tile + 1; bt * own_tile <= we; ++bt)
 				tile_seq[bt] = (uint32_t)i + 1u;
 			if (i == 0)
 				tile_seq[0] = 0;
 			if (i == n - 1) {
 				voff[n] = e;
-				tile_seq[((uint32_t)e + own_tile - 1) / own_tile] = (uint32_t)n;
+				tile_seq[(we + own_tile - 1) / own_tile] = (uint32_t)n;
 			}
 			o = e;
+			w = we;
 			continue;
 		}
 		for (uint64_t bt = (o + GEN_TILE - 1) / GEN_TILE; bt * GEN_TILE < e; ++bt)

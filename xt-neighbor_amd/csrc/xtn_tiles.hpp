@@ -28,32 +28,22 @@
 // and 8 in for the sub-range path (k_gen<GEN_COARSE>, k_region_scatter,
 // k_bucket), which stays for distances above 4, for fewer than 4096 records,
 // for searches that ask for the separate pass, and for inputs that outgrow a
-// bound here (a bin, a group of more than TL_GROUP_MAX equal keys, a tile of
-// very short strings): such a run raises coarse_ovf and is redone there.
+// bound here (a bin, a group of more than TL_GROUP_MAX equal keys): such a run
+// raises coarse_ovf and is redone there. No order of the rows outgrows a tile
+// (plan_tiles).
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "xtn_kernels.hpp"
+#include "xtn_plan.hpp"
 
 namespace xtn {
 
-constexpr int TL_NT = 1024;
-constexpr int TL_CAP_BITS = 15;
-constexpr int TL_CAP = 1 << TL_CAP_BITS;  // records of a tile, at most
-constexpr int TL_IT = TL_CAP / TL_NT;     // records of a thread
-constexpr int TL_BINS_MAX = 8192;
 constexpr uint32_t TL_NONE = 0xFFFFFFFFu;  // no record (a tile's last index is never used)
 constexpr int TL_GROUP_MAX = 1024;         // equal keys before a record: a longer group is left to the run kernels
 
-// sequences a tile may hold and the bits of an index in it, by distance: the
-// tables of a tile's sequences share LDS with its records
-__host__ __device__ constexpr int tl_seqs(int d) { return d == 1 ? 4095 : d == 2 ? 768 : d == 3 ? 480 : 127; }
-__host__ __device__ constexpr int tl_idx_bits(int d) { return d == 1 ? 12 : d == 2 ? 10 : d == 3 ? 9 : 7; }
-// bits of a variant's length kept in its record: enough to tell d + 1
-// numbers of deletions apart
-__host__ __device__ constexpr int tl_len_bits(int d) { return d <= 3 ? 2 : 3; }
 constexpr int TL_MAX_D = 4;  // at 5 half of the records are listed and the bins go in parts: 2.4 ms against
                              // 2.0 for 9000 CDR3s on the sub-range path
 constexpr int DEL_SETS4 = DEL_SETS3 + 3060;
@@ -99,7 +89,7 @@ __device__ __forceinline__ uint32_t set_term(uint64_t hw) {  // the query set's 
 struct TileArgs {
 	const uint64_t* pk;
 	const uint64_t* voff;
-	const uint32_t* first;   // first sequence of each tile, [ntiles] = n
+	const uint32_t* first;   // first sequence of each tile, [ntiles] = n (k_pack_scan)
 	uint32_t* out;           // 2^slot_bits slots per tile
 	uint16_t* offs;          // a row of `pitch` per tile: the start of each bin, then the tile's total
 	unsigned long long* ovf;
@@ -232,7 +222,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 	const int cnt = (int)(s1 - s0);
 	const int most = SEQS < (1 << a.lb) - 1 ? SEQS : (1 << a.lb) - 1;
 	if (cnt <= 0 || cnt > most || s1 > a.n) {  // uniform (past n: a packing that gave up left the table undone)
-		tile_refuse(a, row, nb, cnt > 0);
+		tile_refuse(a, row, nb, cnt > 0);  // (the tiling leaves a tile no more than its limit)
 		return;
 	}
 	const uint64_t v0 = a.voff[s0];
@@ -421,22 +411,6 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles1(TileArgs a) {
 	tile_out(s_rec, a.out + (tile << a.slot_bits), total);
 }
 
-// first[b] = the first sequence whose records start at or after b * tile (b <=
-// ntiles; the n sequences hold V > 0 records in all)
-__global__ __launch_bounds__(256) void k_tile_first(const uint64_t* __restrict__ voff, int32_t n, uint32_t tile,
-                                                    uint32_t ntiles, uint32_t* __restrict__ first) {
-	const int i = blockIdx.x * 256 + threadIdx.x;
-	if (i >= n)
-		return;
-	const uint32_t o = (uint32_t)voff[i], e = (uint32_t)voff[i + 1];
-	for (uint32_t b = o / tile + 1; b * tile <= e; ++b)
-		first[b] = (uint32_t)i + 1u;
-	if (i == 0)
-		first[0] = 0;
-	if (i == n - 1)
-		first[ntiles] = (uint32_t)n;
-}
-
 // The tiles' rows of bin starts to one row per bin, [nb + 1][cpitch], in
 // blocks of 64 x 64; columns past the last tile read as 0. n_rec: the
 // records of all tiles (the last bin row holds the tiles' totals).
@@ -472,12 +446,6 @@ __global__ __launch_bounds__(256) void k_tile_cols(const uint16_t* __restrict__ 
 }
 
 // ------------------------------------------------------------- pairs --
-
-// threads of a bin's workgroup, two workgroups per CU (one's loads and
-// barriers under the other's work: 430 us against 476 at 1M CDR3s, d = 2, for
-// one of 1024 threads over half as many bins); the wide form takes the records
-// that the narrow one would need too many bins for
-constexpr int BIN_NT = 512, BIN_WIDE_NT = 1024;
 
 struct BinArgs {
 	const uint32_t* rec;     // the tiles
