@@ -136,10 +136,11 @@ typedef struct {
 	int64_t coarse_in_generator; /* 1: the generator ordered the records itself, into
 	                                tiles ordered by bin or by their top 8 hash
 	                                bits; 0: a separate pass did (always after
-	                                the generator's order outgrew a bound on
-	                                this handle, until new sequences), or the
-	                                tiles held more equal pairs than records
-	                                (many copies of some strings) */
+	                                a sub-range of the generator's pass
+	                                overflowed on this handle, until new
+	                                sequences), or the tiles held more equal
+	                                pairs than records (many copies of some
+	                                strings) */
 	int64_t n_records;     /* deletion records written: n_variants less the
 	                          repeated variants of a sequence (deleting any
 	                          residue of a run of equal ones gives the same

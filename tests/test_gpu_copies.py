@@ -1,5 +1,8 @@
 """Rows that come several times, on the GPU: the records stay in tiles, with
-the oracle's output, also where equal pairs outnumber the records."""
+the oracle's output, also where equal pairs outnumber the records; one string
+of more copies than a bin's lists follow goes through the generator's coarse
+pass, which writes no record for a repeated variant, and not through the
+separate pass."""
 import os
 
 import numpy as np
@@ -39,3 +42,15 @@ def test_copies_stay_in_tiles(n, copies, d, measure):
     with xtn.Engine(distance=d, measure=measure, profile=True) as eng:
         eng.set_sequences(chars=chars, offsets=offsets)
         assert searched(eng, want) == dict(tiles=1, bins=1, gen=0, gen_coarse=0)
+
+
+@pytest.mark.parametrize("n,d,measure", [(9_000, 2, 0), (60_000, 1, 1), (2_000, 3, 0)])
+def test_outgrown_tiles_go_to_the_coarse_pass(n, d, measure):
+    # one string 1100 times, spread over the rows
+    seqs = xtn.decode(*xtn.synth_nn(410 + d, n, planted=0.3, max_edits=1)) + ["CASSLGTDTQYF"] * 1100
+    chars, offsets = xtn.encode([seqs[i] for i in np.random.default_rng(d).permutation(len(seqs))])
+    want = oracle.nn_port_mt(chars, offsets, d, measure, THREADS)[0].astype(np.int64)
+    with xtn.Engine(distance=d, measure=measure, profile=True) as eng:
+        eng.set_sequences(chars=chars, offsets=offsets)
+        assert searched(eng, want) == dict(tiles=0, bins=0, gen=0, gen_coarse=1)
+        assert d == 1 or eng.stats()["n_records"] < eng.stats()["n_variants"]

@@ -129,6 +129,7 @@ struct xtn_handle {
 	bool groups_off = false;    // a group of ids got more candidates than fit: the tail's passes until new
 	                            // sequences
 	bool bin_parts = false;     // a bin listed more records than fit: bins in parts until new sequences
+	bool tiles_off = false;     // the tiles or bins outgrew a bound: the other layouts until new sequences
 	bool coarse_off = false;    // a sub-range of the generator's coarse pass overflowed: the separate
 	                            // pass until new sequences
 	double tune_ms = 0, tune_ms_default = 0;
@@ -1303,7 +1304,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	auto tiles_wanted = [&]() {
 		return d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && (int64_t)V < (int64_t)INT32_MAX &&
 		       (h->no_alloc ? (int64_t)V <= h->cfg.max_records_per_chunk : h->cfg.max_records_per_chunk <= 0) && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
-		       !h->coarse_off && !h->tail_safe &&
+		       !h->tiles_off && !h->tail_safe &&
 		       ((int64_t)V <= bucket_records || h->tune_target >= DEFAULT_BUCKET_TARGET);
 	};
 	// chunk plan: the records of one chunk (plus the sort buffer and the
@@ -1867,11 +1868,12 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			// point accepts: there the other layout counts them all.
 			many_pairs = tiled && head.rc.pairs_small > V;
 			if (head.rc.coarse_ovf || (many_pairs && h->no_alloc)) {
-				// a sub-range of the generator's coarse pass overflowed and lost
-				// records, or the tiles and bins outgrew a bound: the run again
-				// with the separate pass, which these sequences keep from now on
-				h->coarse_off = true;
-				if ((int64_t)V > sorted_budget)  // the chunks of the separate pass
+				// the tiles or bins outgrew a bound (the other layouts from now on,
+				// the generator's coarse pass among them), or a sub-range of that
+				// pass overflowed and lost records (the separate pass from now on):
+				// the run again
+				(tiled ? h->tiles_off : h->coarse_off) = true;
+				if (tiled && (int64_t)V > sorted_budget)  // the chunks of the other layouts
 					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
 				grouped = false;
 				prologue_done = false;
@@ -2454,6 +2456,7 @@ int xtn_set_sequences(xtn_handle* h, const char* chars, const uint32_t* offsets,
 	h->prefix_len.swap(plen);
 	h->len_cum.clear();
 	h->tail_full = false;
+	h->tiles_off = false;
 	h->coarse_off = false;
 	h->bin_parts = false;
 	h->groups_off = false;
