@@ -114,7 +114,9 @@ typedef struct {
 	                          multiplicity; the copies a sequence's repeated
 	                          variants would add are not there when the
 	                          generator left those out, nor, in tiles, those
-	                          of a pair within one edit beyond its first) */
+	                          of a pair within one edit beyond its first,
+	                          unless a run's equal pairs of records outnumber
+	                          the records: then all of these) */
 	int64_t n_unique;      /* unique candidate pairs verified (U) */
 	int64_t n_output;      /* pairs (NN) or repertoire entries (overlap) out */
 	double ms_total;       /* device pipeline wall time */

@@ -1732,11 +1732,11 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	// rounds over the smaller id of a pair, processed in ascending order
 	std::deque<std::pair<uint32_t, uint32_t>> rounds;
 	rounds.emplace_back(0u, (uint32_t)nseq);
-	int64_t out_total = 0, max_round = 0;
+	int64_t out_total = 0, max_round = 0, n_candidates = 0;
 	Grouping g1;
 	bool grouped = false;  // single chunk: the grouping is done once for every round
 	int64_t n_written = 0;  // records the generator wrote, counted once for every round
-	bool many_pairs = false;  // tiles that met more equal pairs than records
+	int64_t many_pairs = 0;  // equal pairs of tiles that met more of them than records
 	bool no_graph = false;  // a replay needed the host: the rest of this run is eager
 	TailPlan tp;
 	CtlHead head{};
@@ -1866,7 +1866,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			// generator's coarse pass and 44.2 through the separate pass. Not in the
 			// static scratch, whose room for candidates is part of what its entry
 			// point accepts: there the other layout counts them all.
-			many_pairs = tiled && head.rc.pairs_small > V;
+			many_pairs = tiled && head.rc.pairs_small > V ? (int64_t)head.rc.pairs_small : 0;
 			if (head.rc.coarse_ovf || (many_pairs && h->no_alloc)) {
 				// the tiles or bins outgrew a bound (the other layouts from now on,
 				// the generator's coarse pass among them), or a sub-range of that
@@ -1990,7 +1990,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				continue;
 			}
 		}
-		st.n_candidates += n_pairs;
+		n_candidates += n_pairs;
 		st.n_unique += (int64_t)head.n_unique;
 		out_total += (int64_t)head.n_out;
 		max_round = std::max(max_round, n_pairs);
@@ -2010,6 +2010,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	} else if (used_coarse) {
 		st.n_records = n_written;
 	}
+	st.n_candidates += many_pairs ? many_pairs : n_candidates;
 	h->last_pairs = max_round;
 	h->last_unique = st.n_unique;
 	h->last_out = out_total;
