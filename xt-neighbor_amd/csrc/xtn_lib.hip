@@ -1862,7 +1862,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			n_written = std::max<int64_t>(n_written, (int64_t)head.rc.n_records);
 			// More equal pairs than records (many copies of some strings) stay
 			// in the bins, which leave out most of them before the tail: 3
-			// copies of 100 000 CDR3s, d = 2, 7.9 ms against 30.8 through the
+			// copies of 100 000 CDR3s, d = 2, 2.2 ms against 30.8 through the
 			// generator's coarse pass and 44.2 through the separate pass. Not in the
 			// static scratch, whose room for candidates is part of what its entry
 			// point accepts: there the other layout counts them all.
@@ -1880,12 +1880,15 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				continue;
 			}
 			if (tiled && head.rc.n_big) {
-				// bins listed more records than fit: the run again with the bins
-				// in parts, which these sequences keep from now on
+				// bins listed more records than fit, or met a long group: the
+				// bins again, in parts, which these sequences keep from now on
+				// (the tiles are in place; only a replay left no plan of them)
 				h->bin_parts = true;
 				no_graph = no_graph || via_graph;
-				grouped = false;
-				prologue_done = false;
+				if (via_graph) {
+					grouped = false;
+					prologue_done = false;
+				}
 				continue;
 			}
 			if (!head.error && (int64_t)head.rc.n_cand <= pcap && head.rc.append == 0 &&

@@ -42,7 +42,13 @@
 namespace xtn {
 
 constexpr uint32_t TL_NONE = 0xFFFFFFFFu;  // no record (a tile's last index is never used)
-constexpr int TL_GROUP_MAX = 1024;         // equal keys before a record: a longer group is left to the run kernels
+// equal keys before a record: a longer group is left to the run kernels, which
+// spread its pairs over the chip (one string 1100 times among 300 000 rows, d =
+// 1: 10.8 ms there)
+constexpr int TL_GROUP_MAX = 1024;
+// the same for the 18-group form without rounds: a longer group costs its
+// workgroup 16 us or more (8 ns a pair), and the form with parts takes it
+constexpr int TL_GROUP_LONG = 64;
 
 constexpr int TL_MAX_D = 4;  // at 5 half of the records are listed and the bins go in parts: 2.4 ms against
                              // 2.0 for 9000 CDR3s on the sub-range path
@@ -488,10 +494,8 @@ __device__ __forceinline__ uint32_t residue_set(uint64_t lo, uint32_t hi26) {
 // for every further deletion as well (about a dozen at distance 2, a hundred
 // at 3): the pair goes out only from the variant with the fewest deletions, which
 // both sides hold and whose length is known from the two strings.
-__device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint32_t ia, uint32_t ib, uint32_t len,
-                                          int len_bits, int distance) {
-	const uint64_t la = pk[2 * (int64_t)ia], wa = pk[2 * (int64_t)ia + 1];
-	const uint64_t lb = pk[2 * (int64_t)ib], wb = pk[2 * (int64_t)ib + 1];
+__device__ __forceinline__ bool tile_pair(uint64_t la, uint64_t wa, uint64_t lb, uint64_t wb, uint32_t len,
+                                          int len_bits, int distance) {  // (the two packed prefixes)
 	const uint32_t ha = (uint32_t)wa & PK_SLOT_HI_MASK, hb = (uint32_t)wb & PK_SLOT_HI_MASK;
 	const int La = (int)(wa >> 56), Lb = (int)(wb >> 56);
 	const int lm = (1 << len_bits) - 1;
@@ -528,7 +532,14 @@ __device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint3
 	return front + back < m || (La > Lb ? ma : mb) == 1;
 }
 
+__device__ __forceinline__ bool tile_pair(const uint64_t* __restrict__ pk, uint32_t ia, uint32_t ib, uint32_t len,
+                                          int len_bits, int distance) {
+	return tile_pair(pk[2 * (int64_t)ia], pk[2 * (int64_t)ia + 1], pk[2 * (int64_t)ib], pk[2 * (int64_t)ib + 1], len,
+	                 len_bits, distance);
+}
+
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 
 // Bins over resident workgroups. NT threads hold QPT groups of four records
 // each.
@@ -543,9 +554,9 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 //      of two sequences are candidate pairs (tile_pair)
 // PARTS: a bin that lists more than SVC records (an input with many
 // duplicates or neighbours) goes through the steps once per part of its
-// records by their top key bits; without it such a bin raises bins_ovf
-// (n_big) and the host runs the instantiation that has it, which the common
-// case would pay for in registers (8% of the kernel).
+// records by their top key bits; without it such a bin raises n_big and the
+// host runs the instantiation that has it, which the common case would pay for
+// in registers (8% of the kernel).
 // QPT 18: bins of up to 36864 slots, an eighth of whose records may be
 // listed; QPT 9 (distances 3 and 4, where a neighbouring pair shares hundreds
 // of variants): half as many slots and a list for half of their records.
@@ -558,6 +569,7 @@ template <int NT, int QPT, bool PARTS>
 __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 	constexpr int X = NT / BIN_NT;  // the wide form: everything twice, one workgroup per CU
 	constexpr bool FEW = QPT == 3;
+	constexpr bool ROUNDS = PARTS || FEW;
 	constexpr int B1 = FEW ? 16 : 17 + X, B2 = B1 - 2, HBITS = (QPT == 18 ? 11 : 10) + X;
 	static_assert((X == 1 || X == 2) && (QPT == 18 || QPT == 9 || FEW), "bitmaps of 7 bits or more and a quarter of that per record");
 	static_assert(!FEW || !PARTS, "every record fits the list");
@@ -585,6 +597,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 	__shared__ uint32_t s_tmp[NT / WAVE + 1];
 	__shared__ unsigned long long s_base;
 	__shared__ uint32_t s_nsv, s_npl;
+	__shared__ int s_stop;
 	static_assert(sizeof(u1) + sizeof(u2) + sizeof(s_bm2) <= 79 * 1024 * X, "two workgroups per CU");
 	const int t = threadIdx.x;
 	const int lane = lane_id();
@@ -609,6 +622,8 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		}
 		if (t == 0)
 			s_nsv = s_npl = 0;
+		if (ROUNDS && t == 0)
+			s_stop = 0;
 		// 1. eight tiles per thread and round
 		constexpr int TR = FEW ? 1 : 8;
 		uint32_t nq = 0;
@@ -776,62 +791,179 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		for (uint32_t i = t; i < nsv; i += NT)
 			u2.g.next[i] = (uint16_t)atomicExch(&u2.g.head[(u1.sv.rec[i] >> a.key_low) & (HEADS - 1)], i);
 		__syncthreads();
-		auto candidate = [&](uint32_t i, uint32_t n, uint64_t* p) -> bool {
-			const uint32_t ri = u1.sv.rec[i], rn = u1.sv.rec[n];
-			const uint32_t x = a.first[u1.sv.tile[i]] + (ri & lmask), y = a.first[u1.sv.tile[n]] + (rn & lmask);
-			if (x == y)
-				return false;
-			const uint32_t lo = x < y ? x : y, hi = x < y ? y : x;
-			if (lo < a.id_lo || lo >= a.id_hi)
-				return false;
-			*p = ((uint64_t)lo << a.idb) | hi;
-			return tile_pair(a.pk, lo, hi, (ri >> a.lb) & ((1u << a.len_bits) - 1u), a.len_bits,
-			                 a.distance);
-		};
-		for (uint32_t i = t; i < nsv; i += NT) {
-			const uint32_t r = u1.sv.rec[i];
-			uint32_t same = 0;
-			for (uint32_t n = u2.g.next[i]; n != 0xFFFFu;) {
-				const uint32_t rn = u1.sv.rec[n];  // record and link read together
-				const uint32_t nn = u2.g.next[n];
-				const uint32_t m = n;
-				n = nn;
-				if ((r ^ rn) >> a.lb)
-					continue;
-				const uint32_t q = atomicAdd(&s_npl, 1u);
-				if (q < (uint32_t)PLC) {
-					u2.g.pl[q] = (i << 16) | m;
-				} else {
-					uint64_t p;
-					if (candidate(i, m, &p)) {
-						const unsigned long long slot = atomicAdd(&a.ctr->n_cand, 1ull);
-						if ((int64_t)slot < a.pcap)
-							a.pairs[slot] = p;
+		// Every record walks its list; the pairs that it finds go to a list in
+		// LDS, which all threads evaluate. Where that list is full,
+		//   - ROUNDS: a thread takes its walk up again after the pairs listed so
+		//     far, so that the many pairs of a long group are not left to the
+		//     threads that meet them, one dependent load after the other;
+		//   - else it evaluates the pair itself, as long as no group is longer
+		//     than TL_GROUP_LONG (with rounds the kernel holds more registers than
+		//     the gather leaves: 447 us against 430 at 1M CDR3s, d = 2).
+		// Resident searches with rounds against without: 10 copies of each of
+		// 30 000 rows, d = 2, 7.5 ms against 40; 3 copies of 100 000 2.1 against
+		// 7.9; one string 300 times among 300 000 rows, d = 1, 1.2 against 1.7.
+		if constexpr (ROUNDS) {
+			int u = t;  // kept from the compiler, which would hold what it makes of it in registers that the gather needs
+			asm volatile("" : "+v"(u));
+			constexpr int EV = PARTS && QPT == 18 ? 5 : 2;
+			uint32_t i = u, n = 0xFFFFu, same = 0;
+			bool mid = false;  // the walk of record i stands at link n
+			bool checked = false;
+			for (;;) {
+				for (; i < nsv; i += NT) {
+					const uint32_t r = u1.sv.rec[i];
+					if (!mid) {
+						n = u2.g.next[i];
+						same = 0;
+					}
+					mid = false;
+					while (n != 0xFFFFu) {
+						const uint32_t rn = u1.sv.rec[n];  // record and link read together
+						const uint32_t nn = u2.g.next[n];
+						const uint32_t m = n;
+						n = nn;
+						if ((r ^ rn) >> a.lb)
+							continue;
+						const uint32_t q = atomicAdd(&s_npl, 1u);
+						if (q >= (uint32_t)PLC) {
+							n = m;
+							mid = true;
+							break;
+						}
+						u2.g.pl[q] = (i << 16) | m;
+						if (++same >= (uint32_t)TL_GROUP_MAX) {
+							atomicOr(&a.ctr->coarse_ovf, 1ull);
+							break;
+						}
+					}
+					if (mid)
+						break;
+				}
+				__syncthreads();
+				const uint32_t listed = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_npl);
+				const uint32_t npl = listed < (uint32_t)PLC ? listed : (uint32_t)PLC;
+				if (u == 0)
+					atomicAdd(&a.ctr->pairs_small, (unsigned long long)npl);
+				for (uint32_t q0 = 0; q0 < npl; q0 += EV * NT) {  // uniform
+					uint32_t lo[EV], hi[EV], ok = 0;
+					u64x2 pl[EV], ph[EV];
+					uint32_t len[EV];
+#pragma unroll
+					for (int k = 0; k < EV; ++k)
+						if (q0 + k * NT + u < npl) {
+							const uint32_t w = u2.g.pl[q0 + k * NT + u];
+							const uint32_t rx = u1.sv.rec[w >> 16], ry = u1.sv.rec[w & 0xFFFFu];
+							const uint32_t x = a.first[u1.sv.tile[w >> 16]] + (rx & lmask);
+							const uint32_t y = a.first[u1.sv.tile[w & 0xFFFFu]] + (ry & lmask);
+							lo[k] = x < y ? x : y;
+							hi[k] = x < y ? y : x;
+							len[k] = (rx >> a.lb) & ((1u << a.len_bits) - 1u);
+							if (x != y && lo[k] >= a.id_lo && lo[k] < a.id_hi) {
+								ok |= 1u << k;
+								pl[k] = reinterpret_cast<const u64x2*>(a.pk)[lo[k]];
+								ph[k] = reinterpret_cast<const u64x2*>(a.pk)[hi[k]];
+							}
+						}
+#pragma unroll
+					for (int k = 0; k < EV; ++k)
+						if (((ok >> k) & 1u) &&
+						    !tile_pair(pl[k].x, pl[k].y, ph[k].x, ph[k].y, len[k], a.len_bits, a.distance))
+							ok &= ~(1u << k);
+					unsigned long long slot = block_append<NT>(&a.ctr->n_cand, (uint32_t)__popc(ok), s_tmp, &s_base);
+#pragma unroll
+					for (int k = 0; k < EV; ++k)
+						if ((ok >> k) & 1u) {
+							if ((int64_t)slot < a.pcap)
+								a.pairs[slot] = ((uint64_t)lo[k] << a.idb) | hi[k];
+							++slot;
+						}
+				}
+				if (listed <= (uint32_t)PLC) {  // every walk is at its end
+					__syncthreads();
+					break;
+				}
+				if (!checked) {  // once: a group too long for the rounds is found before they are spent on it
+					checked = true;
+					for (uint32_t j = u; j < nsv; j += NT) {
+						const uint32_t r = u1.sv.rec[j];
+						int equal = 0;
+						for (uint32_t m = u2.g.next[j]; m != 0xFFFFu; m = u2.g.next[m])
+							equal += (r ^ u1.sv.rec[m]) >> a.lb == 0u;
+						if (equal >= TL_GROUP_MAX) {
+							atomicOr(&a.ctr->coarse_ovf, 1ull);
+							s_stop = 1;
+						}
 					}
 				}
-				if (++same >= (uint32_t)TL_GROUP_MAX) {
-					atomicOr(&a.ctr->coarse_ovf, 1ull);
+				if (u == 0) {  // (s_npl read by all before the append's barriers)
+					s_npl = 0;
+					if (__hip_atomic_load(&a.ctr->coarse_ovf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+						s_stop = 1;  // another bin gave the run up
+				}
+				__syncthreads();
+				if (__builtin_amdgcn_readfirstlane(s_stop)) {  // the run is redone elsewhere
+					__syncthreads();
 					break;
 				}
 			}
-		}
-		__syncthreads();
-		uint32_t npl = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_npl);
-		if (t == 0)
-			atomicAdd(&a.ctr->pairs_small, (unsigned long long)npl);
-		npl = npl < (uint32_t)PLC ? npl : (uint32_t)PLC;
-		for (uint32_t q0 = 0; q0 < npl; q0 += NT) {  // uniform
-			bool ok = false;
-			uint64_t p = 0;
-			if (q0 + t < npl) {
-				const uint32_t w = u2.g.pl[q0 + t];
-				ok = candidate(w >> 16, w & 0xFFFFu, &p);
+		} else {
+			auto candidate = [&](uint32_t i, uint32_t n, uint64_t* p) -> bool {
+				const uint32_t ri = u1.sv.rec[i], rn = u1.sv.rec[n];
+				const uint32_t x = a.first[u1.sv.tile[i]] + (ri & lmask), y = a.first[u1.sv.tile[n]] + (rn & lmask);
+				if (x == y)
+					return false;
+				const uint32_t lo = x < y ? x : y, hi = x < y ? y : x;
+				if (lo < a.id_lo || lo >= a.id_hi)
+					return false;
+				*p = ((uint64_t)lo << a.idb) | hi;
+				return tile_pair(a.pk, lo, hi, (ri >> a.lb) & ((1u << a.len_bits) - 1u), a.len_bits,
+				                 a.distance);
+			};
+			for (uint32_t i = t; i < nsv; i += NT) {
+				const uint32_t r = u1.sv.rec[i];
+				uint32_t same = 0;
+				for (uint32_t n = u2.g.next[i]; n != 0xFFFFu;) {
+					const uint32_t rn = u1.sv.rec[n];  // record and link read together
+					const uint32_t nn = u2.g.next[n];
+					const uint32_t m = n;
+					n = nn;
+					if ((r ^ rn) >> a.lb)
+						continue;
+					const uint32_t q = atomicAdd(&s_npl, 1u);
+					if (q < (uint32_t)PLC) {
+						u2.g.pl[q] = (i << 16) | m;
+					} else {
+						uint64_t p;
+						if (candidate(i, m, &p)) {
+							const unsigned long long slot = atomicAdd(&a.ctr->n_cand, 1ull);
+							if ((int64_t)slot < a.pcap)
+								a.pairs[slot] = p;
+						}
+					}
+					if (++same >= (uint32_t)(QPT == 18 ? TL_GROUP_LONG : TL_GROUP_MAX)) {
+						atomicOr(QPT == 18 ? &a.ctr->n_big : &a.ctr->coarse_ovf, 1ull);
+						break;
+					}
+				}
 			}
-			const unsigned long long slot = block_append<NT>(&a.ctr->n_cand, ok ? 1u : 0u, s_tmp, &s_base);
-			if (ok && (int64_t)slot < a.pcap)
-				a.pairs[slot] = p;
+			__syncthreads();
+			uint32_t npl = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_npl);
+			if (t == 0)
+				atomicAdd(&a.ctr->pairs_small, (unsigned long long)npl);
+			npl = npl < (uint32_t)PLC ? npl : (uint32_t)PLC;
+			for (uint32_t q0 = 0; q0 < npl; q0 += NT) {  // uniform
+				bool ok = false;
+				uint64_t p = 0;
+				if (q0 + t < npl) {
+					const uint32_t w = u2.g.pl[q0 + t];
+					ok = candidate(w >> 16, w & 0xFFFFu, &p);
+				}
+				const unsigned long long slot = block_append<NT>(&a.ctr->n_cand, ok ? 1u : 0u, s_tmp, &s_base);
+				if (ok && (int64_t)slot < a.pcap)
+					a.pairs[slot] = p;
+			}
+			__syncthreads();
 		}
-		__syncthreads();
 		fresh = false;
 		if (!PARTS || ++part == 1 << lp) {
 			part = 0;
