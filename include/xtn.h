@@ -139,8 +139,8 @@ typedef struct {
 	                                tiles ordered by bin or by their top 8 hash
 	                                bits; 0: a separate pass did (always after
 	                                a sub-range of the generator's pass
-	                                overflowed on this handle, until new
-	                                sequences), or the tiles held more equal
+	                                overflowed for these rows at this
+	                                distance, until new sequences), or the tiles held more equal
 	                                pairs than records (many copies of some
 	                                strings) */
 	int64_t n_records;     /* deletion records written: n_variants less the

@@ -31,6 +31,7 @@
 #include <initializer_list>
 #include <map>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/xtn.h"
@@ -126,12 +127,23 @@ struct xtn_handle {
 	int tune_low = 0;           // pair bits left unsorted for the select's in-group ranking: 0, 8, 16, 24
 	int tune_coarse_sep = 0;    // 1: the records' first ordering pass as a pass of its own (tuned)
 	bool tail_full = false;     // a group outgrew the select's window: full sorts until new sequences
-	bool groups_off = false;    // a group of ids got more candidates than fit: the tail's passes until new
-	                            // sequences
-	bool bin_parts = false;     // a bin listed more records than fit: bins in parts until new sequences
-	bool tiles_off = false;     // the tiles or bins outgrew a bound: the other layouts until new sequences
-	bool coarse_off = false;    // a sub-range of the generator's coarse pass overflowed: the separate
-	                            // pass until new sequences
+	// what the searches of some rows met, by distance, rows and query sets
+	// (nn_pipeline): until new sequences
+	struct RowsKey {
+		int64_t rows, nseq, sets;  // rows: the first, -1 for rows of a map
+		int32_t d;
+		bool operator<(const RowsKey& o) const {
+			return std::tie(d, rows, nseq, sets) < std::tie(o.d, o.rows, o.nseq, o.sets);
+		}
+	};
+	struct RowsMet {
+		bool groups_off = false;  // a group of ids got more candidates than fit: the tail's passes
+		bool bin_parts = false;   // a bin listed more records than fit, or met a long group: bins in parts
+		bool tiles_off = false;   // the tiles or bins outgrew a bound: the other layouts
+		bool coarse_off = false;  // a sub-range of the generator's coarse pass overflowed: the separate pass
+	};
+	std::map<RowsKey, RowsMet> met;
+	int64_t sets_id = 0;  // of the query sets being searched together
 	double tune_ms = 0, tune_ms_default = 0;
 	bool capturing = false;
 	bool no_alloc = false;  // xtn_nn_noalloc: every buffer is a slice of the static scratch
@@ -959,6 +971,7 @@ struct Grouping {
 	int64_t rtiles = 0;
 	BucketArgs ba{};
 	bool tiles = false;  // tiles ordered by bin (xtn_tiles.hpp) instead of any of the above
+	bool parts = false;  // bins in parts
 	TileArgs ta{};
 	BinArgs bn{};
 };
@@ -1139,7 +1152,7 @@ int issue_buckets(xtn_handle* h, Grouping& g, uint32_t lo, uint32_t hi, int64_t 
 		    {{k_bins<BIN_WIDE_NT, 18, false>, k_bins<BIN_WIDE_NT, 18, true>},
 		     {k_bins<BIN_WIDE_NT, 9, false>, k_bins<BIN_WIDE_NT, 9, true>}}};
 		const BinFn fn = bn.groups == 3 ? k_bins<BIN_NT, 3, false>
-		                                : fns[bn.nt == BIN_WIDE_NT][bn.groups == 9][h->bin_parts];
+		                                : fns[bn.nt == BIN_WIDE_NT][bn.groups == 9][g.parts];
 		fn<<<grid, bn.nt, 0, h->stream>>>(bn);
 		HIP_LAUNCH_CHECK(h);
 		return XTN_OK;
@@ -1250,6 +1263,15 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	const double t0 = now_ms();
 	h->out_len = 0;
 	st.n_sequences = nseq;
+	const xtn_handle::RowsKey rows_key{seq_map ? -1 : (int64_t)row_base, nseq, set_of ? h->sets_id : 0, d};
+	xtn_handle::RowsMet met;
+	if (auto it = h->met.find(rows_key); it != h->met.end())
+		met = it->second;
+	auto keep_met = [&]() {
+		if (h->met.size() >= 4096)
+			h->met.clear();
+		h->met[rows_key] = met;
+	};
 	if (nseq < 2) {
 		HIP_SYNC(h, s);
 		st.ms_total = now_ms() - t0;
@@ -1304,7 +1326,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	auto tiles_wanted = [&]() {
 		return d <= TL_MAX_D && (int64_t)V >= TILES_MIN_RECORDS && (int64_t)V < (int64_t)INT32_MAX &&
 		       (h->no_alloc ? (int64_t)V <= h->cfg.max_records_per_chunk : h->cfg.max_records_per_chunk <= 0) && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 &&
-		       !h->tiles_off && !h->tail_safe &&
+		       !met.tiles_off && !h->tail_safe &&
 		       ((int64_t)V <= bucket_records || h->tune_target >= DEFAULT_BUCKET_TARGET);
 	};
 	// chunk plan: the records of one chunk (plus the sort buffer and the
@@ -1413,7 +1435,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	bool gen_seg = false;
 	std::vector<int64_t> part_t0(nparts + 1, 0);
 	int64_t seg_sub_cap = 0;
-	if (gen_once && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 && !h->coarse_off) {
+	if (gen_once && h->cfg.coarse_separate == 0 && h->tune_coarse_sep == 0 && !met.coarse_off) {
 		TRY(prologue());
 		const int nseg = RS_BINS << COARSE_SUB_BITS;
 		const double mean = (double)V / nseg;
@@ -1446,7 +1468,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		RunCtrs rc{};
 		TRY(read_ctrs(h, &rc));
 		if (rc.coarse_ovf) {
-			h->coarse_off = true;  // a sub-range overflowed: the separate pass below
+			met.coarse_off = true;  // a sub-range overflowed: the separate pass below
+			keep_met();
 		} else {
 			gen_seg = true;
 			const int per = RS_BINS >> pbits;  // top-8-bit digits per part
@@ -1538,6 +1561,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		g.nseq = nseq;
 		if (use_tiles()) {
 			g.tiles = true;
+			g.parts = met.bin_parts;
 			const int64_t cpitch = tplan.cpitch();
 			const int nbins = 1 << tplan.bin_bits, pitch = tplan.pitch();
 			TRY(ensure(h, h->tile_rec, tplan.rec_bytes()));
@@ -1610,7 +1634,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 		// sub_cap slots (the mean with 10 % and eight standard deviations of
 		// headroom; a sub-range that still overflows sends the run back to the
 		// separate pass)
-		g.coarse = g.region && nparts == 1 && !h->coarse_off && !h->tail_safe && h->cfg.coarse_separate == 0 &&
+		g.coarse = g.region && nparts == 1 && !met.coarse_off && !h->tail_safe && h->cfg.coarse_separate == 0 &&
 		           h->tune_coarse_sep == 0;
 		if (g.coarse) {
 			g.nseg = RS_BINS << COARSE_SUB_BITS;
@@ -1760,7 +1784,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			                                            : V <= SMALL_TAIL_RECORDS);
 			// (from distance 4 on one id alone brings thousands of candidates,
 			// which no group holds, once there are some hundred thousand)
-			int groups = !small && h->tune_low == 0 && !h->no_alloc && !h->groups_off && (d < 4 || pcap <= TG_FINE / 2)
+			int groups = !small && h->tune_low == 0 && !h->no_alloc && !met.groups_off && (d < 4 || pcap <= TG_FINE / 2)
 			                 ? (int)tail_groups_max(pcap)
 			                 : 0;
 			if (groups > TG_MAX)
@@ -1808,8 +1832,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				sig.sort_tile = h->tune_sort_tile;
 				sig.select_nt = h->tune_select_nt;
 				sig.low = h->tail_full ? 0 : h->tune_low;
-				sig.coarse = h->coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
-				sig.pad = (h->bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0) | (groups ? 8 : 0);
+				sig.coarse = met.coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
+				sig.pad = (met.bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0) | (groups ? 8 : 0);
 			}
 			const bool tiled = use_tiles();  // also of a replay, which plans nothing
 			bool via_graph = false;
@@ -1872,7 +1896,8 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				// the generator's coarse pass among them), or a sub-range of that
 				// pass overflowed and lost records (the separate pass from now on):
 				// the run again
-				(tiled ? h->tiles_off : h->coarse_off) = true;
+				(tiled ? met.tiles_off : met.coarse_off) = true;
+				keep_met();
 				if (tiled && (int64_t)V > sorted_budget)  // the chunks of the other layouts
 					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
 				grouped = false;
@@ -1881,9 +1906,11 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			}
 			if (tiled && head.rc.n_big) {
 				// bins listed more records than fit, or met a long group: the
-				// bins again, in parts, which these sequences keep from now on
+				// bins again, in parts, as for these rows from now on
 				// (the tiles are in place; only a replay left no plan of them)
-				h->bin_parts = true;
+				met.bin_parts = true;
+				keep_met();
+				g1.parts = true;
 				no_graph = no_graph || via_graph;
 				if (via_graph) {
 					grouped = false;
@@ -1894,9 +1921,12 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			if (!head.error && (int64_t)head.rc.n_cand <= pcap && head.rc.append == 0 &&
 			    ((small && (int64_t)head.rc.n_cand > TS_CAP) || (groups && head.overflow))) {
 				// too many for the one workgroup (a later run goes by their count)
-				// or for one of the groups (the passes until new sequences): the
+				// or for one of the groups (the passes from now on): the
 				// passes over the candidates as they lie
-				h->groups_off = h->groups_off || groups > 0;
+				if (groups > 0) {
+					met.groups_off = true;
+					keep_met();
+				}
 				TRY(zero_ctl(h, false, true));
 				TRY(tail_prepare(h, pcap, idb, out_total, &tp));
 				TRY(issue_tail(h, tp, idb, seq_map, row_base, set_of, out_total));
@@ -2460,10 +2490,7 @@ int xtn_set_sequences(xtn_handle* h, const char* chars, const uint32_t* offsets,
 	h->prefix_len.swap(plen);
 	h->len_cum.clear();
 	h->tail_full = false;
-	h->tiles_off = false;
-	h->coarse_off = false;
-	h->bin_parts = false;
-	h->groups_off = false;
+	h->met.clear();
 	return XTN_OK;
 }
 
@@ -2639,6 +2666,10 @@ int xtn_perform_sets(xtn_handle* h, const uint32_t* set_offsets, int32_t n_sets,
 			                                                       r1 - r0, h->set_of.as<uint32_t>());
 			HIP_LAUNCH_CHECK(h);
 		}
+		uint64_t id = 1469598103934665603ull;  // FNV-1a
+		for (int32_t k = 0; k <= n_sets; ++k)
+			id = (id ^ set_offsets[k]) * 1099511628211ull;
+		h->sets_id = (int64_t)id;
 		TRY(nn_pipeline(h, (int32_t)(r1 - r0), nullptr, r0, h->set_of.as<uint32_t>()));
 		// the query set holding a row, as k_set_of finds it
 		auto set_of = [&](uint32_t row) -> uint32_t {
