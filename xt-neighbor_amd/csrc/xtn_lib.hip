@@ -139,6 +139,7 @@ struct xtn_handle {
 	struct RowsMet {
 		bool groups_off = false;  // a group of ids got more candidates than fit: the tail's passes
 		bool bin_parts = false;   // a bin listed more records than fit, or met a long group: bins in parts
+		int tight = 0;            // times a bin outgrew its slots (plan_tiles)
 		bool tiles_off = false;   // the tiles or bins outgrew a bound: the other layouts
 		bool coarse_off = false;  // a sub-range of the generator's coarse pass overflowed: the separate pass
 	};
@@ -1345,9 +1346,13 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 	}
 	budget = std::max<int64_t>(budget, 1 << 16);
 	const int64_t sorted_budget = budget;  // a chunk of the other layouts
-	TilePlan tplan = tiles_wanted() ? plan_tiles(lens, nseq, d, h->n_cu) : TilePlan{};
-	if ((double)tplan.rec_bytes() + (double)tplan.offs_bytes() + (double)tplan.cols_bytes() > (double)free_b * 0.6)
-		tplan = TilePlan{};
+	TilePlan tplan;
+	auto make_tplan = [&]() {
+		tplan = tiles_wanted() ? plan_tiles(lens, nseq, d, h->n_cu, met.tight) : TilePlan{};
+		if ((double)tplan.rec_bytes() + (double)tplan.offs_bytes() + (double)tplan.cols_bytes() > (double)free_b * 0.6)
+			tplan = TilePlan{};
+	};
+	make_tplan();
 	if (h->no_alloc && (tplan.bin_groups != 3 || tplan.rec_bytes() > h->tile_rec.cap ||
 	                    tplan.offs_bytes() > h->tile_offs.cap || 4 * (size_t)(tplan.ntiles + 1) > h->tseq.cap))
 		tplan = TilePlan{};  // more than the slices of the static scratch hold
@@ -1833,7 +1838,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				sig.select_nt = h->tune_select_nt;
 				sig.low = h->tail_full ? 0 : h->tune_low;
 				sig.coarse = met.coarse_off || h->cfg.coarse_separate || h->tune_coarse_sep ? 0 : 1;
-				sig.pad = (met.bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0) | (groups ? 8 : 0);
+				sig.pad = (met.bin_parts ? 1 : 0) | (use_tiles() ? 2 : 0) | (small ? 4 : 0) | (groups ? 8 : 0) | met.tight << 4;
 			}
 			const bool tiled = use_tiles();  // also of a replay, which plans nothing
 			bool via_graph = false;
@@ -1884,6 +1889,19 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			}
 			TRY(read_head(h, &head));
 			n_written = std::max<int64_t>(n_written, (int64_t)head.rc.n_records);
+			if (tiled && head.rc.coarse_ovf == TL_BIN_FULL && met.tight < 2 && !h->no_alloc) {
+				// a bin outgrew its slots: more bins, as for these rows from now on
+				++met.tight;
+				make_tplan();
+				met.tiles_off = tplan.ntiles == 0;
+				keep_met();
+				if (met.tiles_off && (int64_t)V > sorted_budget)
+					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
+				no_graph = no_graph || via_graph;
+				grouped = false;
+				prologue_done = false;
+				continue;
+			}
 			// More equal pairs than records (many copies of some strings) stay
 			// in the bins, which leave out most of them before the tail: 3
 			// copies of 100 000 CDR3s, d = 2, 2.2 ms against 30.8 through the

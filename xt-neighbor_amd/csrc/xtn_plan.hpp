@@ -90,7 +90,9 @@ struct TilePlan {
 // standing together (rows sorted by length) outgrew a tile here and there: 1
 // of 3840 tiles for 1M CDR3s at d = 2, which cost the whole run the tiles, 1.69
 // ms instead of 0.90. Ordinary lengths weigh 0 to 2 % more than their records.
-inline TilePlan plan_tiles(const LenCounts& len, int64_t n, int d, int n_cu) {
+// tight: how often a bin of these rows has outgrown its slots; each time the
+// bins get a fifth more room than their mean needs, and not the few slots.
+inline TilePlan plan_tiles(const LenCounts& len, int64_t n, int d, int n_cu, int tight = 0) {
 	const int64_t vmax = (int64_t)host_variant_count(MAX_PREFIX, d), most = TL_CAP - vmax;
 	const int64_t V = len.records(d, 0);
 	const double avg = (double)V / (double)n;
@@ -126,7 +128,10 @@ inline TilePlan plan_tiles(const LenCounts& len, int64_t n, int d, int n_cu) {
 	// The fewest bins whose runs fit the bin kernel's registers (a run, the
 	// records that one tile has for one bin, is Poisson and takes a group per
 	// four of them), and enough of them that bin and record leave 11 keys per
-	// record: two records meet by chance once in 20 or so.
+	// record: two records meet by chance once in 20 or so. They fit with a margin
+	// of 3.5 % and of six standard deviations over the tiles' runs: the spread is
+	// what counts for bins of few slots (177 000 CDR3s, d = 1: mean 1474 of 1536
+	// groups, deviation 19, the fullest of 512 bins 1535).
 	const double key_bits = std::log2((double)V) + 3.5;
 	const double tile_recs = (double)V / (double)p.ntiles;
 	// a bin for every resident workgroup of the narrow form (two per CU)
@@ -135,21 +140,26 @@ inline TilePlan plan_tiles(const LenCounts& len, int64_t n, int d, int n_cu) {
 	auto bins_for = [&](int nt, int groups) {
 		for (int bits = min_bits; (1 << bits) <= TL_BINS_MAX; ++bits) {
 			const double lambda = tile_recs / (1 << bits);
-			double q = 0, w = std::exp(-lambda);
-			if (lambda > 200)
+			double q = 0, q2 = 0, w = std::exp(-lambda);  // a run's groups, and their squares
+			if (lambda > 200) {
 				q = lambda / 4 + 0.375;
-			else
+				q2 = q * q + lambda / 16 + 0.08;
+			} else {
 				for (int k = 1; k < 400; ++k) {
 					w *= lambda / k;
 					q += w * ((k + 3) / 4);
+					q2 += w * ((k + 3) / 4) * ((k + 3) / 4);
 				}
-			if (q * (double)p.ntiles <= 0.965 * nt * groups && bits + 32 - tl_len_bits(d) - p.idx_bits >= key_bits)
+			}
+			const double mean = q * (double)p.ntiles, spread = std::sqrt((q2 - q * q) * (double)p.ntiles);
+			const double room = nt * groups * (1.0 - 0.2 * tight);
+			if (std::max(mean / 0.965, mean + 6.0 * spread) <= room && bits + 32 - tl_len_bits(d) - p.idx_bits >= key_bits)
 				return bits;
 		}
 		return 0;
 	};
 	// The form of few slots where the fewest bins suffice.
-	if (bins_for(BIN_NT, 3) == min_bits) {
+	if (!tight && bins_for(BIN_NT, 3) == min_bits) {
 		p.bin_bits = min_bits;
 		p.bin_groups = 3;
 		return p;

@@ -42,6 +42,9 @@
 namespace xtn {
 
 constexpr uint32_t TL_NONE = 0xFFFFFFFFu;  // no record (a tile's last index is never used)
+// coarse_ovf where the only bound outgrown is a bin's slots: the tiles are
+// planned again with more bins
+constexpr uint32_t TL_BIN_FULL = 2;
 // equal keys before a record: a longer group is left to the run kernels, which
 // spread its pairs over the chip (one string 1100 times among 300 000 rows, d =
 // 1: 10.8 ms there)
@@ -677,7 +680,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		}
 		if (nq > (uint32_t)QCAP) {  // uniform
 			if (t == 0)
-				atomicOr(&a.ctr->coarse_ovf, 1ull);
+				atomicOr(&a.ctr->coarse_ovf, (unsigned long long)TL_BIN_FULL);
 			__syncthreads();
 			b += step;
 			continue;
