@@ -63,6 +63,18 @@ def lengths(name, n, rng):
     return rng.integers(0, 19, n)  # any
 
 
+@pytest.mark.parametrize("d,length,n", [(2, 1, 80_000_000), (1, 2, 100_000_000), (2, 2, 60_000_000), (4, 1, 30_000_000),
+                                        (1, 18, 20_000_000), (2, 18, 2_500_000), (3, 18, 400_000), (4, 18, 100_000)])
+def test_tiles_and_slots_have_room_for_their_numbers(lib, d, length, n):
+    # a listed record keeps its tile in 16 bits, a group of records its first
+    # slot in 30
+    counts = np.zeros(19, dtype=np.int64)
+    counts[length] = n
+    p = plan(lib, counts, d)
+    assert p["ntiles"] <= 65535
+    assert p["ntiles"] << p["slot_bits"] < 1 << 30
+
+
 @pytest.mark.parametrize("d", [1, 2, 3, 4])
 @pytest.mark.parametrize("name", ["cdr3", "wide", "two", "mostly long", "short", "any"])
 @pytest.mark.parametrize("n", [37, 3_001, 60_013, 700_001])

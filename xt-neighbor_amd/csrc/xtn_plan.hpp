@@ -17,6 +17,7 @@ constexpr int TL_CAP_BITS = 15;
 constexpr int TL_CAP = 1 << TL_CAP_BITS;  // records of a tile, at most
 constexpr int TL_IT = TL_CAP / TL_NT;     // records of a thread
 constexpr int TL_BINS_MAX = 8192;
+constexpr int64_t TL_TILES_MAX = 65535, TL_SLOTS_MAX = ((int64_t)1 << 30) - 1;
 
 // sequences a tile may hold and the bits of an index in it, by distance: the
 // tables of a tile's sequences share LDS with its records
@@ -125,6 +126,12 @@ inline TilePlan plan_tiles(const LenCounts& len, int64_t n, int d, int n_cu, int
 	if (!p.ntiles)
 		return p;
 	p.slot_bits = bits_for(tile + vmax - 1);
+	// a listed record keeps its tile in 16 bits, a group of records its first
+	// slot in 30 (k_bins)
+	if (p.ntiles > TL_TILES_MAX || p.ntiles << p.slot_bits > TL_SLOTS_MAX) {
+		p.ntiles = 0;
+		return p;
+	}
 	// The fewest bins whose runs fit the bin kernel's registers (a run, the
 	// records that one tile has for one bin, is Poisson and takes a group per
 	// four of them), and enough of them that bin and record leave 11 keys per

@@ -585,12 +585,12 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		uint32_t bm1[(1 << B1) / 32];
 		struct {
 			uint32_t rec[SVC];
-			uint16_t tile[SVC];
+			uint16_t tile[SVC];  // at most TL_TILES_MAX
 		} sv;
 	} u1;
 	__shared__ uint32_t s_bm2[(1 << B2) / 32];
 	__shared__ union {
-		uint32_t list[QCAP];  // (first record << 2) | records - 1
+		uint32_t list[QCAP];  // (first record << 2) | records - 1, slots below TL_SLOTS_MAX
 		struct {
 			uint32_t head[HEADS];
 			uint32_t pl[PLC];     // two listed records of equal key
