@@ -541,7 +541,7 @@ int radix_sort(xtn_handle* h, DBuf& keys, DBuf& keys_alt, DBuf* vals, DBuf* vals
 // pinned staging, one half filled by the copy engine while the other goes to
 // its place. A copy into unpinned memory goes through the runtime's own
 // staging instead: 22 against 13 us for the control block, 148 against 95 for
-// 2.7 MB, 619 against 240 for 11.5 MB.
+// 2.7 MB, 652 against 445 for 11.6 MB.
 struct FetchPart {
 	void* dst;
 	const void* src;
@@ -551,13 +551,21 @@ constexpr size_t DL_HALF = (size_t)1 << 20;
 
 int fetch(xtn_handle* h, std::initializer_list<FetchPart> parts, hipStream_t s) {
 	if (!h->dl_pin && !h->no_alloc) {  // (the no-allocation form keeps no pinned memory)
-		if (hipHostMalloc(&h->dl_pin, 2 * DL_HALF, hipHostMallocDefault) != hipSuccess) {
+		// the staging with both its events or not at all
+		bool ok = hipHostMalloc(&h->dl_pin, 2 * DL_HALF, hipHostMallocDefault) == hipSuccess;
+		if (!ok)
+			h->dl_pin = nullptr;
+		for (hipEvent_t& e : h->dl_ev)
+			if (ok && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+				e = nullptr;
+				ok = false;
+			}
+		if (!ok) {
 			(void)hipGetLastError();
+			if (h->dl_pin)
+				(void)hipHostFree(h->dl_pin);
 			h->dl_pin = nullptr;
 		}
-		for (hipEvent_t& e : h->dl_ev)
-			if (h->dl_pin && !e)
-				HIP_TRY(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
 	}
 	size_t total = 0;
 	for (const FetchPart& p : parts)
@@ -602,6 +610,23 @@ int fetch(xtn_handle* h, std::initializer_list<FetchPart> parts, hipStream_t s) 
 	TRY(drain(half));
 	TRY(drain(half ^ 1));
 	++h->stats.n_syncs;
+	return XTN_OK;
+}
+
+// fetch into a caller's memory: pinned (or any other that the runtime knows)
+// is the copy engine's own destination, without the staging and the copy out of
+// it (11.6 MB into pinned memory: 221 us against 456)
+int fetch_out(xtn_handle* h, std::initializer_list<FetchPart> parts, hipStream_t s) {
+	for (const FetchPart& p : parts) {
+		hipPointerAttribute_t at{};
+		if (hipPointerGetAttributes(&at, p.dst) != hipSuccess || at.type == hipMemoryTypeUnregistered) {
+			(void)hipGetLastError();
+			return fetch(h, parts, s);
+		}
+	}
+	for (const FetchPart& p : parts)
+		HIP_TRY(h, hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
+	HIP_SYNC(h, s);
 	return XTN_OK;
 }
 
@@ -2532,8 +2557,8 @@ int xtn_copy_nn_output(xtn_handle* h, xtn_int2* pairs, int8_t* distances, int64_
 	const int64_t n = std::min<int64_t>(cap, h->out_len);
 	if (n <= 0)
 		return XTN_OK;
-	return fetch(h, {{pairs, h->out_pairs.p, sizeof(xtn_int2) * (size_t)n}, {distances, h->out_dist.p, (size_t)n}},
-	             h->stream);
+	return fetch_out(h, {{pairs, h->out_pairs.p, sizeof(xtn_int2) * (size_t)n}, {distances, h->out_dist.p, (size_t)n}},
+	                 h->stream);
 }
 
 int xtn_perform(xtn_handle* h, const xtn_seq_info* info, xtn_callback callback, void* user) {
