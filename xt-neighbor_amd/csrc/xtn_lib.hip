@@ -1282,11 +1282,19 @@ void launch_gen_coarse(const GenArgs& ga, unsigned grid, hipStream_t s) {
 }
 
 int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t row_base = 0,
-                const uint32_t* set_of = nullptr) {
+                const uint32_t* set_of = nullptr, double t_first = 0) {
 	hipStream_t s = h->stream;
 	const int d = h->cfg.distance;
 	xtn_stats& st = h->stats;
-	const double t0 = now_ms();
+	const double t0 = t_first > 0 ? t_first : now_ms();
+	// the search from its start in another number of chunks: its time goes on,
+	// the counts of rounds that are done lapse
+	const int64_t unique0 = st.n_unique, rounds0 = st.n_rounds;
+	auto again = [&]() -> int {
+		st.n_unique = unique0;
+		st.n_rounds = rounds0;
+		return nn_pipeline(h, nseq, seq_map, row_base, set_of, t0);
+	};
 	h->out_len = 0;
 	st.n_sequences = nseq;
 	const xtn_handle::RowsKey rows_key{seq_map ? -1 : (int64_t)row_base, nseq, set_of ? h->sets_id : 0, d};
@@ -1921,7 +1929,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				met.tiles_off = tplan.ntiles == 0;
 				keep_met();
 				if (met.tiles_off && (int64_t)V > sorted_budget)
-					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
+					return again();
 				no_graph = no_graph || via_graph;
 				grouped = false;
 				prologue_done = false;
@@ -1942,7 +1950,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				(tiled ? met.tiles_off : met.coarse_off) = true;
 				keep_met();
 				if (tiled && (int64_t)V > sorted_budget)  // the chunks of the other layouts
-					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
+					return again();
 				grouped = false;
 				prologue_done = false;
 				continue;
@@ -1998,7 +2006,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 				// (packing included, whose offsets share the flag)
 				h->tail_safe = true;
 				if ((int64_t)V > sorted_budget && nparts == 1)
-					return nn_pipeline(h, nseq, seq_map, row_base, set_of);
+					return again();
 				grouped = false;
 				prologue_done = false;
 				continue;
