@@ -1619,6 +1619,7 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			ta.bin_bits = tplan.bin_bits;
 			ta.lb = tplan.idx_bits;
 			ta.sets = set_of ? 1 : 0;
+			ta.repeats = h->no_alloc ? 1 : 0;
 			BinArgs& bn = g.bn;
 			bn.rec = ta.out;
 			bn.cols = h->tile_cols.as<uint16_t>();
@@ -1938,11 +1939,12 @@ int nn_pipeline(xtn_handle* h, int32_t nseq, const uint32_t* seq_map, uint32_t r
 			// More equal pairs than records (many copies of some strings) stay
 			// in the bins, which leave out most of them before the tail: 3
 			// copies of 100 000 CDR3s, d = 2, 2.2 ms against 30.8 through the
-			// generator's coarse pass and 44.2 through the separate pass. Not in the
-			// static scratch, whose room for candidates is part of what its entry
-			// point accepts: there the other layout counts them all.
+			// generator's coarse pass and 44.2 through the separate pass. The static
+			// scratch's room for candidates, every equal pair counted, is part of what
+			// its entry point accepts: where they may not fit, the other layout
+			// decides.
 			many_pairs = tiled && head.rc.pairs_small > V ? (int64_t)head.rc.pairs_small : 0;
-			if (head.rc.coarse_ovf || (many_pairs && h->no_alloc)) {
+			if (head.rc.coarse_ovf || (tiled && h->no_alloc && (int64_t)head.rc.pairs_small > pmax)) {
 				// the tiles or bins outgrew a bound (the other layouts from now on,
 				// the generator's coarse pass among them), or a sub-range of that
 				// pass overflowed and lost records (the separate pass from now on):

@@ -106,6 +106,7 @@ struct TileArgs {
 	int32_t bin_bits;        // 6..13
 	int32_t lb;              // index bits of a record
 	int32_t sets;            // the prefixes carry query sets
+	int32_t repeats;         // repeated variants too (the search in static scratch, which counts them)
 	uint32_t n;              // sequences
 	int32_t slot_bits;       // a tile's slots, at most TL_CAP
 };
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(TL_NT, 4) void k_tiles(TileArgs a) {
 #pragma unroll
 		for (int k = 2; k <= D; ++k)
 			tab[(k - 1) * W + NO_DEL] = pre[k - 1] ^ pre[k];
-		u.s.info[i] = run_mask(lo, hw) | ((uint32_t)(hw >> 56) << MAX_PREFIX);
+		u.s.info[i] = (a.repeats ? 0u : run_mask(lo, hw)) | ((uint32_t)(hw >> 56) << MAX_PREFIX);
 	}
 	if (t == 0)
 		u.s.start[cnt] = (uint16_t)total;
