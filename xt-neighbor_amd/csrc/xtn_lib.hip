@@ -273,7 +273,7 @@ int grow_keep(xtn_handle* h, DBuf& b, size_t bytes, size_t keep) {
 
 // The lengths of rows [r0, r0 + n): the counts before every LEN_BLOCK rows,
 // made once for a handle's rows, and the rows at the two ends one by one.
-constexpr int64_t LEN_BLOCK = 1024;
+constexpr int64_t LEN_BLOCK = 256;
 
 void add_lengths(const uint8_t* len, int64_t n, LenCounts* out) {
 	uint32_t c[4][MAX_PREFIX + 1] = {};  // (four: neighbours are often alike)

@@ -40,17 +40,27 @@ inline int bits_for(int64_t maxval) {
 	return b;
 }
 
-// sum_{k <= min(d, L)} C(L, k) for the 18-residue prefix of a len-residue
-// sequence (the count k_pack computes on the device)
-inline uint64_t host_variant_count(uint32_t len, int d) {
-	const int L = len < (uint32_t)MAX_PREFIX ? (int)len : MAX_PREFIX;
-	const int m = d < L ? d : L;
-	uint64_t c = 1, total = 1;
-	for (int j = 1; j <= m; ++j) {
-		c = c * (uint64_t)(L - j + 1) / (uint64_t)j;
-		total += c;
+// sum_{k <= min(d, L)} C(L, k) by distance and length
+struct VariantCounts {
+	uint32_t v[MAX_PREFIX + 1][MAX_PREFIX + 1] = {};
+	constexpr VariantCounts() {
+		for (int d = 0; d <= MAX_PREFIX; ++d)
+			for (int L = 0; L <= MAX_PREFIX; ++L) {
+				uint64_t c = 1, total = 1;
+				for (int j = 1; j <= d && j <= L; ++j) {
+					c = c * (uint64_t)(L - j + 1) / (uint64_t)j;
+					total += c;
+				}
+				v[d][L] = (uint32_t)total;  // at most 2^18
+			}
 	}
-	return total;
+};
+
+// the variants of the 18-residue prefix of a len-residue sequence (the count
+// k_pack computes on the device)
+inline uint64_t host_variant_count(uint32_t len, int d) {
+	static constexpr VariantCounts counts;
+	return counts.v[d < MAX_PREFIX ? d : MAX_PREFIX][len < (uint32_t)MAX_PREFIX ? len : (uint32_t)MAX_PREFIX];
 }
 
 // sequences by the length of their prefix
@@ -156,6 +166,8 @@ inline TilePlan plan_tiles(const LenCounts& len, int64_t n, int d, int n_cu, int
 					w *= lambda / k;
 					q += w * ((k + 3) / 4);
 					q2 += w * ((k + 3) / 4) * ((k + 3) / 4);
+					if (k > lambda && w < 1e-12)
+						break;
 				}
 			}
 			const double mean = q * (double)p.ntiles, spread = std::sqrt((q2 - q * q) * (double)p.ntiles);

@@ -809,7 +809,7 @@ __global__ __launch_bounds__(NT, 4) void k_bins(BinArgs a) {
 		if constexpr (ROUNDS) {
 			int u = t;  // kept from the compiler, which would hold what it makes of it in registers that the gather needs
 			asm volatile("" : "+v"(u));
-			constexpr int EV = PARTS && QPT == 18 ? 5 : 2;
+			constexpr int EV = FEW ? 1 : QPT == 18 ? 5 : 2;
 			uint32_t i = u, n = 0xFFFFu, same = 0;
 			bool mid = false;  // the walk of record i stands at link n
 			bool checked = false;
