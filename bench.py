@@ -590,7 +590,7 @@ def main():
         "launches_per_step": st["n_launches"],
         "syncs_per_step": st["n_syncs"],
         "graph_replay": bool(st["graph_replays"]),
-        "tail_sort_passes": st["tail_passes"],
+        "tail_sort_passes": st["tail_passes"] if prof["sort_pairs"][0] else 0,
         "coarse_in_generator": bool(st["coarse_in_generator"]),
         "output_pairs": out_len,
         "variants": st["n_variants"],

@@ -128,9 +128,9 @@ typedef struct {
 	int64_t n_launches;    /* kernel launches of the last call */
 	int64_t n_syncs;       /* host waits on the device of the last call */
 	int64_t graph_replays; /* runs issued as one captured graph launch */
-	int64_t tail_passes;   /* 8-bit LSD passes that sort the candidates where
-	                          they are sorted as one (not where a workgroup
-	                          or groups of neighbouring ids take them): fewer
+	int64_t tail_passes;   /* 8-bit LSD passes of a sort of the candidates as
+	                          one (which doesn't run where a workgroup or
+	                          groups of neighbouring ids take them): fewer
 	                          than the pair bits need when the select ranks
 	                          the low bits of each group in LDS, all of them
 	                          after a group outgrew the select's window on

@@ -17,20 +17,20 @@
 //                over these finds the pairs, and the pairs go out as
 //                candidates
 //
-// Measured at 1M CDR3s, d = 2 (1.12e8 records): k_tiles 324 us (vector
-// instructions busy 71% of the time), k_tile_cols 25 us, k_bins 428 us (half
-// of its wave cycles wait; vector units, LDS and the address unit are each
-// busy 30 to 45%), against 465 + 427 + 298 us for the three kernels of the
+// Measured at 1M CDR3s, d = 2 (1.12e8 records): k_tiles 318 us (vector units
+// busy 60% of the time, LDS 48%), k_tile_cols 25 us, k_bins 430 us (half of its
+// wave cycles wait; vector and address units are busy 46% of the time, LDS
+// 28%), against 465 + 427 + 298 us for the three kernels of the
 // sub-range path; the candidates fall from 2.69M to 0.88M (tile_pair), which
 // takes another 45 us off their sort. 10 000 CDR3s, d = 1 (160 003 records):
 // tiles 9, bins 15 us.
 // Per record this moves 4 bytes out and 4 back, against 8 out, 8 in, 8 out
 // and 8 in for the sub-range path (k_gen<GEN_COARSE>, k_region_scatter,
 // k_bucket), which stays for distances above 4, for fewer than 4096 records,
-// for searches that ask for the separate pass, and for inputs that outgrow a
-// bound here (a bin, a group of more than TL_GROUP_MAX equal keys): such a run
-// raises coarse_ovf and is redone there. No order of the rows outgrows a tile
-// (plan_tiles).
+// for searches that ask for the separate pass, and for inputs with a group of
+// more than TL_GROUP_MAX equal keys: such a run raises coarse_ovf and is redone
+// there. No order of the rows outgrows a tile (plan_tiles); a bin over its
+// slots has the tiles planned again with more bins first.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -493,8 +493,9 @@ __device__ __forceinline__ uint32_t residue_set(uint64_t lo, uint32_t hi26) {
 // Two sequences whose records share a key: whether they go out as a candidate
 // pair. Each deletion takes at most one residue out of a string's set of
 // residues, so sets further apart than the two sides' deletions show that
-// only the keys met (a chance of 2^-32 a pair of records, but there are
-// 10^15 pairs). Two prefixes within one edit of each other share a variant
+// only the keys met (bin and record together keep at most 32 bits of the key,
+// about 11 keys for each record, so one record in 20 or so meets another by
+// chance). Two prefixes within one edit of each other share a variant
 // for every further deletion as well (about a dozen at distance 2, a hundred
 // at 3): the pair goes out only from the variant with the fewest deletions, which
 // both sides hold and whose length is known from the two strings.
